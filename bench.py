@@ -43,7 +43,8 @@ METRIC = ("GCUPS + aligned pairs/s on 1 MI355X; learned-filter vs plain at "
 # packed int16 VALU peak: 256 CU x 64 lanes x 2 halves x 2.4 GHz
 PEAK_I16_TOPS = 78.6
 PEAK_I32_TOPS = 39.3
-OPS_PER_CELL = {"sw": 10, "swt": 10, "nwt": 9}   # algorithmic int ops / cell
+# algorithmic int ops / cell
+OPS_PER_CELL = {"sw": 10, "swt": 10, "nwt": 9, "nwl": 9}
 
 
 def log(*a):
@@ -74,6 +75,8 @@ TRAFFIC_PROFILES = {
 
 def rocprof_name(kernel):
     """k_dp<nwt.c3.l64r8.i16> -> void pa::k_dp<8, 64, false, true, true>"""
+    if kernel.startswith("k_dp<nwl."):
+        return "pa::k_nw_linear"
     m = re.match(r"k_dp<(sw|swt|nwt)\.c\d\.l(\d+)r(\d+)\.(i16|i32)>", kernel)
     if not m:
         return None

@@ -1196,3 +1196,5 @@ hipError_t launch_traceback(const TbArgs &a, int shape, bool stage, int grid,
 }
 
 }  // namespace pa
+
+#include "k_dp_linear.h"

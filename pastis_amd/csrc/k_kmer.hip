@@ -520,7 +520,7 @@ int build_set(pa_ctx *c, KmerState *K, KmerSet &S, bool rows,
     hipLaunchKernelGGL(k_kmer_extract, dim3(nblocks(nslots)), dim3(kTB), 0, s,
                        P<uint8_t>(const_cast<Buf &>(kcb)),
                        P<uint64_t>(rows ? c->roffs : c->coffs),
-                       (uint64_t)(uintptr_t)cb.p, P<uint64_t>(K->slots), nseq,
+                       (uint64_t)(uintptr_t)seq_base(cb), P<uint64_t>(K->slots), nseq,
                        nslots, kc.k, kc.stride, al, invalid,
                        P<uint32_t>(K->keys_a), P<uint64_t>(K->vals_a),
                        (unsigned long long *)K->cnt.p);

@@ -13,6 +13,8 @@ namespace pa {
 constexpr int kClasses = 4;
 constexpr int kBins = 2 * kClasses;
 constexpr int kBuckets = 64;
+// most bins of either sort (bin_tasks, bin_linear)
+constexpr int kMaxBins = kLinClasses > kBins ? kLinClasses : kBins;
 
 hipError_t fill_u32(uint32_t *p, uint32_t v, uint32_t n, hipStream_t s);
 // *dst += *src (one thread; a device-side counter)
@@ -44,8 +46,15 @@ hipError_t bin_tasks(const DpTask *tasks, uint32_t a, uint32_t b,
                      uint32_t cap, uint32_t *counts, uint32_t *hist,
                      uint32_t *fill, unsigned long long *bin_cells,
                      hipStream_t s, const uint32_t *rng = nullptr);
+// The same for the linear-gap kernel: bin = lin_class, one list with the bins
+// one after the other, the last bin first; starts receives their places.
+hipError_t bin_linear(const DpTask *tasks, uint32_t a, uint32_t b,
+                      uint32_t *list, uint32_t *counts, uint32_t *starts,
+                      uint32_t *hist, uint32_t *fill,
+                      unsigned long long *bin_cells, hipStream_t s,
+                      const uint32_t *rng = nullptr);
 hipError_t trace_sizes(const DpTask *tasks, uint64_t n, const DpShapes &sh,
-                       uint64_t *sizes, hipStream_t s);
+                       bool lin, uint64_t *sizes, hipStream_t s);
 hipError_t empty_out(const DpTask *tasks, uint32_t a, uint32_t b, int local,
                      int open, int ext, DpOut *out, hipStream_t s,
                      const uint32_t *rng = nullptr);

@@ -172,20 +172,35 @@ __device__ inline uint32_t task_steps(uint32_t qlen, uint32_t tlen,
     return (npass - 1) * (tlen + 2u * L - 1u) + tlen + 2u * (nl - 1u) + 1u;
 }
 
+// What bin_key needs: the class shapes and the int16 bounds (unused for the
+// linear-gap kernel's sort).
+struct BinArgs {
+    DpShapes sh;
+    int local, maxs, open, ext;
+};
+
 // Bin and bucket of a task (-1: empty task).  Buckets are 1/8 of an octave
 // of the step count wide (16 .. 2^23 steps), the longest in bucket 0.
-__device__ inline int bin_key(const DpTask &t, const DpShapes &sh, int local,
-                              int maxs, int open, int ext)
+template <bool LIN>
+__device__ inline int bin_key(const DpTask &t, const BinArgs &a)
 {
     if (t.qlen == 0 || t.tlen == 0)
         return -1;
-    const int rc = dp_class(t.qlen, sh);
-    const bool i16 =
-        local ? true
-              : global_i16_ok(t.qlen, t.tlen, t.flags, maxs, open, ext);
-    const int bin = 2 * rc + (i16 ? 0 : 1);
+    int bin;
+    uint32_t steps;
+    if (LIN) {
+        bin = lin_class(t.qlen);
+        steps = (t.qlen - 1) / kLinRows * (t.tlen + 127u) + t.tlen +
+                2u * (lin_last_lanes(t.qlen) - 1u) + 1u;
+    } else {
+        const bool i16 = a.local ? true
+                                 : global_i16_ok(t.qlen, t.tlen, t.flags,
+                                                 a.maxs, a.open, a.ext);
+        bin = 2 * dp_class(t.qlen, a.sh) + (i16 ? 0 : 1);
+        steps = task_steps(t.qlen, t.tlen, a.sh);
+    }
     // 8 * log2(steps / 16) from the leading bit and the next three
-    const uint32_t x = task_steps(t.qlen, t.tlen, sh) >> 4;
+    const uint32_t x = steps >> 4;
     int b = 0;
     if (x) {
         const int e = 31 - __builtin_clz(x);
@@ -198,61 +213,80 @@ __device__ inline int bin_key(const DpTask &t, const DpShapes &sh, int local,
 
 // Pass 1: histogram of the (bin, bucket) keys: LDS counters per block, then
 // one global atomic per key that occurs in the block.
+template <int NB>
 __global__ __launch_bounds__(256) void k_bin_hist(
     const DpTask *__restrict__ tasks, uint32_t a, uint32_t b,
-    const uint32_t *rng, DpShapes sh, int local, int maxs, int open, int ext,
-    uint32_t *hist)
+    const uint32_t *rng, BinArgs ba, uint32_t *hist)
 {
     if (rng) {   // task range from the device (chunks sized on the GPU)
         a = rng[0];
         b = rng[1];
     }
-    __shared__ uint32_t h[kBins * kBuckets];
-    for (int k = threadIdx.x; k < kBins * kBuckets; k += blockDim.x)
+    __shared__ uint32_t h[NB * kBuckets];
+    for (int k = threadIdx.x; k < NB * kBuckets; k += blockDim.x)
         h[k] = 0;
     __syncthreads();
     const uint32_t i = a + blockIdx.x * blockDim.x + threadIdx.x;
-    const int key = i < b ? bin_key(tasks[i], sh, local, maxs, open, ext) : -1;
+    const int key = i < b ? bin_key<NB == kLinClasses>(tasks[i], ba) : -1;
     if (key >= 0)
         atomicAdd(&h[key], 1u);
     __syncthreads();
-    for (int k = threadIdx.x; k < kBins * kBuckets; k += blockDim.x)
+    for (int k = threadIdx.x; k < NB * kBuckets; k += blockDim.x)
         if (h[k])
             atomicAdd(&hist[k], h[k]);
 }
 
-// Pass 2 (one block of 64 threads): fill = exclusive scan of the buckets of
-// each bin, counts = bin totals.
-__global__ void k_bin_scan(const uint32_t *hist, uint32_t *fill,
-                           uint32_t *counts)
+// Pass 2 (one block, a wave per bin, a lane per bucket): fill = exclusive
+// scan of the buckets of each bin, counts = bin totals.  With starts (the
+// linear-gap kernel's single list) the scan of a bin begins where the bins
+// after it end.  One thread per bin took 9.5 us of every batch's latency.
+template <int NB>
+__global__ __launch_bounds__(64 * NB) void k_bin_scan(const uint32_t *hist,
+                                                      uint32_t *fill,
+                                                      uint32_t *counts,
+                                                      uint32_t *starts)
 {
-    const int bin = threadIdx.x;
-    if (bin >= kBins)
-        return;
-    uint32_t run = 0;
-    for (int k = 0; k < kBuckets; ++k) {
-        fill[bin * kBuckets + k] = run;
-        run += hist[bin * kBuckets + k];
+    static_assert(kBuckets == 64, "a lane per bucket");
+    __shared__ uint32_t tot[NB];
+    const int bin = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t own = hist[bin * kBuckets + lane];
+    uint32_t run = own;
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t x = __shfl(run, lane - off);
+        run += lane >= off ? x : 0u;
     }
-    counts[bin] = run;
+    if (lane == 63)
+        tot[bin] = run;
+    __syncthreads();
+    uint32_t base = 0;
+    if (starts)
+        for (int k = bin + 1; k < NB; ++k)
+            base += tot[k];
+    fill[bin * kBuckets + lane] = base + run - own;
+    if (lane == 63) {
+        counts[bin] = run;
+        if (starts)
+            starts[bin] = base;
+    }
 }
 
-// Pass 3: each task goes to its bin's list at its bucket's next slot.  The
-// block counts its keys in LDS (the LDS atomic's old value is the task's
-// rank), reserves one range per key with a global atomic, and scatters.
+// Pass 3: each task goes to its bin's list (cap entries apart; cap 0: one
+// list) at its bucket's next slot.  The block counts its keys in LDS (the
+// LDS atomic's old value is the task's rank), reserves one range per key
+// with a global atomic, and scatters.
+template <int NB>
 __global__ __launch_bounds__(256) void k_bin(
     const DpTask *__restrict__ tasks, uint32_t a, uint32_t b,
-    const uint32_t *rng, DpShapes sh, int local, int maxs, int open, int ext,
-    uint32_t *__restrict__ lists, uint32_t cap, uint32_t *fill,
-    unsigned long long *bin_cells)
+    const uint32_t *rng, BinArgs ba, uint32_t *__restrict__ lists,
+    uint32_t cap, uint32_t *fill, unsigned long long *bin_cells)
 {
     if (rng) {
         a = rng[0];
         b = rng[1];
     }
-    __shared__ uint32_t h[kBins * kBuckets], base[kBins * kBuckets];
+    __shared__ uint32_t h[NB * kBuckets], base[NB * kBuckets];
     __shared__ unsigned long long cc[kBins];
-    for (int k = threadIdx.x; k < kBins * kBuckets; k += blockDim.x)
+    for (int k = threadIdx.x; k < NB * kBuckets; k += blockDim.x)
         h[k] = 0;
     if (threadIdx.x < kBins)
         cc[threadIdx.x] = 0;
@@ -262,16 +296,16 @@ __global__ __launch_bounds__(256) void k_bin(
     uint64_t cells = 0;
     if (i < b) {
         const DpTask t = tasks[i];
-        key = bin_key(t, sh, local, maxs, open, ext);
+        key = bin_key<NB == kLinClasses>(t, ba);
         cells = (uint64_t)t.qlen * t.tlen;
     }
     uint32_t rank = 0;
     if (key >= 0) {
         rank = atomicAdd(&h[key], 1u);
-        atomicAdd(&cc[key / kBuckets], (unsigned long long)cells);
+        atomicAdd(&cc[key / kBuckets % kBins], (unsigned long long)cells);
     }
     __syncthreads();
-    for (int k = threadIdx.x; k < kBins * kBuckets; k += blockDim.x)
+    for (int k = threadIdx.x; k < NB * kBuckets; k += blockDim.x)
         base[k] = h[k] ? atomicAdd(&fill[k], h[k]) : 0u;
     if (threadIdx.x < kBins && cc[threadIdx.x])
         atomicAdd(&bin_cells[threadIdx.x], cc[threadIdx.x]);
@@ -281,15 +315,17 @@ __global__ __launch_bounds__(256) void k_bin(
 }
 
 __global__ void k_trace_sizes(const DpTask *__restrict__ tasks, uint64_t n,
-                              DpShapes sh, uint64_t *__restrict__ sizes)
+                              DpShapes sh, bool lin,
+                              uint64_t *__restrict__ sizes)
 {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
         const DpTask t = tasks[i];
-        sizes[i] = (t.qlen && t.tlen)
-                       ? trace_bytes(t.qlen, t.tlen, rows_per_lane(t.qlen, sh),
-                                     lanes_per_task(t.qlen, sh))
-                       : 0;
+        sizes[i] = !(t.qlen && t.tlen) ? 0
+                   : lin ? lin_trace_bytes(t.qlen, t.tlen)
+                         : trace_bytes(t.qlen, t.tlen,
+                                       rows_per_lane(t.qlen, sh),
+                                       lanes_per_task(t.qlen, sh));
     }
 }
 
@@ -528,6 +564,26 @@ hipError_t build_nw_tasks(const XdTask *xt, uint64_t nt, const XdOut *xo,
     return hipGetLastError();
 }
 
+namespace {
+template <int NB>
+hipError_t bin_run(const DpTask *tasks, uint32_t a, uint32_t b,
+                   const BinArgs &ba, uint32_t *lists, uint32_t cap,
+                   uint32_t *counts, uint32_t *starts, uint32_t *hist,
+                   uint32_t *fill, unsigned long long *bin_cells,
+                   hipStream_t s, const uint32_t *rng)
+{
+    if (b <= a)
+        return hipSuccess;
+    hipLaunchKernelGGL(k_bin_hist<NB>, dim3(blocks(b - a, 256)), dim3(256), 0,
+                       s, tasks, a, b, rng, ba, hist);
+    hipLaunchKernelGGL(k_bin_scan<NB>, dim3(1), dim3(64 * NB), 0, s, hist,
+                       fill, counts, starts);
+    hipLaunchKernelGGL(k_bin<NB>, dim3(blocks(b - a, 256)), dim3(256), 0, s,
+                       tasks, a, b, rng, ba, lists, cap, fill, bin_cells);
+    return hipGetLastError();
+}
+}  // namespace
+
 hipError_t bin_tasks(const DpTask *tasks, uint32_t a, uint32_t b,
                      const DpShapes &sh, int local, int maxs, int open,
                      int ext, uint32_t *lists,
@@ -535,25 +591,28 @@ hipError_t bin_tasks(const DpTask *tasks, uint32_t a, uint32_t b,
                      uint32_t *fill, unsigned long long *bin_cells,
                      hipStream_t s, const uint32_t *rng)
 {
-    if (b <= a)
-        return hipSuccess;
-    hipLaunchKernelGGL(k_bin_hist, dim3(blocks(b - a, 256)), dim3(256), 0, s,
-                       tasks, a, b, rng, sh, local, maxs, open, ext, hist);
-    hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(64), 0, s, hist, fill,
-                       counts);
-    hipLaunchKernelGGL(k_bin, dim3(blocks(b - a, 256)), dim3(256), 0, s, tasks,
-                       a, b, rng, sh, local, maxs, open, ext, lists, cap, fill,
-                       bin_cells);
-    return hipGetLastError();
+    return bin_run<kBins>(tasks, a, b, BinArgs{sh, local, maxs, open, ext},
+                          lists, cap, counts, nullptr, hist, fill, bin_cells,
+                          s, rng);
+}
+
+hipError_t bin_linear(const DpTask *tasks, uint32_t a, uint32_t b,
+                      uint32_t *list, uint32_t *counts, uint32_t *starts,
+                      uint32_t *hist, uint32_t *fill,
+                      unsigned long long *bin_cells, hipStream_t s,
+                      const uint32_t *rng)
+{
+    return bin_run<kLinClasses>(tasks, a, b, BinArgs{}, list, 0, counts,
+                                starts, hist, fill, bin_cells, s, rng);
 }
 
 hipError_t trace_sizes(const DpTask *tasks, uint64_t n, const DpShapes &sh,
-                       uint64_t *sizes, hipStream_t s)
+                       bool lin, uint64_t *sizes, hipStream_t s)
 {
     if (!n)
         return hipSuccess;
     hipLaunchKernelGGL(k_trace_sizes, dim3(blocks(n, 256)), dim3(256), 0, s,
-                       tasks, n, sh, sizes);
+                       tasks, n, sh, lin, sizes);
     return hipGetLastError();
 }
 

@@ -87,11 +87,15 @@ enum {
     C_XDWOVFQ = 33,     // their queue head
     C_XDW2OVF = 34,     // items left by the 256-column band kernel
     C_XDW2OVFQ = 35,    // their queue head
-    C_HIST = 36,        // kBins x kBuckets histogram of the counting sort
-    C_FILL = C_HIST + kBins * kBuckets,   // its running slots
-    C_N = C_FILL + kBins * kBuckets
+    C_LIN = 36,         // linear-gap classes: list lengths, starts, queues
+    C_LINS = C_LIN + kLinClasses,
+    C_LINQ = C_LINS + kLinClasses,
+    C_HIST = C_LINQ + kLinClasses,   // histogram of the counting sort
+    C_FILL = C_HIST + kMaxBins * kBuckets,   // its running slots
+    C_N = C_FILL + kMaxBins * kBuckets
 };
 
+constexpr int kModes = 3;           // DP modes of the kernel statistics
 constexpr int kMaxWgPerCu = 32;     // one-wave workgroups per CU (8 per SIMD)
 constexpr int kXdWideLanes = 65536;  // lanes of the wide (global scratch) re-run
 constexpr int kXdGraphLanes = 4096;  // its lanes in a captured batch
@@ -159,6 +163,7 @@ void resolve_timers(pa_ctx *c)
         case 1: c->stats.ms_xdrop += ms; break;
         case 2: c->stats.ms_nw += ms; break;
         case 3: c->stats.ms_trace += ms; break;
+        case 5: c->klin.ms += ms; c->klin.launches++; break;
         default: c->stats.ms_total += ms; break;
         }
         c->free_events.push_back(t.a);
@@ -218,8 +223,26 @@ int xd_grid(pa_ctx *c, uint64_t nitems)
         1, std::min<uint64_t>((nitems + 63) / 64, (uint64_t)c->ncu * per_cu));
 }
 
+// Persistent grid of the linear-gap kernel and its boundary-row stride.
+int lin_grid(pa_ctx *c, uint64_t ntasks)
+{
+    int per_cu = nw_linear_occupancy();
+    if (c->tune.dp_wg_per_cu > 0)
+        per_cu = std::min(per_cu, (int)c->tune.dp_wg_per_cu);
+    return (int)std::max<uint64_t>(
+        1, std::min<uint64_t>(ntasks, (uint64_t)c->ncu * per_cu));
+}
+
+uint32_t lin_bnd_stride(const pa_ctx *c)
+{
+    return (c->max_clen + kLinBndPad + 15u) & ~15u;
+}
+
 int ensure_bnd(pa_ctx *c, bool local, bool trace)
 {
+    if (!local && c->lin_ok)
+        return grow(c, c->bnd,
+                    (size_t)lin_grid(c, ~0ull) * lin_bnd_stride(c));
     // one boundary row per task slot of the persistent workgroups of the
     // run's DP grids: per class, its grid (dp_grid) times the task slots of
     // its shape's one-wave workgroup
@@ -283,6 +306,7 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
         return rc;
     // a fill kernel, not a memset node, so that the sequence can be captured
     HIPCHK(c, fill_u32(P<uint32_t>(c->tflags), 0, (uint32_t)((nt + 3) / 4), s));
+    const bool lin = !local && c->lin_ok;
     std::vector<std::pair<uint64_t, uint64_t>> chunks;
     std::vector<uint64_t> chunk_base;   // trace offset of each chunk's first
     if (trace && c->g_chunks > 0) {
@@ -292,7 +316,7 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
             return rc;
         if ((rc = grow(c, c->toffs, nt * sizeof(uint64_t) + 8)))
             return rc;
-        HIPCHK(c, trace_sizes(P<DpTask>(c->tasks), nt, c->shapes,
+        HIPCHK(c, trace_sizes(P<DpTask>(c->tasks), nt, c->shapes, lin,
                               P<uint64_t>(c->sizes), s));
         // sizes[nt] = 0 so that toffs[nt] is the total (a fill kernel: no
         // memset node in a captured graph)
@@ -318,7 +342,7 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
             return rc;
         if ((rc = grow(c, c->toffs, nt * sizeof(uint64_t) + 8)))
             return rc;
-        HIPCHK(c, trace_sizes(P<DpTask>(c->tasks), nt, c->shapes,
+        HIPCHK(c, trace_sizes(P<DpTask>(c->tasks), nt, c->shapes, lin,
                               P<uint64_t>(c->sizes), s));
         size_t tmp = 0;
         HIPCHK(c, hipcub::DeviceScan::ExclusiveSum(
@@ -419,8 +443,16 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
                                             2 * c->g_chunks) + ci
                        : nullptr;
         HIPCHK(c, fill_u32(ctr, 0, C_XDQ, s));
-        HIPCHK(c, fill_u32(ctr + C_HIST, 0, C_N - C_HIST, s));
-        HIPCHK(c, bin_tasks(P<DpTask>(c->tasks), a, b, c->shapes,
+        HIPCHK(c, fill_u32(ctr + C_LIN, 0, C_N - C_LIN, s));
+        if (lin)
+            HIPCHK(c, bin_linear(
+                          P<DpTask>(c->tasks), a, b, lists, ctr + C_LIN,
+                          ctr + C_LINS, ctr + C_HIST, ctr + C_FILL,
+                          (unsigned long long *)P<uint64_t>(c->bincells) +
+                              kModes * kBins,
+                          s, rng));
+        else
+            HIPCHK(c, bin_tasks(P<DpTask>(c->tasks), a, b, c->shapes,
                             local ? 1 : 0, c->maxs,
                             c->cfg.gap_open, c->cfg.gap_ext, lists,
                             (uint32_t)nt, ctr + C_BIN, ctr + C_HIST,
@@ -431,6 +463,33 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
         HIPCHK(c, empty_out(P<DpTask>(c->tasks), a, b, local ? 1 : 0,
                             c->cfg.gap_open, c->cfg.gap_ext,
                             P<DpOut>(c->dpout), s, rng));
+        if (lin) {
+            LinArgs la{};
+            la.tasks = P<DpTask>(c->tasks);
+            la.list = lists;
+            la.counts = ctr + C_LIN;
+            la.starts = ctr + C_LINS;
+            la.queues = ctr + C_LINQ;
+            la.pmat = (const uint32_t *)(P<int8_t>(c->dmat) + kPmatRot);
+            la.out = P<DpOut>(c->dpout);
+            la.trace = P<uint8_t>(c->trace) - base;
+            la.trace_off = P<uint64_t>(c->toffs);
+            la.trace_base = tbase;
+            la.bnd = P<uint8_t>(c->bnd);
+            la.bnd_stride = lin_bnd_stride(c);
+            la.gap = c->cfg.gap_open;
+            {
+                Scope sc(c, kind, s);
+                Scope k(c, 5, s);
+                HIPCHK(c, launch_nw_linear(la, lin_grid(c, b - a), s));
+            }
+            {
+                Scope sc(c, 3, s);
+                HIPCHK(c, launch_traceback_linear(la, b - a, s));
+            }
+            c->stats.launches += 2;
+            continue;
+        }
         DpArgs args{};
         args.codes = nullptr;  // task offsets hold absolute device addresses
         args.tasks = P<DpTask>(c->tasks);
@@ -806,9 +865,9 @@ int align_xd_dev(pa_ctx *c, const pa_pair *d_pairs, uint64_t n,
     Scope tot(c, 4, s);
     if ((rc = run_xdrop(c, d_pairs, n, s)))
         return rc;
-    const ResBound rb{(uint64_t)(uintptr_t)c->rcodes.p,
+    const ResBound rb{(uint64_t)(uintptr_t)seq_base(c->rcodes),
                       (const uint32_t *)((char *)c->rcodes.p + c->rpre_off)};
-    const ResBound cbd{(uint64_t)(uintptr_t)c->ccodes.p,
+    const ResBound cbd{(uint64_t)(uintptr_t)seq_base(c->ccodes),
                        (const uint32_t *)((char *)c->ccodes.p + c->cpre_off)};
     HIPCHK(c, build_nw_tasks(P<XdTask>(c->xdt), nt, P<XdOut>(c->xdo),
                              P<DpTask>(c->tasks), rb, cbd,
@@ -855,7 +914,7 @@ int upload_set(pa_ctx *c, bool rows, const uint8_t *res, const uint64_t *offs,
         lens[i] = (uint32_t)L;
         mx = std::max(mx, (uint32_t)L);
     }
-    std::vector<uint8_t> codes(total + 64, (uint8_t)kSentinel);
+    std::vector<uint8_t> codes(kSeqPad + total + 64, (uint8_t)kSentinel);
     // k-mer letters: a residue upper-cased with & 0xDF must be one of the 25
     // letters (add_kmers, src/kmer/KmerOps.cpp:61-73); '*' never is, since
     // '*' & 0xDF is not a letter
@@ -878,7 +937,7 @@ int upload_set(pa_ctx *c, bool rows, const uint8_t *res, const uint64_t *offs,
         } else {
             k = x == 23 ? 255 : x;
         }
-        codes[i] = x;
+        codes[kSeqPad + i] = x;
         kc[i] = k;
     }
     // Residue-bound prefix sums (ResBound) after the codes: the best score of
@@ -895,7 +954,7 @@ int upload_set(pa_ctx *c, bool rows, const uint8_t *res, const uint64_t *offs,
     uint32_t acc = 0;   // wraps around; span differences stay exact
     for (uint64_t i = 0; i < total; ++i) {
         pre[i] = acc;
-        acc += best[codes[i]];
+        acc += best[codes[kSeqPad + i]];
     }
     pre[total] = acc;
     Buf &cb = rows ? c->rcodes : c->ccodes;
@@ -910,7 +969,7 @@ int upload_set(pa_ctx *c, bool rows, const uint8_t *res, const uint64_t *offs,
     if ((rc = grow(c, ob, (nseq + 1) * sizeof(uint64_t))))
         return rc;
     std::vector<uint64_t> abs(nseq + 1);
-    const uint64_t dev = (uint64_t)(uintptr_t)cb.p;
+    const uint64_t dev = (uint64_t)(uintptr_t)seq_base(cb);
     for (uint64_t i = 0; i <= nseq; ++i)
         abs[i] = dev + (offs[i] - base);
     HIPCHK(c, hipMemcpyAsync(cb.p, codes.data(), codes.size(),
@@ -1080,6 +1139,14 @@ int pa_create(const pa_config *cfg, pa_ctx **out)
                 (int8_t)(c->nib_ok && q < kAlpha && x < kAlpha
                              ? c->mat[q * 32 + x] - lo
                              : 0);
+    // the nibbles of the linear-gap kernel, shifted and rotated (kPmatRot)
+    c->lin_ok = c->nib_ok && c->cfg.gap_open > c->cfg.gap_ext &&
+                lo == 2 * c->cfg.gap_open;
+    for (int k = 0; k < 1024; ++k) {
+        const int n = dm[kPmatNib + k] & 15;
+        dm[kPmatRot + k] = (int8_t)(n << 2);
+        dm[kPmatRot + 1024 + k] = (int8_t)(((n & 3) << 6) | (n >> 2));
+    }
     c->shapes = shapes_for(c, c->tune);
     if (grow(c, c->dmat, kPmatBytes) ||
         hipMemcpy(c->dmat.p, dm.data(), kPmatBytes, hipMemcpyHostToDevice) !=
@@ -1087,8 +1154,8 @@ int pa_create(const pa_config *cfg, pa_ctx **out)
         pa_destroy(c);
         return PA_ERR_NOMEM;
     }
-    if (grow(c, c->bincells, 3 * kBins * sizeof(uint64_t)) ||
-        hipMemset(c->bincells.p, 0, 3 * kBins * sizeof(uint64_t)) !=
+    if (grow(c, c->bincells, (kModes + 1) * kBins * sizeof(uint64_t)) ||
+        hipMemset(c->bincells.p, 0, (kModes + 1) * kBins * sizeof(uint64_t)) !=
             hipSuccess ||
         grow(c, c->cells, 4 * sizeof(uint64_t)) ||
         hipMemset(c->cells.p, 0, 4 * sizeof(uint64_t)) != hipSuccess) {
@@ -1743,7 +1810,9 @@ int pa_reset_stats(pa_ctx *c)
             k = pa_ctx::KStat{};
     if (c->cells.p)
         HIPCHK(c, hipMemset(c->cells.p, 0, 32));
-    HIPCHK(c, hipMemset(c->bincells.p, 0, 3 * kBins * sizeof(uint64_t)));
+    c->klin = pa_ctx::KStat{};
+    HIPCHK(c, hipMemset(c->bincells.p, 0,
+                        (kModes + 1) * kBins * sizeof(uint64_t)));
     return PA_OK;
 }
 
@@ -1754,7 +1823,7 @@ int pa_get_kernel_stats(pa_ctx *c, pa_kernel_stat *out, int cap, int *n)
     hipSetDevice(c->device);
     HIPCHK(c, hipStreamSynchronize(c->st));
     resolve_timers(c);
-    uint64_t cells[3 * kBins];
+    uint64_t cells[(kModes + 1) * kBins];
     HIPCHK(c, hipMemcpy(cells, c->bincells.p, sizeof(cells),
                         hipMemcpyDeviceToHost));
     static const char *mname[3] = {"sw", "swt", "nwt"};
@@ -1785,6 +1854,18 @@ int pa_get_kernel_stats(pa_ctx *c, pa_kernel_stat *out, int cap, int *n)
             }
             ++k;
         }
+    if (c->klin.launches) {
+        if (k < cap) {
+            pa_kernel_stat &o = out[k];
+            std::memset(&o, 0, sizeof(o));
+            std::snprintf(o.name, sizeof(o.name), "nwl.r%d.i16", kLinR);
+            o.launches = c->klin.launches;
+            o.ms = c->klin.ms;
+            for (int b = 0; b < kBins; ++b)
+                o.cells += cells[kModes * kBins + b];
+        }
+        ++k;
+    }
     *n = k;
     return PA_OK;
 }

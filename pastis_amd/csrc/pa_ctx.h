@@ -17,7 +17,8 @@ struct Buf {
 };
 
 struct Timer {
-    int kind;  // 0 sw, 1 xdrop, 2 nw, 3 trace, 4 total
+    int kind;  // 0 sw, 1 xdrop, 2 nw, 3 trace, 4 total, 5 linear kernel,
+               // 100 + 16 * mode + bin: a DP kernel class
     hipEvent_t a, b;
 };
 
@@ -95,6 +96,7 @@ struct pa_ctx {
         uint64_t launches = 0;
         double ms = 0;
     } kstat[3][pa::kBins + pa::kClasses];   // DP mode x (bins, int32 re-runs)
+    KStat klin;                   // linear-gap global kernel, all classes
     std::vector<Timer> pending;
     std::vector<hipEvent_t> free_events;
     pa_stats stats{};
@@ -136,6 +138,11 @@ struct pa_ctx {
     // .. nib_min + 15; if not, shapes replaces the 4-bit-profile shapes
     bool nib_ok = true;
     int nib_min = 0;
+    // the global alignments run in the linear-gap kernel (k_dp_linear.h):
+    // gaps never extended (open > ext) and score - 2 open within 0 .. 15
+    // over the alphabet, starting at 0 (BLOSUM62 with open -2, the
+    // as-called reading of -g -11 -e -2)
+    bool lin_ok = false;
     // No event timers (pa_sw_scores_noalloc: event objects are allocated).
     bool quiet = false;
     // Cap on the task slots (boundary rows) of a DP grid (0 = none); the
@@ -154,6 +161,15 @@ inline DpShapes shapes_for(const pa_ctx *c, const pa_tuning &t)
         for (int k = 0; k < 4; ++k)
             sh.shape[k] = (uint8_t)shape_byte_fallback(sh.shape[k]);
     return sh;
+}
+
+// Sentinels ahead of the first sequence of a store (a kernel's window of
+// residues may start up to 7 bytes before a sequence).
+constexpr size_t kSeqPad = 64;
+// device address of a store's first residue
+inline uint8_t *seq_base(const Buf &codes)
+{
+    return (uint8_t *)codes.p + kSeqPad;
 }
 
 inline int fail(pa_ctx *c, int code, const std::string &msg)

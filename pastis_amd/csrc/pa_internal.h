@@ -82,7 +82,10 @@ constexpr uint32_t kTaskSat = 1u;  // int16 saturated, needs the int32 re-run
 // 11); with any other matrix the context runs their 4-row counterparts.
 constexpr size_t kPmatUntraced = 1024, kPmatLocal = 2048, kPmatGlobal = 3072,
                  kPmatNib = 4096;
-constexpr size_t kPmatBytes = 5120;
+// Profiles of the linear-gap kernel (k_dp_linear.h): kPmatRot gives the same
+// nibble n as n << 2, the 1 KB after it as n rotated to bits 6, 7, 0, 1.
+constexpr size_t kPmatRot = 5120;
+constexpr size_t kPmatBytes = 7168;
 // Global task whose scores are bounded by the residue bound below (no cell
 // exceeds min over the two spans of the sum of each residue's best score),
 // small enough for the traced int16 kernels.
@@ -253,6 +256,82 @@ __host__ __device__ inline uint64_t trace_rec(uint32_t qlen, uint32_t tlen,
     return (uint64_t)p * trace_seg_steps(tlen + 2u * L - 1u) * L +
            (uint64_t)seg * nact * kTraceSeg + lane * kTraceSeg + off;
 }
+
+// Linear-gap global alignment (k_dp_linear.h).  A lane holds 2 * kLinR rows.
+// A class has a lane count per task (lin_lanes); as many tasks as fit sit
+// side by side in a wave.  Tasks take the narrowest class that holds their
+// rows, those of more than kLinRows rows the last class in several passes.
+// The counts are those where the tasks of a wave change (64 / L), so few
+// lanes stay idle: rows are rounded up to 32, lanes to 60 .. 64 per wave.
+constexpr int kLinR = 16;
+constexpr int kLinClasses = 15;
+constexpr int kLinRows = 2 * kLinR * 64;
+// bytes of one trace record: the 2-bit codes of a lane's rows at one step
+constexpr int kLinRec = kLinR / 2;
+// bytes of a boundary row besides its columns (k_dp_linear.h)
+constexpr uint32_t kLinBndPad = 288;
+
+__host__ __device__ inline int lin_lanes(int cls)
+{
+    return cls < 10 ? cls + 1
+           : cls == 10 ? 12
+           : cls == 11 ? 16
+           : cls == 12 ? 21
+           : cls == 13 ? 32
+                       : 64;
+}
+__host__ __device__ inline int lin_class(uint32_t qlen)
+{
+    const uint32_t need = (qlen + 2u * kLinR - 1u) / (2u * kLinR);
+    return need <= 10   ? (int)need - 1
+           : need <= 12 ? 10
+           : need <= 16 ? 11
+           : need <= 21 ? 12
+           : need <= 32 ? 13
+                        : 14;
+}
+// lanes of the last pass
+__host__ __device__ inline uint32_t lin_last_lanes(uint32_t qlen)
+{
+    const uint32_t rem = qlen - (qlen - 1) / kLinRows * kLinRows;
+    return (rem + 2u * kLinR - 1u) / (2u * kLinR);
+}
+// Trace layout as above with R = kLinR, L = 64 (a class's lane count does not
+// enter: a task with fewer rows than a pass has one pass of its own lanes),
+// and records of kLinRec bytes.  Offsets are multiples of 64.
+__host__ __device__ inline uint64_t lin_pass_bytes(uint32_t tlen)
+{
+    return (uint64_t)trace_seg_steps(tlen + 127u) * 64u * kLinRec;
+}
+__host__ __device__ inline uint64_t lin_trace_bytes(uint32_t qlen,
+                                                    uint32_t tlen)
+{
+    const uint32_t nl = lin_last_lanes(qlen);
+    return (uint64_t)((qlen - 1) / kLinRows) * lin_pass_bytes(tlen) +
+           (uint64_t)trace_seg_steps(tlen + 2u * (nl - 1u) + 1u) * nl *
+               kLinRec;
+}
+// Arguments of the linear-gap kernels: the task list, class after class (the
+// last class first), and per class its start, length and work-queue head.
+struct LinArgs {
+    const DpTask *tasks;
+    const uint32_t *list;
+    const uint32_t *starts;
+    const uint32_t *counts;
+    uint32_t *queues;
+    const uint32_t *pmat;       // kPmatRot
+    DpOut *out;
+    uint8_t *trace;
+    const uint64_t *trace_off;
+    const uint64_t *trace_base; // as DpArgs::trace_base
+    uint8_t *bnd;               // boundary rows, one per workgroup
+    uint32_t bnd_stride;
+    int32_t gap;
+};
+hipError_t launch_nw_linear(const LinArgs &a, int grid, hipStream_t s);
+int nw_linear_occupancy();
+hipError_t launch_traceback_linear(const LinArgs &a, uint32_t ntasks,
+                                   hipStream_t s);
 
 // X-drop extension task: one seed of one pair.
 struct XdTask {

@@ -145,7 +145,7 @@ bool better(double cand, double inc, const Times &c, const Times &i)
 
 // The coordinate search; `t` starts as the installed tuning and ends as the
 // choice.
-int search(Tuner &tu, bool xdrop, pa_tuning &t)
+int search(Tuner &tu, bool xdrop, bool lin, pa_tuning &t)
 {
     int rc;
     Times cur;
@@ -179,6 +179,8 @@ int search(Tuner &tu, bool xdrop, pa_tuning &t)
         {128, 256, 512}, {96, 192, 384}, {128, 256, 768}, {128, 384, 768},
         {64, 256, 512},  {128, 192, 512}};
     for (const auto &e : edges) {
+        if (lin)   // the linear-gap kernel has fixed classes
+            break;
         if (std::equal(e, e + 3, t.dp_edge))
             continue;
         pa_tuning cand = t;
@@ -195,7 +197,7 @@ int search(Tuner &tu, bool xdrop, pa_tuning &t)
     // 3. the kernel shape of each class
     for (int k = 0; k < kClasses; ++k)
         for (int sh = 0; sh < kShapes; ++sh) {
-            if (sh == t.dp_shape[k])
+            if (lin || sh == t.dp_shape[k])
                 continue;
             pa_tuning cand = t;
             cand.dp_shape[k] = sh;
@@ -225,7 +227,7 @@ int search(Tuner &tu, bool xdrop, pa_tuning &t)
     }
 
     // 5. traceback staging
-    if (cur.trace > 0) {
+    if (cur.trace > 0 && !lin) {
         pa_tuning cand = t;
         cand.tb_stage = 1 - t.tb_stage;
         Times tm;
@@ -238,7 +240,7 @@ int search(Tuner &tu, bool xdrop, pa_tuning &t)
     }
 
     // 6. tracebacks beside the DP or after it, by wall time
-    if (cur.trace > 0) {
+    if (cur.trace > 0 && !lin) {
         const int start_ov = t.tb_overlap;
         for (int ov = 0; ov < 3; ++ov) {
             if (ov == start_ov)
@@ -299,7 +301,12 @@ extern "C" int pa_autotune(pa_ctx *c, const pa_pair *d_pairs, uint64_t n,
         return fail(c, PA_ERR_ARG, "pa_autotune needs pairs to time");
     if (hipSetDevice(c->device) != hipSuccess)
         return fail(c, PA_ERR_HIP, "hipSetDevice");
-    const auto key = std::make_tuple(c->device, target, (int)c->cfg.mode);
+    const bool xdrop = target == PA_TUNE_ALIGN && c->cfg.mode == PA_MODE_XDROP;
+    // a choice made with the linear-gap kernel says nothing about the shapes
+    // of the others
+    const bool lin = xdrop && c->lin_ok;
+    const auto key =
+        std::make_tuple(c->device, target, (int)c->cfg.mode + (lin ? 2 : 0));
     if (!(flags & PA_TUNE_FORCE)) {
         std::lock_guard<std::mutex> lk(g_mu);
         auto it = g_cache.find(key);
@@ -327,13 +334,12 @@ extern "C" int pa_autotune(pa_ctx *c, const pa_pair *d_pairs, uint64_t n,
     pa_tuning t = start;
     int rc = PA_OK;
     hipError_t e = gather(d_pairs, n, m, dp, c->st);
-    const bool xdrop = target == PA_TUNE_ALIGN && c->cfg.mode == PA_MODE_XDROP;
     if (e != hipSuccess) {
         rc = fail(c, PA_ERR_HIP,
                   std::string("pa_autotune gather: ") + hipGetErrorString(e));
     } else {
         Tuner tu(c, dp, m, target, dout);
-        rc = search(tu, xdrop, t);
+        rc = search(tu, xdrop, lin, t);
     }
     if (!rc && mv && std::memcmp(&t, &start, sizeof(t)) != 0) {
         // the choice against the starting tuning on a larger share of the set
