@@ -277,107 +277,176 @@ __global__ __launch_bounds__(256) void k_select(
 }
 
 // ---- training -------------------------------------------------------------
+// Value of lane k as a wave-uniform float.
+__device__ inline float lane_value(float v, int k)
+{
+    return __uint_as_float((unsigned)__builtin_amdgcn_readlane(
+        (int)__float_as_uint(v), k));
+}
+
 // Per sample of the batch: standardize, forward, weighted BCE, backward to
 // dz1, dz2, dz3.  Scratch rows (fp32): xb[16] h1b[64] h2b[64] dz1[64] dz2[64]
 // dz3[1].
-__global__ __launch_bounds__(256) void k_train_fwd_bwd(
+//
+// A wave per sample, a lane per hidden unit: the lane keeps its columns of
+// W1 and W2 and its row of W2 in registers for all its wave's samples, the
+// other operand of a product comes from readlane, and every sum runs in the
+// order of the terms.  A batch of 4096 samples then fills the chip (1,024
+// waves) at about 600 instructions per sample; one thread per sample left
+// 240 CUs idle with its activations in scratch memory (134 us per batch of
+// 4096, now 18).
+constexpr int kTrainWaves = 4;    // waves per workgroup
+
+__global__ __launch_bounds__(64 * kTrainWaves) void k_train_fwd_bwd(
     const float *__restrict__ feats, const float *__restrict__ mean,
     const float *__restrict__ istd, const uint8_t *__restrict__ labels,
     const uint32_t *__restrict__ order, uint64_t base, uint32_t B,
     const float *wb, float pos_weight, float *__restrict__ scratch,
     float *__restrict__ loss_sum)
 {
-    __shared__ float w[kNParam];
-    for (int i = threadIdx.x; i < kNParam; i += blockDim.x)
-        w[i] = wb[i];
-    __syncthreads();
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= B)
-        return;
-    const uint32_t idx = order[base + s];
-    float *row = scratch + (size_t)s * kScratchRow;
-    float *h1b = row + kNF, *h2b = h1b + kH, *dz1 = h2b + kH, *dz2 = dz1 + kH;
-    float xb[kNF], z1[kH], z2[kH], h1[kH];
-    for (int k = 0; k < kNF; ++k) {
-        xb[k] = bf16r(__fmul_rn(__fsub_rn(feats[(size_t)idx * kNF + k], mean[k]),
-                                istd[k]));
-        row[k] = xb[k];
+    const int j = threadIdx.x & 63;
+    const uint32_t wave = blockIdx.x * kTrainWaves + (threadIdx.x >> 6);
+    float w1c[kNF], w2c[kH], w2r[kH];
+#pragma unroll
+    for (int k = 0; k < kNF; ++k)
+        w1c[k] = wb[kOffW1 + k * kH + j];
+#pragma unroll
+    for (int k = 0; k < kH; ++k) {
+        w2c[k] = wb[kOffW2 + k * kH + j];
+        w2r[k] = wb[kOffW2 + j * kH + k];
     }
-    for (int j = 0; j < kH; ++j) {
+    const float b1 = wb[kOffB1 + j], b2 = wb[kOffB2 + j], w3 = wb[kOffW3 + j];
+    const float mu = mean[j & (kNF - 1)], is = istd[j & (kNF - 1)];
+    float loss = 0.f;   // of this wave's samples
+    for (uint32_t s = wave; s < B; s += gridDim.x * kTrainWaves) {
+        const uint32_t idx = order[base + s];
+        float *row = scratch + (size_t)s * kScratchRow;
+        const float xb = bf16r(__fmul_rn(
+            __fsub_rn(feats[(size_t)idx * kNF + (j & (kNF - 1))], mu), is));
         float acc = 0.f;
+#pragma unroll
         for (int k = 0; k < kNF; ++k)
-            acc = fmaf(xb[k], w[kOffW1 + k * kH + j], acc);  // exact product
-        z1[j] = __fadd_rn(acc, w[kOffB1 + j]);
-        h1[j] = bf16r(z1[j] > 0.f ? z1[j] : 0.f);
-        h1b[j] = h1[j];
-    }
-    float z3 = 0.f;
-    for (int j = 0; j < kH; ++j) {
-        float acc = 0.f;
+            acc = fmaf(lane_value(xb, k), w1c[k], acc);  // exact product
+        const float z1 = __fadd_rn(acc, b1);
+        const float h1 = bf16r(z1 > 0.f ? z1 : 0.f);
+        acc = 0.f;
+#pragma unroll
         for (int k = 0; k < kH; ++k)
-            acc = fmaf(h1[k], w[kOffW2 + k * kH + j], acc);
-        z2[j] = __fadd_rn(acc, w[kOffB2 + j]);
-        const float h2 = bf16r(z2[j] > 0.f ? z2[j] : 0.f);
-        h2b[j] = h2;
-        z3 = fmaf(h2, w[kOffW3 + j], z3);
-    }
-    z3 = __fadd_rn(z3, w[kOffB3]);
-    const float p = (float)(1.0 / (1.0 + exp(-(double)z3)));
-    const float y = labels[idx] ? 1.f : 0.f;
-    const float eps = 1e-7f;
-    const float lp = logf(p > eps ? p : eps), lq = logf(1.f - p > eps ? 1.f - p : eps);
-    atomicAdd(loss_sum, -(pos_weight * y * lp + (1.f - y) * lq));
-    // dL/dz3 of the mean loss
-    const float dz3 = __fdiv_rn(
-        __fsub_rn(__fmul_rn(__fsub_rn(1.f, y), p),
-                  __fmul_rn(__fmul_rn(pos_weight, y), __fsub_rn(1.f, p))),
-        (float)B);
-    row[kScratchRow - 1] = dz3;
-    for (int j = 0; j < kH; ++j) {
-        const float dh2 = __fmul_rn(dz3, w[kOffW3 + j]);
-        dz2[j] = z2[j] > 0.f ? dh2 : 0.f;
-    }
-    for (int i = 0; i < kH; ++i) {
-        float acc = 0.f;
+            acc = fmaf(lane_value(h1, k), w2c[k], acc);
+        const float z2 = __fadd_rn(acc, b2);
+        const float h2 = bf16r(z2 > 0.f ? z2 : 0.f);
+        float z3 = 0.f;
+#pragma unroll
         for (int k = 0; k < kH; ++k)
-            acc = __fadd_rn(acc, __fmul_rn(dz2[k], w[kOffW2 + i * kH + k]));
-        dz1[i] = z1[i] > 0.f ? acc : 0.f;
+            z3 = fmaf(lane_value(h2, k), lane_value(w3, k), z3);
+        z3 = __fadd_rn(z3, wb[kOffB3]);
+        const float p = (float)(1.0 / (1.0 + exp(-(double)z3)));
+        const float y = labels[idx] ? 1.f : 0.f;
+        // dL/dz3 of the mean loss
+        const float dz3 = __fdiv_rn(
+            __fsub_rn(__fmul_rn(__fsub_rn(1.f, y), p),
+                      __fmul_rn(__fmul_rn(pos_weight, y),
+                                __fsub_rn(1.f, p))),
+            (float)B);
+        const float dh2 = __fmul_rn(dz3, w3);
+        const float dz2 = z2 > 0.f ? dh2 : 0.f;
+        acc = 0.f;
+#pragma unroll
+        for (int k = 0; k < kH; ++k)
+            acc = __fadd_rn(acc, __fmul_rn(lane_value(dz2, k), w2r[k]));
+        if (j < kNF)
+            row[j] = xb;
+        row[kNF + j] = h1;
+        row[kNF + kH + j] = h2;
+        row[kNF + 2 * kH + j] = z1 > 0.f ? acc : 0.f;
+        row[kNF + 3 * kH + j] = dz2;
+        if (j == 0) {
+            row[kScratchRow - 1] = dz3;
+            const float eps = 1e-7f;
+            const float lp = logf(p > eps ? p : eps),
+                        lq = logf(1.f - p > eps ? 1.f - p : eps);
+            loss += -(pos_weight * y * lp + (1.f - y) * lq);
+        }
+    }
+    // one atomic per workgroup (one per sample took 40 us of the kernel)
+    __shared__ float part[kTrainWaves];
+    if (j == 0)
+        part[threadIdx.x >> 6] = loss;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kTrainWaves; ++w)
+            loss += part[w];
+        atomicAdd(loss_sum, loss);
     }
 }
 
-// One thread per parameter: sums over the batch in sample order.
-__global__ void k_train_wgrad(const float *__restrict__ scratch, uint32_t B,
-                              float *__restrict__ grad)
+// Sums over the batch in sample order, one thread per parameter; a wave has
+// the 64 parameters that share one factor: row i of W1 or W2 (factors xb[i]
+// or h1b[i], and dz1 or dz2), w3 (dz3 and h2b), or a bias (no factor).  What
+// bounds it is the chain of B additions, so two tiles of samples are on
+// their way (64 consecutive floats a row) while a third is summed:
+// 1000 us per batch of 4096 with a load between the additions, now 100.
+constexpr int kWgTile = 64;
+constexpr int kWgBlocks = kNF + 1 + kH + 1 + 1 + 1;
+
+__global__ __launch_bounds__(64) void k_train_wgrad(
+    const float *__restrict__ scratch, uint32_t B, float *__restrict__ grad)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kNParam)
-        return;
     // row offsets: xb 0, h1b kNF, h2b kNF+kH, dz1 kNF+2kH, dz2 kNF+3kH,
     // dz3 kScratchRow-1; ao = -1 marks a bias (single factor)
     constexpr int oH1 = kNF, oH2 = kNF + kH, oD1 = kNF + 2 * kH,
                   oD2 = kNF + 3 * kH, oD3 = kScratchRow - 1;
-    int ao, bo;
-    if (p < kOffB1) {          // W1[i][j] += xb[i] * dz1[j]
-        ao = p / kH; bo = oD1 + p % kH;
-    } else if (p < kOffW2) {   // b1[j] += dz1[j]
-        ao = -1; bo = oD1 + (p - kOffB1);
-    } else if (p < kOffB2) {   // W2[i][j] += h1b[i] * dz2[j]
-        const int q = p - kOffW2;
-        ao = oH1 + q / kH; bo = oD2 + q % kH;
-    } else if (p < kOffW3) {   // b2[j] += dz2[j]
-        ao = -1; bo = oD2 + (p - kOffB2);
-    } else if (p < kOffB3) {   // w3[i] += h2b[i] * dz3
-        ao = oH2 + (p - kOffW3); bo = oD3;
-    } else {                   // b3 += dz3
-        ao = -1; bo = oD3;
+    const int j = threadIdx.x & 63;
+    int b = blockIdx.x, ao = -1, bo, out, nout = 64;
+    if (b < kNF) {                      // W1[b][j] += xb[b] * dz1[j]
+        ao = b; bo = oD1 + j; out = kOffW1 + b * kH + j;
+    } else if ((b -= kNF) == 0) {       // b1[j] += dz1[j]
+        bo = oD1 + j; out = kOffB1 + j;
+    } else if ((b -= 1) < kH) {         // W2[b][j] += h1b[b] * dz2[j]
+        ao = oH1 + b; bo = oD2 + j; out = kOffW2 + b * kH + j;
+    } else if ((b -= kH) == 0) {        // b2[j] += dz2[j]
+        bo = oD2 + j; out = kOffB2 + j;
+    } else if (b == 1) {                // w3[j] += h2b[j] * dz3
+        ao = oD3; bo = oH2 + j; out = kOffW3 + j;
+    } else {                            // b3 += dz3
+        bo = oD3; out = kOffB3; nout = 1;
     }
-    float acc = 0.f;
-    for (uint32_t s = 0; s < B; ++s) {
-        const float *row = scratch + (size_t)s * kScratchRow;
-        const float v = ao >= 0 ? __fmul_rn(row[ao], row[bo]) : row[bo];
-        acc = __fadd_rn(acc, v);
+    const bool one = ao < 0;
+    // factor of sample s0 + lane, values of the tile's samples; samples past the end repeat the last one and are not summed
+    auto load = [&](uint32_t s0, float &f, float *v) {
+        const uint32_t sa = min(s0 + (uint32_t)j, B - 1);
+        f = one ? 1.f : scratch[(size_t)sa * kScratchRow + ao];
+#pragma unroll
+        for (int t = 0; t < kWgTile; ++t)
+            v[t] = scratch[(size_t)min(s0 + (uint32_t)t, B - 1) *
+                               kScratchRow + bo];
+    };
+    float acc = 0.f, f0, f1, f2, v0[kWgTile], v1[kWgTile], v2[kWgTile];
+    // sums tile s0 from (f, v), then refills them with the tile three on
+    auto tile = [&](uint32_t s0, float &f, float *v) {
+        if (s0 + kWgTile <= B) {
+#pragma unroll
+            for (int t = 0; t < kWgTile; ++t)
+                acc = __fadd_rn(acc, __fmul_rn(lane_value(f, t), v[t]));
+        } else if (s0 < B) {
+#pragma unroll
+            for (int t = 0; t < kWgTile; ++t)
+                if (s0 + t < B)
+                    acc = __fadd_rn(acc, __fmul_rn(lane_value(f, t), v[t]));
+        }
+        if (s0 + 3 * kWgTile < B)
+            load(s0 + 3 * kWgTile, f, v);
+    };
+    load(0, f0, v0);
+    load(min((uint32_t)kWgTile, B - 1), f1, v1);
+    load(min(2u * kWgTile, B - 1), f2, v2);
+    for (uint32_t s0 = 0; s0 < B; s0 += 3 * kWgTile) {
+        tile(s0, f0, v0);
+        tile(s0 + kWgTile, f1, v1);
+        tile(s0 + 2 * kWgTile, f2, v2);
     }
-    grad[p] = acc;
+    if (j < nout)
+        grad[out] = acc;
 }
 
 __global__ void k_adam(float *__restrict__ w, float *__restrict__ m,
@@ -482,10 +551,13 @@ hipError_t train_step(const float *feats, const float *mean,
                       float lr, float beta1, float beta2, float eps, int t,
                       bool update, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_train_fwd_bwd, dim3(nblk(B, 256)), dim3(256), 0, s,
-                       feats, mean, istd, labels, order, base, B, wb, pos_weight, scratch,
+    // four samples per wave at the largest usual batch, so that the weights
+    // are loaded once for several samples
+    const unsigned grid = std::min(nblk(B, kTrainWaves), 256u);
+    hipLaunchKernelGGL(k_train_fwd_bwd, dim3(grid), dim3(64 * kTrainWaves), 0,
+                       s, feats, mean, istd, labels, order, base, B, wb, pos_weight, scratch,
                        loss_sum);
-    hipLaunchKernelGGL(k_train_wgrad, dim3(nblk(kNParam, 64)), dim3(64), 0, s,
+    hipLaunchKernelGGL(k_train_wgrad, dim3(kWgBlocks), dim3(64), 0, s,
                        scratch, B, grad);
     if (update) {
         const float c1 = (float)(1.0 - pow((double)beta1, (double)t));

@@ -85,21 +85,24 @@ int upload_stdz(pa_ctx *c)
 }
 
 // mean and 1/std of every feature over the n samples (double sums in sample
-// order; constant features get istd 1)
+// order; constant features get istd 1).  The features' sums advance together:
+// one at a time each waits for its own additions.
 void standardization(const float *feats, uint64_t n, float *mean, float *istd)
 {
-    for (int k = 0; k < kNF; ++k) {
-        double s = 0.0;
-        for (uint64_t i = 0; i < n; ++i)
-            s += feats[i * kNF + k];
-        const double mu = n ? s / (double)n : 0.0;
-        double q = 0.0;
-        for (uint64_t i = 0; i < n; ++i) {
-            const double d = feats[i * kNF + k] - mu;
-            q += d * d;
+    double s[kNF] = {}, q[kNF] = {}, mu[kNF];
+    for (uint64_t i = 0; i < n; ++i)
+        for (int k = 0; k < kNF; ++k)
+            s[k] += feats[i * kNF + k];
+    for (int k = 0; k < kNF; ++k)
+        mu[k] = n ? s[k] / (double)n : 0.0;
+    for (uint64_t i = 0; i < n; ++i)
+        for (int k = 0; k < kNF; ++k) {
+            const double d = feats[i * kNF + k] - mu[k];
+            q[k] += d * d;
         }
-        const double sd = n ? std::sqrt(q / (double)n) : 0.0;
-        mean[k] = (float)mu;
+    for (int k = 0; k < kNF; ++k) {
+        const double sd = n ? std::sqrt(q[k] / (double)n) : 0.0;
+        mean[k] = (float)mu[k];
         istd[k] = sd > 1e-6 ? (float)(1.0 / sd) : 1.0f;
     }
 }
