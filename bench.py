@@ -44,7 +44,8 @@ METRIC = ("GCUPS + aligned pairs/s on 1 MI355X; learned-filter vs plain at "
 PEAK_I16_TOPS = 78.6
 PEAK_I32_TOPS = 39.3
 # algorithmic int ops / cell
-OPS_PER_CELL = {"sw": 10, "swt": 10, "nwt": 9, "nwl": 9}
+OPS_PER_CELL = {"sw": 10, "swt": 10, "nwt": 9, "swl": 10, "swtl": 10,
+                "nwl": 9}
 
 
 def log(*a):
@@ -75,8 +76,11 @@ TRAFFIC_PROFILES = {
 
 def rocprof_name(kernel):
     """k_dp<nwt.c3.l64r8.i16> -> void pa::k_dp<8, 64, false, true, true>"""
-    if kernel.startswith("k_dp<nwl."):
-        return "pa::k_nw_linear"
+    linear = {"nwl": "pa::k_nw_linear", "swl": "void pa::k_sw_linear<false>",
+              "swtl": "void pa::k_sw_linear<true>"}
+    mode = kernel[len("k_dp<"):].split(".")[0]
+    if mode in linear:
+        return linear[mode]
     m = re.match(r"k_dp<(sw|swt|nwt)\.c\d\.l(\d+)r(\d+)\.(i16|i32)>", kernel)
     if not m:
         return None

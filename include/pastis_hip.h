@@ -412,9 +412,10 @@ int pa_synchronize(struct pa_ctx *ctx);
  * swt = local traced, nwt = global traced), row class (c0..c3, with the
  * class's current kernel shape, e.g. l64r8 = 64 lanes x 8 rows per lane)
  * and arithmetic (i16 packed, i32); "rerun" classes are the int32 re-runs
- * of saturated tasks.  Example: "nwt.c3.l64r8.i16".  "nwl.r16.i16" is the
- * linear-gap global kernel, which runs all its tasks in one launch.  cells
- * are DP cells of the tasks the class ran. */
+ * of saturated tasks.  Example: "nwt.c3.l64r8.i16".  "swl.r16.i16",
+ * "swtl.r16.i16" and "nwl.r16.i16" are the same modes in the linear-gap
+ * kernels, which run all their tasks in one launch.  cells are DP cells of
+ * the tasks the class ran. */
 typedef struct pa_kernel_stat {
     char name[24];
     uint64_t launches;
@@ -443,11 +444,12 @@ enum pa_dp_shape {
     PA_SHAPE_L8R8 = 5       /* 128 */
 };
 
-/* Global alignments whose gaps are never extended (gap_open > gap_ext) under
- * a matrix with scores 2 gap_open .. 2 gap_open + 15 (BLOSUM62 with gap_open
- * -2, the as-called reading of the reference's defaults) run in a kernel of
- * their own: of the fields below only dp_wg_per_cu and the xd_ ones apply to
- * them. */
+/* Alignments whose gaps are never extended (gap_open > gap_ext, as in the
+ * as-called reading of the reference's defaults) run in linear-gap kernels of
+ * their own: local ones under any matrix whose scores span at most 16 values
+ * with a negative minimum, global ones when that minimum is also 2 gap_open
+ * (BLOSUM62 with gap_open -2).  Of the fields below only dp_wg_per_cu and the
+ * xd_ ones apply to them. */
 typedef struct pa_tuning {
     int32_t dp_wg_per_cu;   /* persistent DP workgroups (one wave) per CU,
                                1..32; 0 = as many as occupancy allows */

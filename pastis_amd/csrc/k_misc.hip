@@ -189,7 +189,7 @@ __device__ inline int bin_key(const DpTask &t, const BinArgs &a)
     int bin;
     uint32_t steps;
     if (LIN) {
-        bin = lin_class(t.qlen);
+        bin = lin_class(t.qlen, t.tlen);
         steps = (t.qlen - 1) / kLinRows * (t.tlen + 127u) + t.tlen +
                 2u * (lin_last_lanes(t.qlen) - 1u) + 1u;
     } else {

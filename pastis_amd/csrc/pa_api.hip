@@ -90,7 +90,8 @@ enum {
     C_LIN = 36,         // linear-gap classes: list lengths, starts, queues
     C_LINS = C_LIN + kLinClasses,
     C_LINQ = C_LINS + kLinClasses,
-    C_HIST = C_LINQ + kLinClasses,   // histogram of the counting sort
+    C_LINP = C_LINQ + kLinClasses,   // items of the pipelined class
+    C_HIST,             // histogram of the counting sort
     C_FILL = C_HIST + kMaxBins * kBuckets,   // its running slots
     C_N = C_FILL + kMaxBins * kBuckets
 };
@@ -163,7 +164,12 @@ void resolve_timers(pa_ctx *c)
         case 1: c->stats.ms_xdrop += ms; break;
         case 2: c->stats.ms_nw += ms; break;
         case 3: c->stats.ms_trace += ms; break;
-        case 5: c->klin.ms += ms; c->klin.launches++; break;
+        case 5:
+        case 6:
+        case 7:
+            c->klin[t.kind - 5].ms += ms;
+            c->klin[t.kind - 5].launches++;
+            break;
         default: c->stats.ms_total += ms; break;
         }
         c->free_events.push_back(t.a);
@@ -223,26 +229,46 @@ int xd_grid(pa_ctx *c, uint64_t nitems)
         1, std::min<uint64_t>((nitems + 63) / 64, (uint64_t)c->ncu * per_cu));
 }
 
-// Persistent grid of the linear-gap kernel and its boundary-row stride.
-int lin_grid(pa_ctx *c, uint64_t ntasks)
+// Linear-gap kernels: persistent grid, boundary-row slots of the pipelined
+// class (any number from 2 on is correct; twice the grid never waits for a
+// slot) and their sizes in c->bnd: the progress words, then the rows.
+struct LinLayout {
+    uint32_t grid, slots, words;
+    size_t prog_bytes() const { return (size_t)slots * 16; }
+    size_t bytes() const
+    {
+        return prog_bytes() + (size_t)(slots + grid) * words * 8;
+    }
+};
+
+bool use_linear(const pa_ctx *c, bool local)
 {
-    int per_cu = nw_linear_occupancy();
-    if (c->tune.dp_wg_per_cu > 0)
-        per_cu = std::min(per_cu, (int)c->tune.dp_wg_per_cu);
-    return (int)std::max<uint64_t>(
-        1, std::min<uint64_t>(ntasks, (uint64_t)c->ncu * per_cu));
+    return local ? c->lin_local : c->lin_global;
 }
 
-uint32_t lin_bnd_stride(const pa_ctx *c)
+LinLayout lin_layout(pa_ctx *c, bool local, bool trace)
 {
-    return (c->max_clen + kLinBndPad + 15u) & ~15u;
+    int per_cu = dp_linear_occupancy(local, trace);
+    if (c->tune.dp_wg_per_cu > 0)
+        per_cu = std::min(per_cu, (int)c->tune.dp_wg_per_cu);
+    LinLayout l;
+    l.grid = (uint32_t)(c->ncu * per_cu);
+    l.slots = 2 * l.grid;
+    l.words = (c->max_clen + 1u) / 2u + kLinBndPad;
+    if (c->slot_cap > 0) {   // a workspace of fixed size (pa_noalloc.hip)
+        const uint64_t fit = c->bnd.cap / ((size_t)l.words * 8 + 16);
+        l.slots = (uint32_t)std::max<uint64_t>(
+            2, std::min<uint64_t>(l.slots, fit / 8));
+        l.grid = (uint32_t)std::max<uint64_t>(
+            1, std::min<uint64_t>(l.grid, fit - l.slots));
+    }
+    return l;
 }
 
 int ensure_bnd(pa_ctx *c, bool local, bool trace)
 {
-    if (!local && c->lin_ok)
-        return grow(c, c->bnd,
-                    (size_t)lin_grid(c, ~0ull) * lin_bnd_stride(c));
+    if (use_linear(c, local))
+        return grow(c, c->bnd, lin_layout(c, local, trace).bytes());
     // one boundary row per task slot of the persistent workgroups of the
     // run's DP grids: per class, its grid (dp_grid) times the task slots of
     // its shape's one-wave workgroup
@@ -306,7 +332,8 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
         return rc;
     // a fill kernel, not a memset node, so that the sequence can be captured
     HIPCHK(c, fill_u32(P<uint32_t>(c->tflags), 0, (uint32_t)((nt + 3) / 4), s));
-    const bool lin = !local && c->lin_ok;
+    const bool lin = use_linear(c, local);
+    const LinLayout ll = lin ? lin_layout(c, local, trace) : LinLayout{};
     std::vector<std::pair<uint64_t, uint64_t>> chunks;
     std::vector<uint64_t> chunk_base;   // trace offset of each chunk's first
     if (trace && c->g_chunks > 0) {
@@ -449,7 +476,7 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
                           P<DpTask>(c->tasks), a, b, lists, ctr + C_LIN,
                           ctr + C_LINS, ctr + C_HIST, ctr + C_FILL,
                           (unsigned long long *)P<uint64_t>(c->bincells) +
-                              kModes * kBins,
+                              (kModes + dmode) * kBins,
                           s, rng));
         else
             HIPCHK(c, bin_tasks(P<DpTask>(c->tasks), a, b, c->shapes,
@@ -470,24 +497,40 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
             la.counts = ctr + C_LIN;
             la.starts = ctr + C_LINS;
             la.queues = ctr + C_LINQ;
-            la.pmat = (const uint32_t *)(P<int8_t>(c->dmat) + kPmatRot);
+            la.mat = P<int8_t>(c->dmat);
             la.out = P<DpOut>(c->dpout);
-            la.trace = P<uint8_t>(c->trace) - base;
-            la.trace_off = P<uint64_t>(c->toffs);
+            la.trace = trace ? P<uint8_t>(c->trace) - base : nullptr;
+            la.trace_off = trace ? P<uint64_t>(c->toffs) : nullptr;
             la.trace_base = tbase;
-            la.bnd = P<uint8_t>(c->bnd);
-            la.bnd_stride = lin_bnd_stride(c);
+            la.prog = P<uint64_t>(c->bnd);
+            la.bnd = P<uint64_t>(c->bnd) + 2 * ll.slots;
+            la.bnd_words = ll.words;
+            la.pipe_slots = ll.slots;
+            la.pipe_start = lists + nt;
+            la.pipe_items = ctr + C_LINP;
+            la.sat_list = sat;
+            la.sat_count = ctr + C_SAT;
+            la.sat_queue = ctr + C_SATQ;
+            la.tflags = P<uint8_t>(c->tflags);
+            la.reruns = (unsigned long long *)P<uint64_t>(c->cells) + 2;
             la.gap = c->cfg.gap_open;
+            la.nib_min = c->nib_min;
+            const uint32_t grid = std::min(b - a, ll.grid);
             {
                 Scope sc(c, kind, s);
-                Scope k(c, 5, s);
-                HIPCHK(c, launch_nw_linear(la, lin_grid(c, b - a), s));
+                Scope k(c, 5 + dmode, s);
+                // progress words of the pipelined items: none yet
+                HIPCHK(c, fill_u32((uint32_t *)la.prog, 0, 2 * ll.slots, s));
+                HIPCHK(c, launch_dp_linear(la, local, trace, (int)grid,
+                                           (int)std::min(
+                                               grid, (uint32_t)c->ncu),
+                                           s));
             }
-            {
+            if (trace) {
                 Scope sc(c, 3, s);
-                HIPCHK(c, launch_traceback_linear(la, b - a, s));
+                HIPCHK(c, launch_traceback_linear(la, local, b - a, s));
             }
-            c->stats.launches += 2;
+            c->stats.launches += trace ? 2 : 1;
             continue;
         }
         DpArgs args{};
@@ -1139,13 +1182,15 @@ int pa_create(const pa_config *cfg, pa_ctx **out)
                 (int8_t)(c->nib_ok && q < kAlpha && x < kAlpha
                              ? c->mat[q * 32 + x] - lo
                              : 0);
-    // the nibbles of the linear-gap kernel, shifted and rotated (kPmatRot)
-    c->lin_ok = c->nib_ok && c->cfg.gap_open > c->cfg.gap_ext &&
-                lo == 2 * c->cfg.gap_open;
+    // the linear-gap kernels' forms of the nibbles (kPmatRot, kPmatPair)
+    c->lin_local = c->nib_ok && c->cfg.gap_open > c->cfg.gap_ext;
+    c->lin_global = c->lin_local && lo == 2 * c->cfg.gap_open;
     for (int k = 0; k < 1024; ++k) {
         const int n = dm[kPmatNib + k] & 15;
         dm[kPmatRot + k] = (int8_t)(n << 2);
         dm[kPmatRot + 1024 + k] = (int8_t)(((n & 3) << 6) | (n >> 2));
+        dm[kPmatPair + k] = (int8_t)n;
+        dm[kPmatPair + 1024 + k] = (int8_t)(n << 4);
     }
     c->shapes = shapes_for(c, c->tune);
     if (grow(c, c->dmat, kPmatBytes) ||
@@ -1154,8 +1199,8 @@ int pa_create(const pa_config *cfg, pa_ctx **out)
         pa_destroy(c);
         return PA_ERR_NOMEM;
     }
-    if (grow(c, c->bincells, (kModes + 1) * kBins * sizeof(uint64_t)) ||
-        hipMemset(c->bincells.p, 0, (kModes + 1) * kBins * sizeof(uint64_t)) !=
+    if (grow(c, c->bincells, 2 * kModes * kBins * sizeof(uint64_t)) ||
+        hipMemset(c->bincells.p, 0, 2 * kModes * kBins * sizeof(uint64_t)) !=
             hipSuccess ||
         grow(c, c->cells, 4 * sizeof(uint64_t)) ||
         hipMemset(c->cells.p, 0, 4 * sizeof(uint64_t)) != hipSuccess) {
@@ -1810,9 +1855,10 @@ int pa_reset_stats(pa_ctx *c)
             k = pa_ctx::KStat{};
     if (c->cells.p)
         HIPCHK(c, hipMemset(c->cells.p, 0, 32));
-    c->klin = pa_ctx::KStat{};
+    for (auto &k : c->klin)
+        k = pa_ctx::KStat{};
     HIPCHK(c, hipMemset(c->bincells.p, 0,
-                        (kModes + 1) * kBins * sizeof(uint64_t)));
+                        2 * kModes * kBins * sizeof(uint64_t)));
     return PA_OK;
 }
 
@@ -1823,7 +1869,7 @@ int pa_get_kernel_stats(pa_ctx *c, pa_kernel_stat *out, int cap, int *n)
     hipSetDevice(c->device);
     HIPCHK(c, hipStreamSynchronize(c->st));
     resolve_timers(c);
-    uint64_t cells[(kModes + 1) * kBins];
+    uint64_t cells[2 * kModes * kBins];
     HIPCHK(c, hipMemcpy(cells, c->bincells.p, sizeof(cells),
                         hipMemcpyDeviceToHost));
     static const char *mname[3] = {"sw", "swt", "nwt"};
@@ -1854,15 +1900,19 @@ int pa_get_kernel_stats(pa_ctx *c, pa_kernel_stat *out, int cap, int *n)
             }
             ++k;
         }
-    if (c->klin.launches) {
+    for (int m = 0; m < 3; ++m) {
+        if (!c->klin[m].launches)
+            continue;
         if (k < cap) {
+            static const char *lname[3] = {"swl", "swtl", "nwl"};
             pa_kernel_stat &o = out[k];
             std::memset(&o, 0, sizeof(o));
-            std::snprintf(o.name, sizeof(o.name), "nwl.r%d.i16", kLinR);
-            o.launches = c->klin.launches;
-            o.ms = c->klin.ms;
+            std::snprintf(o.name, sizeof(o.name), "%s.r%d.i16", lname[m],
+                          kLinR);
+            o.launches = c->klin[m].launches;
+            o.ms = c->klin[m].ms;
             for (int b = 0; b < kBins; ++b)
-                o.cells += cells[kModes * kBins + b];
+                o.cells += cells[(kModes + m) * kBins + b];
         }
         ++k;
     }

@@ -17,8 +17,8 @@ struct Buf {
 };
 
 struct Timer {
-    int kind;  // 0 sw, 1 xdrop, 2 nw, 3 trace, 4 total, 5 linear kernel,
-               // 100 + 16 * mode + bin: a DP kernel class
+    int kind;  // 0 sw, 1 xdrop, 2 nw, 3 trace, 4 total, 5 + mode: a linear
+               // kernel, 100 + 16 * mode + bin: a DP kernel class
     hipEvent_t a, b;
 };
 
@@ -96,7 +96,7 @@ struct pa_ctx {
         uint64_t launches = 0;
         double ms = 0;
     } kstat[3][pa::kBins + pa::kClasses];   // DP mode x (bins, int32 re-runs)
-    KStat klin;                   // linear-gap global kernel, all classes
+    KStat klin[3];   // linear-gap kernels, all classes, by DP mode
     std::vector<Timer> pending;
     std::vector<hipEvent_t> free_events;
     pa_stats stats{};
@@ -138,11 +138,11 @@ struct pa_ctx {
     // .. nib_min + 15; if not, shapes replaces the 4-bit-profile shapes
     bool nib_ok = true;
     int nib_min = 0;
-    // the global alignments run in the linear-gap kernel (k_dp_linear.h):
-    // gaps never extended (open > ext) and score - 2 open within 0 .. 15
-    // over the alphabet, starting at 0 (BLOSUM62 with open -2, the
-    // as-called reading of -g -11 -e -2)
-    bool lin_ok = false;
+    // gaps are never extended (open > ext) and the matrix fits 4 bits: the
+    // local alignments run in the linear-gap kernels (k_dp_linear.h), the
+    // global ones too when scores - 2 open are 0 .. 15 (BLOSUM62 with open
+    // -2, the as-called reading of -g -11 -e -2)
+    bool lin_local = false, lin_global = false;
     // No event timers (pa_sw_scores_noalloc: event objects are allocated).
     bool quiet = false;
     // Cap on the task slots (boundary rows) of a DP grid (0 = none); the

@@ -82,10 +82,11 @@ constexpr uint32_t kTaskSat = 1u;  // int16 saturated, needs the int32 re-run
 // 11); with any other matrix the context runs their 4-row counterparts.
 constexpr size_t kPmatUntraced = 1024, kPmatLocal = 2048, kPmatGlobal = 3072,
                  kPmatNib = 4096;
-// Profiles of the linear-gap kernel (k_dp_linear.h): kPmatRot gives the same
-// nibble n as n << 2, the 1 KB after it as n rotated to bits 6, 7, 0, 1.
-constexpr size_t kPmatRot = 5120;
-constexpr size_t kPmatBytes = 7168;
+// Profiles of the linear-gap kernels (k_dp_linear.h), two tables each, for
+// the two rows of a profile byte.  Traced: the same nibble n as n << 2, and n
+// rotated to bits 6, 7, 0, 1; score only: n and n << 4.
+constexpr int kPmatRot = 5120, kPmatPair = 7168;
+constexpr size_t kPmatBytes = 9216;
 // Global task whose scores are bounded by the residue bound below (no cell
 // exceeds min over the two spans of the sum of each residue's best score),
 // small enough for the traced int16 kernels.
@@ -264,12 +265,23 @@ __host__ __device__ inline uint64_t trace_rec(uint32_t qlen, uint32_t tlen,
 // The counts are those where the tasks of a wave change (64 / L), so few
 // lanes stay idle: rows are rounded up to 32, lanes to 60 .. 64 per wave.
 constexpr int kLinR = 16;
-constexpr int kLinClasses = 15;
+constexpr int kLinClasses = 16;
+// class whose tasks' passes run on a wave each, one behind the other: more
+// than one pass, and columns enough to hide the 200 or so by which a pass
+// follows the one before (a short task keeps its passes on one wave)
+constexpr int kLinPipe = kLinClasses - 1;
+constexpr uint32_t kLinPipeCols = 2048;
 constexpr int kLinRows = 2 * kLinR * 64;
 // bytes of one trace record: the 2-bit codes of a lane's rows at one step
 constexpr int kLinRec = kLinR / 2;
-// bytes of a boundary row besides its columns (k_dp_linear.h)
-constexpr uint32_t kLinBndPad = 288;
+// 8-byte words of a boundary row besides its columns (two a word)
+constexpr uint32_t kLinBndPad = 80;
+// Scores from which a result counts as re-run in int32 (what 16 bits hold),
+// and the lower ones from which the linear-gap kernels run a task again: their
+// maximum is taken in half-float order, below 0x7c00, and a step adds at most
+// 14 to a score.
+constexpr int kSat = 32766, kSatTraced = 8190;
+constexpr int kLinSat = 0x7c00 - 16, kLinSatTraced = 0x7c00 / 4 - 16;
 
 __host__ __device__ inline int lin_lanes(int cls)
 {
@@ -280,8 +292,10 @@ __host__ __device__ inline int lin_lanes(int cls)
            : cls == 13 ? 32
                        : 64;
 }
-__host__ __device__ inline int lin_class(uint32_t qlen)
+__host__ __device__ inline int lin_class(uint32_t qlen, uint32_t tlen)
 {
+    if (qlen > kLinRows && tlen >= kLinPipeCols)
+        return kLinPipe;
     const uint32_t need = (qlen + 2u * kLinR - 1u) / (2u * kLinR);
     return need <= 10   ? (int)need - 1
            : need <= 12 ? 10
@@ -319,19 +333,29 @@ struct LinArgs {
     const uint32_t *starts;
     const uint32_t *counts;
     uint32_t *queues;
-    const uint32_t *pmat;       // kPmatRot
+    const int8_t *mat;          // scoring matrix and profile tables (kPmat*)
     DpOut *out;
     uint8_t *trace;
     const uint64_t *trace_off;
     const uint64_t *trace_base; // as DpArgs::trace_base
-    uint8_t *bnd;               // boundary rows, one per workgroup
-    uint32_t bnd_stride;
-    int32_t gap;
+    // boundary rows of bnd_words words: pipe_slots for pipelined passes, then
+    // one per workgroup
+    uint64_t *bnd;
+    uint32_t bnd_words;
+    uint32_t pipe_slots;
+    uint64_t *prog;             // per slot: progress (zeroed), then values
+    uint32_t *pipe_start;       // first item of each pipelined task
+    uint32_t *pipe_items;
+    uint32_t *sat_list, *sat_count, *sat_queue;   // int32 re-runs (local)
+    uint8_t *tflags;
+    unsigned long long *reruns;
+    int32_t gap, nib_min;
 };
-hipError_t launch_nw_linear(const LinArgs &a, int grid, hipStream_t s);
-int nw_linear_occupancy();
-hipError_t launch_traceback_linear(const LinArgs &a, uint32_t ntasks,
-                                   hipStream_t s);
+hipError_t launch_dp_linear(const LinArgs &a, bool local, bool trace, int grid,
+                            int rerun_grid, hipStream_t s);
+int dp_linear_occupancy(bool local, bool trace);
+hipError_t launch_traceback_linear(const LinArgs &a, bool local,
+                                   uint32_t ntasks, hipStream_t s);
 
 // X-drop extension task: one seed of one pair.
 struct XdTask {

@@ -30,7 +30,7 @@ constexpr int kMaxSlots = 1024;            // boundary rows of kMaxLen
 constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Regions of the scratch array (byte offsets), sized for kMaxPairs pairs.
-constexpr size_t kCtrWords = 2048;         // >= the counter block's words
+constexpr size_t kCtrWords = 4096;         // >= the counter block's words
 constexpr size_t kOffTasks = 0;
 constexpr size_t kOffOut = align256(kOffTasks + kMaxPairs * sizeof(DpTask));
 constexpr size_t kOffFlags = align256(kOffOut + kMaxPairs * sizeof(DpOut));

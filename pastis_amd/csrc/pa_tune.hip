@@ -304,7 +304,7 @@ extern "C" int pa_autotune(pa_ctx *c, const pa_pair *d_pairs, uint64_t n,
     const bool xdrop = target == PA_TUNE_ALIGN && c->cfg.mode == PA_MODE_XDROP;
     // a choice made with the linear-gap kernel says nothing about the shapes
     // of the others
-    const bool lin = xdrop && c->lin_ok;
+    const bool lin = xdrop ? c->lin_global : c->lin_local;
     const auto key =
         std::make_tuple(c->device, target, (int)c->cfg.mode + (lin ? 2 : 0));
     if (!(flags & PA_TUNE_FORCE)) {
