@@ -457,8 +457,9 @@ typedef struct pa_tuning {
     int32_t xd_ring;        /* X-drop LDS ring slots per lane: 16 or 32 */
     int32_t xd_coop;        /* 1: X-drop items go to the 16-lanes-per-item
                                kernel first (band up to 14 columns), the rest
-                               to the one-lane-per-item kernels; 0: one lane
-                               per item only */
+                               to the one-lane-per-item kernels; 0 (default):
+                               by size, 16 lanes per item in small batches
+                               and for far-reaching items, else one */
     int32_t dp_edge[3];     /* DP row classes: a task whose row span has
                                qlen rows is in the first class c with
                                qlen <= dp_edge[c], class 3 takes the rest;

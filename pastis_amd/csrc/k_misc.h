@@ -31,6 +31,13 @@ hipError_t build_xd_tasks(const pa_pair *pairs, uint64_t n, int seed_cnt,
                           int seed_len, const uint64_t *roffs,
                           const uint64_t *coffs, uint64_t nr, uint64_t nc,
                           XdTask *tasks, hipStream_t s);
+// The X-drop work items (2 * task + direction) of nt tasks by falling reach
+// (xd_reach) in `list`, those of long_min and more in long_list instead.
+// hist and fill are kBuckets counters, hist and long_count start at zero.
+hipError_t sort_reach(const XdTask *tasks, uint64_t nt, int seed_len,
+                      uint32_t long_min, uint32_t *hist, uint32_t *fill,
+                      uint32_t *list, uint32_t *count, uint32_t *long_list,
+                      uint32_t *long_count, hipStream_t s);
 hipError_t build_nw_tasks(const XdTask *xt, uint64_t nt, const XdOut *xo,
                           DpTask *tasks, ResBound rows, ResBound cols,
                           unsigned long long *cells,

@@ -111,6 +111,77 @@ __global__ void k_build_xd_tasks(const pa_pair *__restrict__ pairs, uint64_t n,
     tasks[k] = t;
 }
 
+// Bucket of a work item's reach: quarter octaves, the longest first.
+__device__ inline int reach_bucket(uint32_t x)
+{
+    const uint32_t y = x + 4u;   // 2 bits after the leading one
+    const int e = 31 - __builtin_clz(y);
+    const int b = 4 * (e - 2) + (int)((y >> (e - 2)) & 3u);
+    return kBuckets - 1 - (b < kBuckets - 1 ? b : kBuckets - 1);
+}
+
+// Counting sort of the work items (2 * task + direction) by their reach.
+// Pass 1: histogram.  Items of long_min and more are not sorted: they are few
+// and go to a list of their own.
+__global__ __launch_bounds__(256) void k_reach_hist(
+    const XdTask *__restrict__ tasks, uint32_t nt, int seed_len,
+    uint32_t long_min, uint32_t *hist)
+{
+    __shared__ uint32_t h[kBuckets];
+    if (threadIdx.x < kBuckets)
+        h[threadIdx.x] = 0;
+    __syncthreads();
+    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < nt;
+         k += gridDim.x * blockDim.x) {
+        const XdTask t = tasks[k];
+        for (int dir = 0; dir < 2; ++dir) {
+            const uint32_t x = xd_reach(t, dir, seed_len);
+            if (x < long_min)
+                atomicAdd(&h[reach_bucket(x)], 1u);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < kBuckets && h[threadIdx.x])
+        atomicAdd(&hist[threadIdx.x], h[threadIdx.x]);
+}
+
+// Pass 2: each block takes its buckets' places with one atomic a bucket
+// (fill starts as the buckets' exclusive sums, k_bin_scan).
+__global__ __launch_bounds__(256) void k_reach_scatter(
+    const XdTask *__restrict__ tasks, uint32_t nt, int seed_len,
+    uint32_t long_min, uint32_t *fill, uint32_t *__restrict__ list,
+    uint32_t *__restrict__ long_list, uint32_t *long_count)
+{
+    __shared__ uint32_t h[kBuckets], base[kBuckets];
+    if (threadIdx.x < kBuckets)
+        h[threadIdx.x] = 0;
+    __syncthreads();
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    int bucket[2] = {-1, -1};
+    uint32_t rank[2] = {0, 0};
+    if (k < nt) {
+        const XdTask t = tasks[k];
+        for (int dir = 0; dir < 2; ++dir) {
+            const uint32_t x = xd_reach(t, dir, seed_len);
+            if (x < long_min) {
+                bucket[dir] = reach_bucket(x);
+                rank[dir] = atomicAdd(&h[bucket[dir]], 1u);
+            } else {
+                long_list[atomicAdd(long_count, 1u)] = 2 * k + (uint32_t)dir;
+            }
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < kBuckets)
+        base[threadIdx.x] = h[threadIdx.x]
+                                ? atomicAdd(&fill[threadIdx.x], h[threadIdx.x])
+                                : 0u;
+    __syncthreads();
+    for (int dir = 0; dir < 2; ++dir)
+        if (bucket[dir] >= 0)
+            list[base[bucket[dir]] + rank[dir]] = 2 * k + (uint32_t)dir;
+}
+
 // Extension -> global alignment of the extended infixes
 // (globalAlignment(seqsc_ex, seqsr_ex), SeqanXdropAligner.cpp:284-296).
 __global__ void k_build_nw_tasks(const XdTask *__restrict__ xt, uint64_t nt,
@@ -549,6 +620,23 @@ hipError_t build_xd_tasks(const pa_pair *pairs, uint64_t n, int seed_cnt,
     hipLaunchKernelGGL(k_build_xd_tasks, dim3(blocks(n * seed_cnt, 256)),
                        dim3(256), 0, s, pairs, n, seed_cnt, seed_len, roffs,
                        coffs, nr, nc, tasks);
+    return hipGetLastError();
+}
+
+hipError_t sort_reach(const XdTask *tasks, uint64_t nt, int seed_len,
+                      uint32_t long_min, uint32_t *hist, uint32_t *fill,
+                      uint32_t *list, uint32_t *count, uint32_t *long_list,
+                      uint32_t *long_count, hipStream_t s)
+{
+    if (!nt)
+        return hipSuccess;
+    hipLaunchKernelGGL(k_reach_hist, dim3(stride_blocks(nt)), dim3(256), 0, s,
+                       tasks, (uint32_t)nt, seed_len, long_min, hist);
+    hipLaunchKernelGGL(k_bin_scan<1>, dim3(1), dim3(64), 0, s, hist, fill,
+                       count, (uint32_t *)nullptr);
+    hipLaunchKernelGGL(k_reach_scatter, dim3(blocks(nt, 256)), dim3(256), 0, s,
+                       tasks, (uint32_t)nt, seed_len, long_min, fill, list,
+                       long_list, long_count);
     return hipGetLastError();
 }
 

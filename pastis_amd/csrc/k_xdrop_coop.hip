@@ -11,12 +11,22 @@
 //     its own lane and the three live anti-diagonals are three registers;
 //   - the left neighbour (column c-1) is lane c-1 mod 16: one DPP row_ror:1
 //     move; the anti-diagonal maximum is four DPP rotations;
-//   - the new band limits (leading / trailing undefined columns) come from a
-//     ballot of the per-column conditions, read in column order.
+//   - the new band limits (leading / trailing undefined columns) are a row
+//     minimum and a row maximum over the columns that meet the conditions.
+//   - residues come from rings in LDS (the item's next columns and rows, 16
+//     at a time, loaded 16 steps before they are needed), and the score of
+//     the next anti-diagonal is looked up while this one is computed: for the
+//     lane's column and for the one 16 further, which it holds if the band
+//     leaves its column behind.
+// What bounds it is the chain of one anti-diagonal (neighbour, maximum, band
+// limits): about 0.2 us for four items a wave, a quarter of what the per-lane
+// kernel of k_xdrop.hip takes for its 64.  So it runs where the per-lane
+// kernel would leave the chip waiting for single lanes: all items of a small
+// batch, and the items of a large one that may go on for long (run_xdrop).
 // An item whose written range would exceed 16 columns stops and goes to the
-// overflow list; the per-lane kernels of k_xdrop.hip recompute it from
-// scratch.  A row whose item ends takes the next item of the queue at once,
-// so the four rows of a wave stay busy whatever the item lengths.
+// overflow list; the band kernels recompute it from scratch.  A row whose
+// item ends takes the next item of the queue at once, so the four rows of a
+// wave stay busy whatever the item lengths.
 #include <limits.h>
 
 #include "pa_internal.h"
@@ -26,12 +36,17 @@ namespace {
 
 constexpr int32_t kUndef = INT_MIN / 4;
 constexpr int G = 16;   // lanes per item
-constexpr uint32_t kChunk = 32;   // items claimed per queue atomic
+constexpr uint32_t kChunk = 4;    // items claimed per queue atomic
+constexpr int kRing = 128;        // residues per LDS ring (a power of two)
+constexpr int kItems = 16;        // items per workgroup (four waves)
+constexpr int kSteps = 16;        // anti-diagonals between ring refills
 
 // lane (j - k) mod 16 of the same row
 template <int K> __device__ inline int ror(int v)
 {
-    return __builtin_amdgcn_update_dpp(0, v, 0x120 + K, 0xf, 0xf, false);
+    // every lane has a source: no old operand, so that the move folds into
+    // the instruction that uses it
+    return __builtin_amdgcn_mov_dpp(v, 0x120 + K, 0xf, 0xf, true);
 }
 
 __device__ inline int row_max(int v)
@@ -52,19 +67,6 @@ __device__ inline int row_min(int v)
     return v;
 }
 
-// 16 bits of a ballot belonging to this lane's row
-__device__ inline uint32_t row_bits(uint64_t b, int row)
-{
-    return (uint32_t)(b >> (16 * row)) & 0xffffu;
-}
-
-// bit k of the result is bit (k + r) mod 16 of m
-__device__ inline uint32_t rot16(uint32_t m, int r)
-{
-    r &= 15;
-    return ((m >> r) | (m << (16 - r))) & 0xffffu;
-}
-
 struct CoopArgs {
     const XdTask *tasks;
     const uint32_t *list;   // work items k = 2 * task + dir, NULL = 0..count
@@ -78,27 +80,60 @@ struct CoopArgs {
 
 enum : int { kNeed = 0, kRun = 1, kDone = 2 };
 
+// These waves hold the batch's longest chains: they issue ahead of the waves
+// they share a SIMD with (beside the per-lane kernel's six, a step took three
+// times as long).
+__device__ inline void xd_first_issue()
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    __builtin_amdgcn_s_setprio(3);
+#endif
+}
+
 __global__ __launch_bounds__(256) void k_xdrop_coop(CoopArgs a)
 {
+    xd_first_issue();
     __shared__ int8_t mat[32 * 32];
+    // residues of columns (q) and rows (d) of each item
+    __shared__ uint8_t rings[2 * kItems * kRing];
     for (int i = threadIdx.x; i < 32 * 32; i += blockDim.x)
         mat[i] = a.mat[i];
+    // (residue codes are below 32: a slot not yet stored must be, too)
+    for (int i = threadIdx.x; i < 2 * kItems * kRing; i += blockDim.x)
+        rings[i] = 0;
     __syncthreads();
     const uint32_t n = *a.count;
     const int lane = threadIdx.x & 63;
     const int j = lane & 15;
     const int row = lane >> 4;
     const int gap = a.gap, X = a.X;
+    uint8_t *const qring = rings + (threadIdx.x >> 4) * (2 * kRing);
+    uint8_t *const dring = qring + kRing;
 
     // row-uniform state of the current item
     int state = kNeed;
     uint32_t k = 0;
-    const uint8_t PA_GLOBAL *qs = nullptr, *ds = nullptr;
     int cols = 0, rows = 0, d = 0, minCol = 0, maxCol = 0, best = 0;
     int off1 = 0, off2 = 0, off3 = 0, l1 = 0, l2 = 0, l3 = 0;
     bool right = false;
     bool invalid = false;   // kXdInvalid task: empty extents
     uint32_t nc = 0;
+    int64_t dgap = 0;       // d * gap, while a border cell is kept
+    bool edge = false;      // one may be
+    // rings: columns 1 .. qfill and rows 1 .. dfill have been stored, the
+    // next 32 columns and 16 rows are on their way (one each per lane)
+    int qfill = 0, dfill = 0, qpre0 = 0, qpre1 = 0, dpre = 0;
+    // residue addresses: column c at qb[qstep * c], row r at db[qstep * r]
+    const uint8_t PA_GLOBAL *qb = nullptr, *db = nullptr;
+    int qstep = 1;
+    int c = 0;              // this lane's column on anti-diagonal d + 1
+    int qv = 0, sc = 0;     // its residue * 32, its score on anti-diagonal d+1
+    auto q_load = [&](int col) {
+        return col < cols ? (int)qb[qstep > 0 ? col : -col] : 0;
+    };
+    auto d_load = [&](int r) {
+        return r < rows ? (int)db[qstep > 0 ? r : -r] : 0;
+    };
     // this lane's values on anti-diagonals d-2, d-1, d
     int A1 = kUndef, A2 = kUndef, A3 = kUndef;
     // items claimed by this wave and not yet handed out: [cbase, cend)
@@ -127,6 +162,7 @@ __global__ __launch_bounds__(256) void k_xdrop_coop(CoopArgs a)
                     const uint32_t idx = cbase + rank;
                     if (idx >= n) {
                         state = kDone;
+                        cols = rows = 0;   // nothing more to load
                     } else {
                         k = a.list ? glb(a.list)[idx] : idx;
                         const XdTask T = a.tasks[k >> 1];
@@ -135,15 +171,17 @@ __global__ __launch_bounds__(256) void k_xdrop_coop(CoopArgs a)
                         const int beg_h = (int)T.beg_h, beg_v = (int)T.beg_v;
                         right = (k & 1) != 0;
                         if (!right) {   // query V[0, beg_v), database H[0, beg_h)
-                            qs = v;
                             cols = beg_v + 1;
-                            ds = h;
                             rows = beg_h + 1;
+                            qb = v + beg_v;
+                            db = h + beg_h;
+                            qstep = -1;
                         } else {        // suffixes after the seed
-                            qs = v + beg_v + a.seed_len;
                             cols = (int)T.nv - beg_v - a.seed_len + 1;
-                            ds = h + beg_h + a.seed_len;
                             rows = (int)T.nh - beg_h - a.seed_len + 1;
+                            qb = v + beg_v + a.seed_len - 1;
+                            db = h + beg_h + a.seed_len - 1;
+                            qstep = 1;
                         }
                         // anti-diagonal 0: column 0 = 0; anti-diagonal 1:
                         // columns 0 and 1 = gap (undefined when -gap > X)
@@ -159,9 +197,26 @@ __global__ __launch_bounds__(256) void k_xdrop_coop(CoopArgs a)
                         l3 = 2;
                         best = 0;
                         nc = 0;
+                        dgap = gap;
+                        edge = -gap <= X;
                         state = kRun;
-                        if ((T.pad & kXdInvalid) || rows <= 1 || cols <= 1)
+                        if ((T.pad & kXdInvalid) || rows <= 1 || cols <= 1) {
                             state = 3;   // finished without an update
+                        } else {
+                            const int f = 1 + j;
+                            qring[f] = (uint8_t)q_load(f);
+                            qring[f + 16] = (uint8_t)q_load(f + 16);
+                            dring[f] = (uint8_t)d_load(f);
+                            qpre0 = q_load(f + 32);
+                            qpre1 = q_load(f + 48);
+                            dpre = d_load(f + 16);
+                            qfill = 32;
+                            dfill = 16;
+                            // anti-diagonal 2: column 1, row 1 only
+                            c = j;
+                            qv = q_load(max(j, 1)) << 5;
+                            sc = mat[qv | d_load(1)];
+                        }
                         invalid = (T.pad & kXdInvalid) != 0;
                     }
                 }
@@ -173,85 +228,99 @@ __global__ __launch_bounds__(256) void k_xdrop_coop(CoopArgs a)
         if (!__ballot(state != kDone))
             break;
 
-        // ---- one anti-diagonal for running rows whose band is not empty
-        const bool run = state == kRun && minCol < maxCol;
-        // the written range of the new anti-diagonal is [minCol-1, maxCol]
-        const bool ovf = run && maxCol - minCol + 2 > G;
-        const bool step = run && !ovf;
-        int nd = d + 1;
-        int noff3 = minCol - 1;
-        int nl3 = maxCol + 1 - noff3;
-        // this lane's column on the new anti-diagonal
-        const int c = noff3 + ((j - noff3) & 15);
-        const bool inr = c <= maxCol;
-        const bool comp = inr && c >= minCol && c < maxCol;
-        // left neighbours: column c-1 on anti-diagonal d (A3) and d-1 (A2);
-        // column c on d is this lane's A3 (the written ranges nest, so these
-        // registers hold exactly those columns wherever they are read)
-        const int lA3 = ror<1>(A3);
-        const int lA2 = ror<1>(A2);
-        int v = kUndef;
-        {
-            const int lim = best - X;
-            const bool ld = comp && step;
-            const int qp = right ? c - 1 : cols - 1 - c;
-            const int dp = right ? nd - c - 1 : rows - 1 + c - nd;
-            // rows without a live item read a byte of the score table
-            const uint8_t PA_GLOBAL *qa =
-                ld ? qs + qp : glb((const uint8_t *)a.mat);
-            const uint8_t PA_GLOBAL *da =
-                ld ? ds + dp : glb((const uint8_t *)a.mat);
-            const int sc = mat[(int)(*qa & 31) * 32 + (*da & 31)];
-            int tmp = max(lA3, A3) + gap;
-            tmp = max(tmp, lA2 + sc);
-            const int cv = tmp < lim ? kUndef : tmp;
-            const bool edge_ok = (long)nd * gap > (long)best - X;
-            const int ev_lo = edge_ok && noff3 == 0 ? nd * gap : kUndef;
-            const int ev_hi = edge_ok && nd == maxCol ? nd * gap : kUndef;
-            v = c == noff3 ? ev_lo : (c == maxCol ? ev_hi : (comp ? cv : kUndef));
+        // ---- residues of the next kSteps anti-diagonals: they read columns
+        // up to minCol + 61 (a band moves up by a column a step and at most
+        // its own width more) and rows up to d + 19 - minCol
+        if (qfill < minCol + 62) {
+            qring[(qfill + 1 + j) & (kRing - 1)] = (uint8_t)qpre0;
+            qring[(qfill + 17 + j) & (kRing - 1)] = (uint8_t)qpre1;
+            qfill += 32;
+            qpre0 = q_load(qfill + 1 + j);
+            qpre1 = q_load(qfill + 17 + j);
         }
-        // anti-diagonal best: d*gap or better defined computed cells
-        const int adb = row_max(comp ? v : INT_MIN);
-        // minCol: first column c >= minCol (column order) where the run of
-        // cells undefined on the new anti-diagonal and (column c-1) on d
-        // stops; column c-1 lies on d's written range [off3, off3+l3) or
-        // the run stops there
-        const bool stop = !(v == kUndef && c - 1 - off3 < l3 && lA3 == kUndef);
-        const uint32_t mlo = row_bits(__ballot(inr && c >= minCol && stop), row);
-        // maxCol: last c in [off, maxCol-1] defined on the new anti-diagonal
-        // or on d
-        const bool keep = v != kUndef || A3 != kUndef;
-        const uint32_t mhi = row_bits(__ballot(inr && c < maxCol && keep), row);
-        if (step) {
-            const uint32_t olo = rot16(mlo, noff3);  // bit i = column off3 + i
-            const uint32_t ohi = rot16(mhi, noff3);
-            // lowest set bit at or above minCol - off3 = 1
-            const uint32_t lo1 = olo & ~1u;
-            const int nmin = lo1 ? noff3 + __builtin_ctz(lo1) : maxCol + 1;
-            const int nmax = ohi ? noff3 + 31 - __builtin_clz(ohi) + 1 : noff3;
-            best = max(best, max(adb, nd * gap));
+        if (dfill < d + 20 - minCol) {
+            dring[(dfill + 1 + j) & (kRing - 1)] = (uint8_t)dpre;
+            dfill += 16;
+            dpre = d_load(dfill + 1 + j);
+        }
+        // ---- kSteps anti-diagonals, or until a row's band is empty or too
+        // wide.  Rows without an item compute on (their results go nowhere):
+        // with the updates under a condition the compiler copies the whole
+        // state twice a step.
+        bool fin = state != kDone && !(state == kRun && minCol < maxCol);
+        uint64_t any = __ballot(fin);
+        for (int st = 0; st < kSteps && !any; ++st) {
+            // the written range of the new anti-diagonal is [minCol-1, maxCol]
+            const bool ovf = maxCol - minCol + 2 > G;
+            const int noff3 = minCol - 1;
+            const int nl3 = maxCol + 1 - noff3;
+            ++d;
+            // residues of the anti-diagonal after the new one, for this
+            // lane's column (A) and the one 16 further (B)
+            const int ra = d + 1 - c;
+            const int dA = dring[ra & (kRing - 1)];
+            const int dB = dring[(ra - 16) & (kRing - 1)];
+            const int qB = qring[(c + 16) & (kRing - 1)] << 5;
+            const bool ge = c >= minCol, comp = ge && c < maxCol;
+            // left neighbours: column c-1 on anti-diagonal d (A3) and d-1
+            // (A2); column c on d is this lane's A3 (the written ranges nest,
+            // so these registers hold exactly those columns wherever they are
+            // read)
+            const int lA3 = ror<1>(A3);
+            const int lA2 = ror<1>(A2);
+            const int tmp = max(max(lA3, A3) + gap, lA2 + sc);
+            int v = comp && tmp >= best - X ? tmp : kUndef;
+            const int scA = mat[qv | dA], scB = mat[qB | dB];
+            // cells of column 0 and row 0, while the gap to them is kept: d *
+            // gap falls and the limit does not, so once it is not, never again
+            if (__ballot(edge)) {
+                dgap += gap;
+                edge = edge && dgap > (int64_t)best - X;
+                if (edge && !comp && (c == 0 || (c == maxCol && d == maxCol)))
+                    v = (int)dgap;
+            }
+            // anti-diagonal best (best >= 0 > any border cell)
+            const int adb = row_max(v);
+            // minCol: first column c >= minCol where the run of cells
+            // undefined on the new anti-diagonal and (column c-1) on d stops;
+            // column c-1 lies on d's written range [off3, off3+l3) or the run
+            // stops there
+            const bool stop =
+                max(v, lA3) != kUndef || c - 1 - off3 >= l3;
+            const int lo =
+                row_min(ge && c <= maxCol && stop ? c : INT_MAX);
+            // maxCol: last c in [off, maxCol-1] defined on the new
+            // anti-diagonal or on d
+            const int hi =
+                row_max(c < maxCol && max(v, A3) != kUndef ? c : -1);
             nc += (uint32_t)(maxCol - minCol);
+            best = max(best, adb);
             A1 = A2;
             A2 = A3;
             A3 = v;
-            d = nd;
             off1 = off2;
             off2 = off3;
             off3 = noff3;
             l1 = l2;
             l2 = l3;
             l3 = nl3;
-            minCol = max(nmin, nd + 2 - rows);
-            maxCol = min(nmax + 1, cols);
+            minCol = max(min(lo, maxCol + 1), d + 2 - rows);
+            maxCol = min(max(hi + 1, noff3) + 1, cols);
+            // the column of the next anti-diagonal, [minCol - 1, + 16): the
+            // same or the one 16 further
+            const bool up = c < minCol - 1;
+            c += up ? 16 : 0;
+            qv = up ? qB : qv;
+            sc = up ? scB : scA;
+            state = ovf && state == kRun ? 4 : state;
+            fin = state != kDone && (state != kRun || minCol >= maxCol);
+            any = __ballot(fin);
         }
-        if (ovf) {
-            state = 4;   // overflow: recomputed by the per-lane kernels
-        }
+        if (!any)
+            continue;
 
         // ---- finish rows whose band emptied (or that never started)
-        const bool fin = (state == kRun && minCol >= maxCol) || state == 3 ||
-                         state == 4;
-        if (__ballot(fin)) {
+        {
             // longest extension: the last computed column of the last
             // anti-diagonal, then the end of d-1, else the best of d-2
             const int rb = row * 16;

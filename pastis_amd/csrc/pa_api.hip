@@ -98,6 +98,14 @@ enum {
 
 constexpr int kModes = 3;           // DP modes of the kernel statistics
 constexpr int kMaxWgPerCu = 32;     // one-wave workgroups per CU (8 per SIMD)
+// X-drop work items of a batch small enough for 16 lanes per item, and the
+// reach (xd_reach) from which an item of a larger batch gets 16 lanes.  A lane
+// alone takes 0.7 us an anti-diagonal in an idle chip and 3 us beside five
+// other waves, a row of 16 lanes 0.2 us: 1,204 items 1.60 -> 0.28 ms, and in
+// 1.6 M items, where the longest took 8.3 ms, both kernels now end together
+// after 3.3 ms (reaches of 768 and more: 5.4 and 3.5 ms).
+constexpr uint64_t kXdSmall = 65536;
+constexpr uint32_t kXdLong = 512;
 constexpr int kXdWideLanes = 65536;  // lanes of the wide (global scratch) re-run
 constexpr int kXdGraphLanes = 4096;  // its lanes in a captured batch
 
@@ -777,7 +785,8 @@ int run_xdrop(pa_ctx *c, const pa_pair *d_pairs, uint64_t n, hipStream_t s)
         return rc;
     if ((rc = grow(c, c->xdo, 2 * n * sizeof(XdOut))))
         return rc;
-    if ((rc = grow(c, c->ovf, 2 * ni * sizeof(uint32_t))))
+    // two overflow lists and the items' order
+    if ((rc = grow(c, c->ovf, 3 * ni * sizeof(uint32_t))))
         return rc;
     uint32_t *ctr = P<uint32_t>(c->ctr);
     uint32_t *ovf = P<uint32_t>(c->ovf), *lng = ovf + ni;
@@ -787,38 +796,77 @@ int run_xdrop(pa_ctx *c, const pa_pair *d_pairs, uint64_t n, hipStream_t s)
                              P<uint64_t>(c->roffs), P<uint64_t>(c->coffs),
                              c->rlen.size(), c->clen.size(),
                              P<XdTask>(c->xdt), s));
+    // Which kernel takes an item first.  Sixteen lanes per item take a fifth
+    // of the time per anti-diagonal that one lane takes, at four times the
+    // instructions: they run all items of a small batch (kXdSmall) and, in a
+    // larger one, those that may extend far (kXdLong), on the second stream
+    // beside the others, which start in the order of their reach so that the
+    // grid does not end on long ones.  Only while the bands fit 16 columns: a
+    // gap costs -xdrop_gap and an extension ends X below its best, so a band
+    // spans about 2 X / -xdrop_gap columns (9 as called, 49 as documented).
+    const bool thin = c->cfg.xdrop / -c->cfg.xdrop_gap <= 5;
+    const bool small16 = thin && !c->tune.xd_coop && ni <= kXdSmall;
+    const bool two = thin && !c->tune.xd_coop && !small16;
+    uint32_t *const order = lng + ni;
+    if (two)
+        HIPCHK(c, sort_reach(P<XdTask>(c->xdt), nt, c->cfg.seed_len, kXdLong,
+                             ctr + C_HIST, ctr + C_FILL, order,
+                             ctr + C_XDN, lng, ctr + C_XDLONG, s));
+    auto coop = [&](const uint32_t *list, uint32_t *count, uint32_t *queue,
+                    uint64_t most, uint32_t *to, uint32_t *to_n,
+                    hipStream_t cs) -> int {
+        const int cg = (int)std::max<uint64_t>(
+            1, std::min<uint64_t>((most + 15) / 16,
+                                  (uint64_t)c->ncu *
+                                      std::min(xdrop_coop_occupancy(),
+                                               kMaxWgPerCu / 4)));
+        HIPCHK(c, launch_xdrop_coop(P<XdTask>(c->xdt), list, count, queue,
+                                    P<int8_t>(c->dmat), c->cfg.xdrop_gap,
+                                    c->cfg.xdrop, c->cfg.seed_len,
+                                    P<XdOut>(c->xdo), to, to_n, cg, cs));
+        c->stats.launches++;
+        return PA_OK;
+    };
     {
         Scope t(c, 1, s);
         const int grid = xd_grid(c, ni);
-        if (c->tune.xd_coop) {
+        if (small16) {
+            if ((rc = coop(nullptr, ctr + C_XDN, ctr + C_XDQ, ni, ovf,
+                           ctr + C_XDOVF, s)))
+                return rc;
+        } else if (c->tune.xd_coop) {
             // 16 lanes per item first; items with a wider band go to the
             // one-lane-per-item kernel through the `lng` list
-            const int cg = (int)std::max<uint64_t>(
-                1, std::min<uint64_t>((ni + 3) / 4,
-                                      (uint64_t)c->ncu *
-                                          std::min(xdrop_coop_occupancy(),
-                                                   kMaxWgPerCu / 4)));
-            HIPCHK(c, launch_xdrop_coop(P<XdTask>(c->xdt), nullptr,
-                                        ctr + C_XDN, ctr + C_XDQ,
-                                        P<int8_t>(c->dmat), c->cfg.xdrop_gap,
-                                        c->cfg.xdrop, c->cfg.seed_len,
-                                        P<XdOut>(c->xdo), lng, ctr + C_XDLONG,
-                                        cg, s));
+            if ((rc = coop(nullptr, ctr + C_XDN, ctr + C_XDQ, ni, lng,
+                           ctr + C_XDLONG, s)))
+                return rc;
             HIPCHK(c, launch_xdrop(P<XdTask>(c->xdt), lng, ctr + C_XDLONG,
                                    ctr + C_XDLONGQ, P<int8_t>(c->dmat),
                                    c->cfg.xdrop_gap, c->cfg.xdrop,
                                    c->cfg.seed_len, nullptr, 0,
                                    P<XdOut>(c->xdo), ovf, ctr + C_XDOVF, grid,
                                    c->tune.xd_ring, s));
-            c->stats.launches += 2;
+            c->stats.launches++;
         } else {
-            HIPCHK(c, launch_xdrop(P<XdTask>(c->xdt), nullptr, ctr + C_XDN,
-                                   ctr + C_XDQ, P<int8_t>(c->dmat),
-                                   c->cfg.xdrop_gap, c->cfg.xdrop,
-                                   c->cfg.seed_len, nullptr, 0,
+            // both kernels append to the same overflow list
+            if (two) {
+                HIPCHK(c, hipEventRecord(c->ev_fork[0], s));
+                HIPCHK(c, hipStreamWaitEvent(c->st2, c->ev_fork[0], 0));
+                if ((rc = coop(lng, ctr + C_XDLONG, ctr + C_XDLONGQ, ni, ovf,
+                               ctr + C_XDOVF, c->st2)))
+                    return rc;
+            }
+            HIPCHK(c, launch_xdrop(P<XdTask>(c->xdt), two ? order : nullptr,
+                                   ctr + C_XDN, ctr + C_XDQ,
+                                   P<int8_t>(c->dmat), c->cfg.xdrop_gap,
+                                   c->cfg.xdrop, c->cfg.seed_len, nullptr, 0,
                                    P<XdOut>(c->xdo), ovf, ctr + C_XDOVF, grid,
                                    c->tune.xd_ring, s));
             c->stats.launches++;
+            if (two) {
+                HIPCHK(c, hipEventRecord(c->ev_join, c->st2));
+                HIPCHK(c, hipStreamWaitEvent(s, c->ev_join, 0));
+            }
         }
     }
     // items whose band outgrew the LDS rings: 16 lanes per item with a

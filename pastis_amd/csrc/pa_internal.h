@@ -369,6 +369,18 @@ static_assert(sizeof(XdTask) == 40, "XdTask layout");
 // The pair names a sequence that is not loaded or its seed does not fit.
 constexpr uint32_t kXdInvalid = 1u;
 
+// Residues an item (direction dir of a task: 0 left, 1 right) can extend over
+// at most, the shorter of its two segments; 0 for an invalid task.
+__host__ __device__ inline uint32_t xd_reach(const XdTask &t, int dir,
+                                             int seed_len)
+{
+    if (t.pad & kXdInvalid)
+        return 0;
+    const uint32_t h = dir ? t.nh - t.beg_h - (uint32_t)seed_len : t.beg_h;
+    const uint32_t v = dir ? t.nv - t.beg_v - (uint32_t)seed_len : t.beg_v;
+    return h < v ? h : v;
+}
+
 // Seed extension result; the left direction writes beg_*, score_left,
 // cells_left, flags_left and the right direction the other half.
 struct XdOut {
