@@ -31,7 +31,9 @@ struct SeqSketch {
 };
 static_assert(sizeof(SeqSketch) == 112, "SeqSketch layout");
 
+// Sketches of nseq sequences; with pre, also the residue bound's sums.
 hipError_t seq_sketch(const uint64_t *offs, uint64_t nseq, SeqSketch *out,
+                      uint32_t *pre, uint64_t base, const uint32_t *best,
                       hipStream_t s);
 hipError_t features(const pa_pair *pairs, uint64_t n, const SeqSketch *rs,
                     uint32_t nr, const SeqSketch *cs, uint32_t nc, float *out,

@@ -56,38 +56,81 @@ __device__ inline float bf16r(float x)
     return __uint_as_float(u);
 }
 
-__global__ void k_seq_sketch(const uint64_t *__restrict__ offs, uint64_t nseq,
-                             SeqSketch *__restrict__ out)
+// A wave per sequence, a lane per residue position: each lane hashes the
+// k-mer that ends at its position, the classes are counted by ballots, and the
+// minima are reduced at the end.  One thread per sequence walked its residues
+// one after the other (20,000 sequences of 335: 1.5 ms, now 0.08; with a
+// sequence of 35,000: 26 ms).
+//
+// pre (optional): inclusive sums of `best` over each sequence's residues, at
+// the residues' offsets from base (ResBound).
+constexpr int kSketchWaves = 4;   // sequences per workgroup
+
+__global__ __launch_bounds__(64 * kSketchWaves) void k_seq_sketch(
+    const uint64_t *__restrict__ offs, uint64_t nseq,
+    SeqSketch *__restrict__ out, uint32_t *__restrict__ pre, uint64_t base,
+    const uint32_t *__restrict__ best)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nseq)
+    const int lane = threadIdx.x & 63;
+    const uint64_t i =
+        (uint64_t)blockIdx.x * kSketchWaves + (threadIdx.x >> 6);
+    if (i >= nseq)   // a whole wave
         return;
     const uint8_t *s = (const uint8_t *)(uintptr_t)offs[i];
     const int L = (int)(offs[i + 1] - offs[i]);
-    uint32_t cnt[10] = {0};
-    uint32_t mh[kSketch];
+    uint32_t cnt[10] = {0}, mh[kSketch];
+#pragma unroll
     for (int h = 0; h < kSketch; ++h)
         mh[h] = 0xffffffffu;
-    uint32_t code = 0, tot = 0;
-    const uint32_t p5 = 15u * 15u * 15u * 15u * 15u;
-    for (int j = 0; j < L; ++j) {
-        const uint32_t m = kMurphy[s[j]];
-        if (m < 10) {
-            cnt[m]++;
-            tot++;
-        }
-        code = (code % p5) * 15u + m;
-        if (j >= kK - 1) {
+    uint32_t sum = 0;
+    for (int j0 = 0; j0 < L; j0 += 64) {
+        const int j = j0 + lane;
+        const bool in = j < L;
+        const uint32_t m = in ? kMurphy[s[j]] : 15u;
+#pragma unroll
+        for (int k = 0; k < 10; ++k)
+            cnt[k] += (uint32_t)__popcll(__ballot(m == (uint32_t)k));
+        if (in && j >= kK - 1) {
+            uint32_t code = 0;   // base-15 number of the last kK classes
+#pragma unroll
+            for (int k = kK - 1; k >= 0; --k)
+                code = code * 15u + kMurphy[s[j - k]];
+#pragma unroll
             for (int h = 0; h < kSketch; ++h) {
-                const uint32_t v = mix32(code ^ (0x9e3779b9u * (uint32_t)(h + 1)));
+                const uint32_t v =
+                    mix32(code ^ (0x9e3779b9u * (uint32_t)(h + 1)));
                 mh[h] = v < mh[h] ? v : mh[h];
             }
         }
+        if (pre) {
+            uint32_t run = in ? best[s[j]] : 0u;
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t x = __shfl(run, lane - off);
+                run += lane >= off ? x : 0u;
+            }
+            if (in)
+                pre[offs[i] - base + (uint64_t)j] = sum + run;
+            sum += __shfl(run, 63);
+        }
     }
+#pragma unroll
+    for (int h = 0; h < kSketch; ++h)
+        for (int off = 32; off >= 1; off >>= 1) {
+            const uint32_t v = __shfl_xor(mh[h], off);
+            mh[h] = v < mh[h] ? v : mh[h];
+        }
+    if (lane != 0)
+        return;
+    uint32_t tot = 0;
+#pragma unroll
+    for (int k = 0; k < 10; ++k)
+        tot += cnt[k];
     SeqSketch o;
     const float ft = (float)(tot ? tot : 1u);
+#pragma unroll
     for (int k = 0; k < 10; ++k)
         o.comp[k] = __fdiv_rn((float)cnt[k], ft);
+#pragma unroll
     for (int h = 0; h < kSketch; ++h)
         o.mh[h] = mh[h];
     o.len = (uint32_t)L;
@@ -489,12 +532,14 @@ inline unsigned nblk(uint64_t n, unsigned b) { return (unsigned)((n + b - 1) / b
 }  // namespace
 
 hipError_t seq_sketch(const uint64_t *offs, uint64_t nseq, SeqSketch *out,
+                      uint32_t *pre, uint64_t base, const uint32_t *best,
                       hipStream_t s)
 {
     if (!nseq)
         return hipSuccess;
-    hipLaunchKernelGGL(k_seq_sketch, dim3(nblk(nseq, 128)), dim3(128), 0, s,
-                       offs, nseq, out);
+    hipLaunchKernelGGL(k_seq_sketch, dim3(nblk(nseq, kSketchWaves)),
+                       dim3(64 * kSketchWaves), 0, s, offs, nseq, out, pre,
+                       base, best);
     return hipGetLastError();
 }
 

@@ -20,6 +20,10 @@ hipError_t fill_u32(uint32_t *p, uint32_t v, uint32_t n, hipStream_t s);
 // *dst += *src (one thread; a device-side counter)
 hipError_t accumulate(const uint32_t *src, unsigned long long *dst,
                       hipStream_t s);
+// Codes (at codes + kSeqPad, sentinels around them) and k-mer letters (in
+// place) of the total bytes at raw; both buffers hold 64 bytes more.
+hipError_t encode_set(uint8_t *raw, uint8_t *codes, uint64_t total,
+                      const uint8_t *tab, hipStream_t s);
 // Pairs naming sequences outside the nr row / nc column sequences become
 // empty tasks (and X-drop tasks whose seed does not fit are flagged
 // kXdInvalid), so no kernel reads outside the sequence store.

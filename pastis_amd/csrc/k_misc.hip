@@ -45,6 +45,40 @@ __global__ void k_fill_u32(uint32_t *p, uint32_t v, uint32_t n)
         p[i] = v;
 }
 
+// Residue codes and k-mer letters of a sequence set's bytes, four at a time.
+// raw (the bytes, total of them) is overwritten by the letters; codes starts
+// kSeqPad bytes before the first residue.  Outside the set: sentinels, and no
+// k-mer letter.
+__global__ __launch_bounds__(256) void k_encode(uint32_t *__restrict__ raw,
+                                                uint32_t *__restrict__ codes,
+                                                uint64_t total,
+                                                const uint8_t *__restrict__ tab)
+{
+    __shared__ uint8_t t[512];   // code, then letter, of each byte
+    t[threadIdx.x] = tab[threadIdx.x];
+    t[threadIdx.x + 256] = tab[threadIdx.x + 256];
+    __syncthreads();
+    constexpr uint64_t pad = kSeqPad / 4;
+    const uint64_t words = (total + 64) / 4;   // of raw
+    for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+         w < words + pad; w += (uint64_t)gridDim.x * blockDim.x) {
+        if (w >= words) {   // the pad before the first residue
+            codes[w - words] = 0x01010101u * kSentinel;
+            continue;
+        }
+        const uint32_t x = raw[w];
+        uint32_t cw = 0, kw = 0;
+        for (int q = 0; q < 4; ++q) {
+            const bool in = 4 * w + q < total;
+            const uint32_t b = (x >> (8 * q)) & 0xffu;
+            cw |= (in ? (uint32_t)t[b] : (uint32_t)kSentinel) << (8 * q);
+            kw |= (in ? (uint32_t)t[256 + b] : 255u) << (8 * q);
+        }
+        codes[pad + w] = cw;
+        raw[w] = kw;
+    }
+}
+
 // Pair -> local-alignment task: rows = row sequence (SeqAn V), columns =
 // column sequence (SeqAn H), as localAlignment(seqsc, seqsr) at
 // SeqanFullAligner.cpp:231.
@@ -202,11 +236,13 @@ __global__ void k_build_nw_tasks(const XdTask *__restrict__ xt, uint64_t nt,
         t.tlen = (uint32_t)(o.end_h - o.beg_h);
         t.id = x.id;
         t.flags = 0;
-        if (t.qlen && t.tlen) {
+        if (t.qlen && t.tlen && rows.pre) {
             // residue bound of the two spans (traced int16 holds 4*score+3)
             const uint64_t iq = t.q_off - rows.base, it = t.t_off - cols.base;
-            const uint32_t uq = rows.pre[iq + t.qlen] - rows.pre[iq];
-            const uint32_t ut = cols.pre[it + t.tlen] - cols.pre[it];
+            const uint32_t uq = rows.pre[iq + t.qlen - 1] -
+                                (o.beg_v > 0 ? rows.pre[iq - 1] : 0u);
+            const uint32_t ut = cols.pre[it + t.tlen - 1] -
+                                (o.beg_h > 0 ? cols.pre[it - 1] : 0u);
             const uint32_t ub = uq < ut ? uq : ut;
             if (4ull * ub + 3ull < 32760ull)
                 t.flags |= kTaskBounded;
@@ -595,6 +631,15 @@ hipError_t accumulate(const uint32_t *src, unsigned long long *dst,
                       hipStream_t s)
 {
     hipLaunchKernelGGL(k_accumulate, dim3(1), dim3(64), 0, s, src, dst);
+    return hipGetLastError();
+}
+
+hipError_t encode_set(uint8_t *raw, uint8_t *codes, uint64_t total,
+                      const uint8_t *tab, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_encode, dim3(stride_blocks(total / 4 + 64)),
+                       dim3(256), 0, s, (uint32_t *)raw, (uint32_t *)codes,
+                       total, tab);
     return hipGetLastError();
 }
 

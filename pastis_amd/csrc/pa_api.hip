@@ -956,10 +956,13 @@ int align_xd_dev(pa_ctx *c, const pa_pair *d_pairs, uint64_t n,
     Scope tot(c, 4, s);
     if ((rc = run_xdrop(c, d_pairs, n, s)))
         return rc;
-    const ResBound rb{(uint64_t)(uintptr_t)seq_base(c->rcodes),
-                      (const uint32_t *)((char *)c->rcodes.p + c->rpre_off)};
-    const ResBound cbd{(uint64_t)(uintptr_t)seq_base(c->ccodes),
-                       (const uint32_t *)((char *)c->ccodes.p + c->cpre_off)};
+    auto bound = [](const Buf &codes, size_t off) {
+        return ResBound{(uint64_t)(uintptr_t)seq_base(codes),
+                        off ? (const uint32_t *)((char *)codes.p + off)
+                            : nullptr};
+    };
+    const ResBound rb = bound(c->rcodes, c->rpre_off),
+                   cbd = bound(c->ccodes, c->cpre_off);
     HIPCHK(c, build_nw_tasks(P<XdTask>(c->xdt), nt, P<XdOut>(c->xdo),
                              P<DpTask>(c->tasks), rb, cbd,
                              (unsigned long long *)P<uint64_t>(c->cells),
@@ -1005,75 +1008,52 @@ int upload_set(pa_ctx *c, bool rows, const uint8_t *res, const uint64_t *offs,
         lens[i] = (uint32_t)L;
         mx = std::max(mx, (uint32_t)L);
     }
-    std::vector<uint8_t> codes(kSeqPad + total + 64, (uint8_t)kSentinel);
-    // k-mer letters: a residue upper-cased with & 0xDF must be one of the 25
-    // letters (add_kmers, src/kmer/KmerOps.cpp:61-73); '*' never is, since
-    // '*' & 0xDF is not a letter
-    std::vector<uint8_t> kc(total + 64, 255);
-    for (uint64_t i = 0; i < total; ++i) {
-        uint8_t x = res[base + i];
-        uint8_t k = 255;
-        if (enc == PA_ENC_ASCII) {
-            const uint8_t up = (uint8_t)(x & 0xDF);
-            k = up < 128 ? encode_ascii(up) : 22;
-            if (k == 22 && up != 'X')
-                k = 255;
-            if (k == 23)
-                k = 255;
-            x = encode_ascii(x);
-        } else if (x >= 25) {
-            return fail(c, PA_ERR_RESIDUE,
-                        "residue code " + std::to_string(x) + " at offset " +
-                            std::to_string(base + i));
-        } else {
-            k = x == 23 ? 255 : x;
-        }
-        codes[kSeqPad + i] = x;
-        kc[i] = k;
+    const uint8_t *raw = res + base;
+    if (enc == PA_ENC_CODES) {
+        bool bad = false;
+        for (uint64_t i = 0; i < total; ++i)   // (vectorised: no early exit)
+            bad |= raw[i] >= 25;
+        for (uint64_t i = 0; bad && i < total; ++i)
+            if (raw[i] >= 25)
+                return fail(c, PA_ERR_RESIDUE,
+                            "residue code " + std::to_string(raw[i]) +
+                                " at offset " + std::to_string(base + i));
     }
-    // Residue-bound prefix sums (ResBound) after the codes: the best score of
-    // each code against any code, in either operand position, at least 0.
-    uint32_t best[32] = {};
-    for (int x = 0; x < kAlpha; ++x) {
-        int m = 0;
-        for (int y = 0; y < kAlpha; ++y)
-            m = std::max(m, (int)std::max(c->mat[x * 32 + y], c->mat[y * 32 + x]));
-        best[x] = (uint32_t)m;
-    }
-    const size_t pre_off = (codes.size() + 3) & ~(size_t)3;
-    std::vector<uint32_t> pre(total + 1);
-    uint32_t acc = 0;   // wraps around; span differences stay exact
-    for (uint64_t i = 0; i < total; ++i) {
-        pre[i] = acc;
-        acc += best[codes[kSeqPad + i]];
-    }
-    pre[total] = acc;
+    // the bytes go up as they are and are encoded there (k_encode); the
+    // residue bound, which only the affine global kernels ask for, follows
+    // the codes
     Buf &cb = rows ? c->rcodes : c->ccodes;
     Buf &ob = rows ? c->roffs : c->coffs;
     Buf &kb = rows ? c->rkc : c->ckc;
-    if ((rc = grow(c, cb, pre_off + pre.size() * sizeof(uint32_t))) ||
-        (rc = grow(c, kb, kc.size())))
+    const bool bound = c->cfg.mode == PA_MODE_XDROP && !c->lin_global;
+    const size_t pre_off = (kSeqPad + total + 64 + 3) & ~(size_t)3;
+    if ((rc = grow(c, cb, pre_off + (bound ? total * sizeof(uint32_t) : 0))) ||
+        (rc = grow(c, kb, total + 64)))
         return rc;
-    HIPCHK(c, hipMemcpyAsync(kb.p, kc.data(), kc.size(), hipMemcpyHostToDevice,
-                             c->st));
-    (rows ? c->rpre_off : c->cpre_off) = pre_off;
+    (rows ? c->rpre_off : c->cpre_off) = bound ? pre_off : 0;
     if ((rc = grow(c, ob, (nseq + 1) * sizeof(uint64_t))))
         return rc;
     std::vector<uint64_t> abs(nseq + 1);
     const uint64_t dev = (uint64_t)(uintptr_t)seq_base(cb);
     for (uint64_t i = 0; i <= nseq; ++i)
         abs[i] = dev + (offs[i] - base);
-    HIPCHK(c, hipMemcpyAsync(cb.p, codes.data(), codes.size(),
-                             hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipMemcpyAsync((char *)cb.p + pre_off, pre.data(),
-                             pre.size() * sizeof(uint32_t),
-                             hipMemcpyHostToDevice, c->st));
+    if (total)
+        HIPCHK(c, hipMemcpyAsync(kb.p, raw, total, hipMemcpyHostToDevice,
+                                 c->st));
     HIPCHK(c, hipMemcpyAsync(ob.p, abs.data(), abs.size() * 8,
                              hipMemcpyHostToDevice, c->st));
+    HIPCHK(c, encode_set(P<uint8_t>(kb), P<uint8_t>(cb), total,
+                         P<uint8_t>(c->dmat) + kTabEnc +
+                             (enc == PA_ENC_ASCII ? 0 : 512),
+                         c->st));
     Buf &sb = rows ? c->rsk : c->csk;
     if ((rc = grow(c, sb, std::max<uint64_t>(nseq, 1) * sizeof(SeqSketch))))
         return rc;
-    HIPCHK(c, seq_sketch(P<uint64_t>(ob), nseq, P<SeqSketch>(sb), c->st));
+    HIPCHK(c, seq_sketch(P<uint64_t>(ob), nseq, P<SeqSketch>(sb),
+                         bound ? (uint32_t *)((char *)cb.p + pre_off) : nullptr,
+                         dev,
+                         (const uint32_t *)(P<int8_t>(c->dmat) + kTabBest),
+                         c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
     if (rows) {
         c->rlen.swap(lens);
@@ -1239,6 +1219,29 @@ int pa_create(const pa_config *cfg, pa_ctx **out)
         dm[kPmatRot + 1024 + k] = (int8_t)(((n & 3) << 6) | (n >> 2));
         dm[kPmatPair + k] = (int8_t)n;
         dm[kPmatPair + 1024 + k] = (int8_t)(n << 4);
+    }
+    // Residue bound: the best score of each code against any code, in either
+    // operand position, at least 0.  Letters: a k-mer letter is a residue
+    // upper-cased with & 0xDF that is one of the 25 letters (add_kmers,
+    // src/kmer/KmerOps.cpp:61-73); '*' never is, since '*' & 0xDF is not a
+    // letter.
+    for (int x = 0; x < 32; ++x) {
+        int m = 0;
+        for (int y = 0; x < kAlpha && y < kAlpha; ++y)
+            m = std::max(m, (int)std::max(c->mat[x * 32 + y],
+                                          c->mat[y * 32 + x]));
+        const uint32_t u = (uint32_t)m;
+        std::memcpy(&dm[kTabBest + 4 * x], &u, 4);
+    }
+    for (int x = 0; x < 256; ++x) {
+        const uint8_t up = (uint8_t)(x & 0xDF);
+        int k = up < 128 ? encode_ascii(up) : 22;
+        if ((k == 22 && up != 'X') || k == 23)
+            k = 255;
+        dm[kTabEnc + x] = (int8_t)encode_ascii((uint8_t)x);
+        dm[kTabEnc + 256 + x] = (int8_t)k;
+        dm[kTabEnc + 512 + x] = (int8_t)x;
+        dm[kTabEnc + 768 + x] = (int8_t)(x == 23 ? 255 : x);
     }
     c->shapes = shapes_for(c, c->tune);
     if (grow(c, c->dmat, kPmatBytes) ||

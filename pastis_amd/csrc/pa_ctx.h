@@ -163,9 +163,6 @@ inline DpShapes shapes_for(const pa_ctx *c, const pa_tuning &t)
     return sh;
 }
 
-// Sentinels ahead of the first sequence of a store (a kernel's window of
-// residues may start up to 7 bytes before a sequence).
-constexpr size_t kSeqPad = 64;
 // device address of a store's first residue
 inline uint8_t *seq_base(const Buf &codes)
 {

@@ -41,6 +41,9 @@ template <class T> __device__ inline T PA_GLOBAL *glb_addr(uint64_t a)
 constexpr int kAlpha = 25;
 constexpr int kSentinel = 25;
 constexpr int kProfChars = 26;
+// Sentinels ahead of the first sequence of a store (a kernel's window of
+// residues may start up to 7 bytes before a sequence).
+constexpr size_t kSeqPad = 64;
 
 // One DP task: the row (V, lanes) and column (H, streamed) sequence spans.
 struct DpTask {
@@ -86,18 +89,23 @@ constexpr size_t kPmatUntraced = 1024, kPmatLocal = 2048, kPmatGlobal = 3072,
 // the two rows of a profile byte.  Traced: the same nibble n as n << 2, and n
 // rotated to bits 6, 7, 0, 1; score only: n and n << 4.
 constexpr int kPmatRot = 5120, kPmatPair = 7168;
-constexpr size_t kPmatBytes = 9216;
+// After them: the best score of each code (32 uint32, ResBound), then for
+// ASCII and for code input the residue code and the k-mer letter of each byte
+// (k_encode).
+constexpr int kTabBest = 9216, kTabEnc = kTabBest + 128;
+constexpr size_t kPmatBytes = kTabEnc + 4 * 256;
 // Global task whose scores are bounded by the residue bound below (no cell
 // exceeds min over the two spans of the sum of each residue's best score),
 // small enough for the traced int16 kernels.
 constexpr uint32_t kTaskBounded = 2u;
 
-// Residue bound of a sequence store: pre[k] = sum over codes[0..k) of
-// max(0, best score of that code against any code), as uint32 with
-// wrap-around (differences over one sequence's span stay exact).
+// Residue bound of a sequence store: pre[k] = sum over the residues of the
+// sequence that holds residue k, up to and with k, of max(0, best score of
+// that code against any code).  Only the affine kernels ask for it (null
+// otherwise).
 struct ResBound {
     uint64_t base;          // device address of the store's first residue
-    const uint32_t *pre;    // prefix sums, one more entry than residues
+    const uint32_t *pre;
 };
 
 // Arguments of the wavefront DP kernels.

@@ -82,7 +82,26 @@ struct FastaParser {
         bool in_name = false, in_seq = false;
         int64_t seq_len = 0;
         S.reserve(n);
+        // bytes of a sequence that need a look: the others are copied in runs
+        bool look[256] = {};
+        for (const char ch : {'>', '\n', '*', 'U', 'u'})
+            look[(uint8_t)ch] = true;
         for (uint64_t i = 0; i < n; ++i) {
+            if (in_name || in_seq) {
+                uint64_t e = i;
+                if (in_name) {   // a header: everything up to its newline
+                    const void *nl = std::memchr(b + i, '\n', n - i);
+                    e = nl ? (uint64_t)((const char *)nl - b) : n;
+                } else {
+                    while (e < n && !look[(uint8_t)b[e]])
+                        ++e;
+                    seq_len += (int64_t)(e - i);
+                }
+                S.insert(S.end(), b + i, b + e);
+                if (e == n)
+                    break;
+                i = e;
+            }
             char ch = b[i];
             const bool last = i + 1 >= n;
             if (ch == '>' && !in_name) {
