@@ -43,14 +43,20 @@ namespace pa {
 // (Alphabet::init, src/Alphabet.cpp:31-51).
 struct KmerAlphabet {
     uint8_t code[kAlpha];    // alphabet code of each residue code
-    int16_t self[kAlpha];    // BLOSUM62 self score of the representative
+    int16_t self[kAlpha];    // BLOSUM62 self score of each code's representative
     int size;
 };
 
+struct KmerGroups {         // occurrences [start, end) of each code
+    Buf start, end, code, cost;
+    uint64_t n = 0;
+    bool built = false;
+};
+
 struct KmerSet {            // sorted occurrences of one sequence set
-    Buf keys, vals, gstart, gcode;
+    Buf keys, vals;
     uint64_t nocc = 0;      // valid occurrences
-    uint64_t ngroups = 0;   // distinct codes
+    KmerGroups groups[2];   // all codes; those of more than one occurrence
     uint64_t gen = ~0ull;   // sequence generation they were built for
     int k = 0, stride = 0, alph = -1;
 };
@@ -64,20 +70,27 @@ struct KmerState {
     pa_kmer_config last{};
     uint64_t last_cb = 0, last_ce = 0, last_gen = ~0ull, last_n = 0;
     bool have_last = false;
+    uint64_t *host = nullptr;   // pinned words for values read back
 };
 
 void kmer_free(KmerState *k)
 {
     if (!k)
         return;
-    for (KmerSet *s : {&k->rows, &k->cols})
-        for (Buf *b : {&s->keys, &s->vals, &s->gstart, &s->gcode})
-            release(*b);
+    for (KmerSet *s : {&k->rows, &k->cols}) {
+        release(s->keys);
+        release(s->vals);
+        for (KmerGroups &g : s->groups)
+            for (Buf *b : {&g.start, &g.end, &g.code, &g.cost})
+                release(*b);
+    }
     for (Buf *b : {&k->slots, &k->keys_a, &k->vals_a, &k->pcount, &k->poff,
                    &k->gscr, &k->pkey, &k->pval, &k->pkey2, &k->pval2, &k->heads,
                    &k->runid, &k->rstart, &k->keep, &k->kpos, &k->tmp,
                    &k->cnt, &k->cand})
         release(*b);
+    if (k->host)
+        hipHostFree(k->host);
     delete k;
 }
 
@@ -116,7 +129,7 @@ bool make_alphabet(int id, KmerAlphabet &a)
         if (code_of_rep[rep[i]] < 0)
             code_of_rep[rep[i]] = next++;
         a.code[i] = (uint8_t)code_of_rep[rep[i]];
-        a.self[i] = kSelfB62[rep[i]];
+        a.self[a.code[i]] = kSelfB62[rep[i]];
     }
     a.size = next;
     return true;
@@ -183,29 +196,57 @@ __global__ void k_kmer_extract(const uint8_t *__restrict__ kc,
         atomicAdd(nbad, (unsigned long long)bad);
 }
 
-// heads[i] = 1 where a new code group starts (i < n)
+// heads[i] = 1 where a new code group (multi: of more than one occurrence)
+// starts (i < n)
 __global__ void k_group_heads(const uint32_t *__restrict__ keys, uint64_t n,
-                              uint32_t *__restrict__ heads)
+                              bool multi, uint32_t *__restrict__ heads)
 {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (uint64_t)gridDim.x * blockDim.x)
-        heads[i] = (i == 0 || keys[i] != keys[i - 1]) ? 1u : 0u;
+        heads[i] = (i == 0 || keys[i] != keys[i - 1]) &&
+                           (!multi || (i + 1 < n && keys[i + 1] == keys[i]))
+                       ? 1u
+                       : 0u;
 }
 
-// group g (inclusive scan value - 1 at a head) -> start, code
+// self score of a k-mer code (sum over its letters' representatives)
+__device__ inline int code_cost(uint32_t code, const KmerAlphabet &al, int k)
+{
+    int cost = 0;
+    for (int j = 0; j < k; ++j) {
+        cost += al.self[code % (uint32_t)al.size];
+        code /= (uint32_t)al.size;
+    }
+    return cost;
+}
+
+// group g (inclusive scan value - 1 from its head on) -> start, end, code,
+// self score
 __global__ void k_group_table(const uint32_t *__restrict__ keys,
                               const uint32_t *__restrict__ heads,
                               const uint64_t *__restrict__ incl, uint64_t n,
+                              bool multi, KmerAlphabet alph, int k,
                               uint64_t *__restrict__ gstart,
-                              uint32_t *__restrict__ gcode)
+                              uint64_t *__restrict__ gend,
+                              uint32_t *__restrict__ gcode,
+                              int16_t *__restrict__ gcost)
 {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        if (heads[i]) {
-            const uint64_t g = incl[i] - 1;
+         i += (uint64_t)gridDim.x * blockDim.x) {
+        const uint32_t key = keys[i];
+        const bool first = i == 0 || keys[i - 1] != key;
+        const bool last = i + 1 == n || keys[i + 1] != key;
+        if (multi && first && last)
+            continue;
+        const uint64_t g = incl[i] - 1;
+        if (first) {
             gstart[g] = i;
-            gcode[g] = keys[i];
+            gcode[g] = key;
+            gcost[g] = (int16_t)code_cost(key, alph, k);
         }
+        if (last)
+            gend[g] = i + 1;
+    }
 }
 
 __device__ inline uint64_t lower_bound_u32(const uint32_t *a, uint64_t n,
@@ -226,147 +267,352 @@ __device__ inline uint64_t lower_bound_u32(const uint32_t *a, uint64_t n,
 __device__ inline uint64_t lower_bound_seq(const uint64_t *vals, uint64_t lo,
                                            uint64_t hi, uint64_t s)
 {
-    while (lo < hi) {
+    while (hi - lo > 4) {
         const uint64_t mid = (lo + hi) / 2;
         if ((vals[mid] >> 16) < s)
             lo = mid + 1;
         else
             hi = mid;
     }
-    return lo;
+    if (lo == hi)
+        return lo;
+    // the last four (most groups hold no more) in loads that do not wait for
+    // one another
+    uint64_t v[4];
+    for (int i = 0; i < 4; ++i)
+        v[i] = vals[lo + i < hi ? lo + i : hi - 1] >> 16;
+    uint64_t n = 0;
+    for (int i = 0; i < 4; ++i)
+        n += lo + i < hi && v[i] < s ? 1 : 0;
+    return lo + n;
 }
 
-// Per column group g: the column occurrences in [c_begin, c_end) and the
-// row group with the same code; products = both counts multiplied.
-struct JoinArgs {
-    const uint64_t *cgstart;   // column groups (and their end at ngroups)
-    const uint32_t *cgcode;
-    const uint64_t *cvals;
-    uint64_t cngroups, cnocc;
-    const uint32_t *rkeys;     // row occurrences (sorted keys)
-    uint64_t rnocc;
-    const uint64_t *rgstart;   // row groups when the sets are shared
-    bool shared;
-    uint64_t c_begin, c_end;
-    // per group: [ca, cb) columns, [ra, rb) rows
-    uint64_t *ca, *ra;
-    uint32_t *cn, *rn;
-    uint64_t *pcount;
+// Groups by the number of their products: one thread emits the products of a
+// small group, a block those of a large one, all blocks together those of a
+// huge one.
+constexpr uint64_t kSmallGroup = 64, kLargeGroup = 1u << 16;
+// Under PA_SYM_UPPER a group of few column occurrences counts only the
+// products that are kept: for a column sequence the row occurrences of lower
+// (global) sequences, a prefix of the row group.  Most groups hold a single
+// occurrence, whose only product is with itself: 60,000 sequences give 35
+// million products of which 7.9 million are kept, and all of them were sorted.  Larger groups count all products and drop some.
+constexpr uint32_t kTriCols = 32;
+
+// symmetric pruning of the product of (global) row R and column C
+__device__ inline bool keep_product(int sym, uint64_t R, uint64_t C)
+{
+    if (sym == PA_SYM_UPPER)
+        return C > R;
+    const bool ro = R & 1, co = C & 1;
+    return sym != PA_SYM_EVEN_ODD ||
+           !(R == C || (R > C ? (ro ^ co) : !(ro ^ co)));
+}
+
+// A short group of a set that is both rows and columns under one base: its
+// occurrences are read at once, and only the products that are kept count.  All
+// but one in forty groups of more than one occurrence are short (60,000
+// sequences); the searches of the general path are chains of dependent loads.
+// 32-bit compares, since these kernels are bound by their instructions: joining
+// and emitting 3.7 million groups took 112 and 219 us with 64-bit ones (and a
+// division per letter of the code) and every wave waiting for its groups that
+// are not short; now 88 and 136 us.
+constexpr uint32_t kShort = 4;
+
+struct ShortGroup {
+    uint64_t v[kShort];
+    uint32_t seq[kShort];
+    bool col[kShort], row[kShort];
+    int sym;
+
+    template <class A>
+    __device__ ShortGroup(const A &a, uint64_t gs, uint64_t ge) : sym(a.sym)
+    {
+        const uint32_t n = (uint32_t)(ge - gs);
+        for (uint32_t i = 0; i < kShort; ++i)
+            v[i] = a.cvals[i < n ? gs + i : gs];
+        for (uint32_t i = 0; i < kShort; ++i) {
+            seq[i] = (uint32_t)(v[i] >> 16);
+            row[i] = i < n;
+            col[i] = i < n && seq[i] >= a.c_begin && seq[i] < a.c_end;
+        }
+    }
+
+    // column occurrence x and row occurrence y make a product
+    __device__ bool product(uint32_t x, uint32_t y) const
+    {
+        const uint32_t c = seq[x], r = seq[y];
+        const bool odd = (r ^ c) & 1;
+        const bool keep = sym == PA_SYM_UPPER ? c > r
+                          : sym == PA_SYM_NONE
+                              ? true
+                              : r != c && !(r > c ? odd : !odd);
+        return col[x] && row[y] && keep;
+    }
 };
 
-__global__ void k_join_count(JoinArgs a)
+struct JoinGroup {
+    uint64_t ca, ra;           // first column / row occurrence
+    uint32_t cn, rn;           // and their numbers
+};
+
+// Per column group g: the column occurrences in [c_begin, c_end) and the
+// row group with the same code; products = both counts multiplied, or the
+// kept ones (kTriCols).
+struct JoinArgs {
+    const uint64_t *cgstart, *cgend;   // column groups
+    const uint32_t *cgcode;
+    const uint64_t *cvals;
+    uint64_t cngroups;
+    const uint32_t *rkeys;     // row occurrences (sorted keys)
+    uint64_t rnocc;
+    bool shared;               // rows and columns are one set
+    bool one_set;              // and of one base
+    uint64_t c_begin, c_end;
+    JoinGroup *grp;            // written where emit_group reads it
+    uint64_t *pcount;
+    const uint64_t *rvals;
+    int sym;                   // pa_symmetric
+    uint64_t up_off;           // row sequences kept: below c + up_off
+    uint32_t *large, *huge;    // group lists and their lengths
+    uint32_t *nlarge, *nhuge;
+};
+
+// Row occurrences of rvals[ra, ra + rn) whose sequence lies below the column
+// sequence c in global indices (up_off = col_base - row_base, wrapping).
+__device__ inline uint64_t rows_below(const uint64_t *rvals, uint64_t ra,
+                                      uint64_t rn, uint64_t c, uint64_t up_off)
 {
-    for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-         g < a.cngroups; g += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t gs = a.cgstart[g];
-        const uint64_t ge = g + 1 < a.cngroups ? a.cgstart[g + 1] : a.cnocc;
-        const uint64_t c0 = lower_bound_seq(a.cvals, gs, ge, a.c_begin);
-        const uint64_t c1 = lower_bound_seq(a.cvals, c0, ge, a.c_end);
-        uint64_t r0, r1;
-        if (a.shared) {
-            r0 = gs;
-            r1 = ge;
-        } else {
-            const uint32_t code = a.cgcode[g];
-            r0 = lower_bound_u32(a.rkeys, a.rnocc, code);
-            r1 = lower_bound_u32(a.rkeys, a.rnocc, code + 1);
+    const int64_t lim = (int64_t)(c + up_off);
+    if (lim <= 0)
+        return 0;
+    if (rn == 1)
+        return (rvals[ra] >> 16) < (uint64_t)lim ? 1 : 0;
+    return lower_bound_seq(rvals, ra, ra + rn, (uint64_t)lim) - ra;
+}
+
+// products of group g = occurrences [gs, ge) of the column set
+__device__ inline uint64_t join_group(const JoinArgs &a, uint64_t g,
+                                      uint64_t gs, uint64_t ge)
+{
+    const uint64_t c0 = lower_bound_seq(a.cvals, gs, ge, a.c_begin);
+    const uint64_t c1 = lower_bound_seq(a.cvals, c0, ge, a.c_end);
+    uint64_t r0 = gs, r1 = ge;
+    if (!a.shared) {
+        const uint32_t code = a.cgcode[g];
+        r0 = lower_bound_u32(a.rkeys, a.rnocc, code);
+        r1 = lower_bound_u32(a.rkeys, a.rnocc, code + 1);
+    }
+    uint64_t np = (c1 - c0) * (r1 - r0);
+    if (np && a.sym == PA_SYM_UPPER && c1 - c0 <= kTriCols) {
+        np = 0;
+        for (uint64_t x = c0; x < c1; ++x)
+            np += rows_below(a.rvals, r0, r1 - r0, a.cvals[x] >> 16, a.up_off);
+    }
+    if (np)
+        a.grp[g] = {c0, r0, (uint32_t)(c1 - c0), (uint32_t)(r1 - r0)};
+    if (np > kLargeGroup)
+        a.huge[atomicAdd(a.nhuge, 1u)] = (uint32_t)g;
+    else if (np > kSmallGroup)
+        a.large[atomicAdd(a.nlarge, 1u)] = (uint32_t)g;
+    return np;
+}
+
+// A block takes kGroupTile groups, a thread each; the few that are not short
+// are listed and counted at the end, so that their searches fill waves of
+// their own instead of holding up every wave.
+constexpr uint32_t kGroupTile = 2048;
+
+__global__ void __launch_bounds__(kTB) k_join_count(JoinArgs a)
+{
+    __shared__ uint16_t list[kGroupTile];
+    __shared__ uint32_t nlist;
+    for (uint64_t g0 = (uint64_t)blockIdx.x * kGroupTile; g0 < a.cngroups;
+         g0 += (uint64_t)gridDim.x * kGroupTile) {
+        if (threadIdx.x == 0)
+            nlist = 0;
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < kGroupTile; i += kTB) {
+            const uint64_t g = g0 + i;
+            if (g >= a.cngroups)
+                break;
+            const uint64_t gs = a.cgstart[g], ge = a.cgend[g];
+            if (a.one_set && ge - gs <= kShort) {
+                const ShortGroup sg(a, gs, ge);
+                uint32_t np = 0;
+                for (uint32_t x = 0; x < kShort; ++x)
+                    for (uint32_t y = 0; y < kShort; ++y)
+                        np += sg.product(x, y) ? 1 : 0;
+                a.pcount[g] = np;
+            } else {
+                list[atomicAdd(&nlist, 1u)] = (uint16_t)i;
+            }
         }
-        a.ca[g] = c0;
-        a.ra[g] = r0;
-        a.cn[g] = (uint32_t)(c1 - c0);
-        a.rn[g] = (uint32_t)(r1 - r0);
-        a.pcount[g] = (c1 - c0) * (r1 - r0);
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < nlist; i += kTB) {
+            const uint64_t g = g0 + list[i];
+            a.pcount[g] = join_group(a, g, a.cgstart[g], a.cgend[g]);
+        }
+        __syncthreads();
     }
 }
 
 struct EmitArgs {
     const uint64_t *poff;     // exclusive scan of products per group
-    uint64_t ngroups, nprod;
-    const uint64_t *ca, *ra;
-    const uint32_t *cn, *rn;
-    const uint32_t *gcode;
+    uint64_t ngroups;
+    const JoinGroup *grp;
+    const int16_t *gcost;
     const uint64_t *cvals, *rvals;
-    KmerAlphabet alph;
-    int k;
+    const uint64_t *cgstart, *cgend;
+    bool one_set;
     int sym;                  // pa_symmetric
-    uint64_t row_base, col_base, c_begin;
+    uint64_t row_base, col_base, c_begin, c_end;
     int rbits;
     uint64_t keymax;
     uint64_t *pkey, *pval;
     unsigned long long *ndrop;
+    const uint64_t *pcount;
+    uint64_t up_off;
+    const uint32_t *large, *huge, *nlarge, *nhuge;
 };
 
-// self score of a k-mer code (sum over its letters' representatives)
-__device__ inline int code_cost(uint32_t code, const KmerAlphabet &al, int k)
+// Products [t0, t1) of group g (column occurrence outer), every step-th: each
+// to put(its place from poff[g] on, key, value); returns the number dropped.
+template <class Put>
+__device__ inline uint64_t emit_group(const EmitArgs &a, uint64_t g, uint64_t t0,
+                                      uint64_t t1, uint64_t step, Put put)
 {
-    // representative self score per alphabet code: the first residue code
-    // mapped to it
-    int cost = 0;
-    for (int j = 0; j < k; ++j) {
-        const uint32_t d = code % (uint32_t)al.size;
-        code /= (uint32_t)al.size;
-        int s = 0;
-        for (int x = 0; x < kAlpha; ++x)
-            if (al.code[x] == d) {
-                s = al.self[x];
-                break;
+    const JoinGroup j = a.grp[g];
+    const uint64_t ca = j.ca, ra = j.ra, rn = j.rn, off = a.poff[g];
+    const uint32_t cn = j.cn;
+    const uint64_t cost = (uint16_t)a.gcost[g];
+    const bool tri = a.sym == PA_SYM_UPPER && cn <= kTriCols;
+    uint64_t drop = 0, bi = 0, first = 0, width = 0;
+    if (tri)
+        width = rows_below(a.rvals, ra, rn, a.cvals[ca] >> 16, a.up_off);
+    for (uint64_t t = t0; t < t1; t += step) {
+        uint64_t ai;
+        if (tri) {   // products first .. first + width of column bi
+            while (t - first >= width) {
+                first += width;
+                ++bi;
+                width = rows_below(a.rvals, ra, rn, a.cvals[ca + bi] >> 16,
+                                   a.up_off);
             }
-        cost += s;
+            ai = t - first;
+        } else {
+            bi = t / rn;
+            ai = t % rn;
+        }
+        const uint64_t cv = a.cvals[ca + bi], rv = a.rvals[ra + ai];
+        const uint64_t c = cv >> 16, r = rv >> 16;
+        const bool keep = keep_product(a.sym, r + a.row_base, c + a.col_base);
+        put(off + t, keep ? ((c - a.c_begin) << a.rbits) | r : a.keymax,
+            ((rv & 0xffffull) << 48) | ((cv & 0xffffull) << 32) | cost);
+        drop += keep ? 0 : 1;
     }
-    return cost;
+    return drop;
 }
 
-constexpr int kPerThread = 8;
-
-// Products in the order of the scanned group offsets: thread t emits
-// products [8t, 8t + 8); inside a group, column occurrence outer.
-__global__ void k_emit_products(EmitArgs a)
+template <class Put>
+__device__ inline void emit_short(const EmitArgs &a, uint64_t g, uint64_t gs,
+                                  uint64_t ge, Put put)
 {
+    uint64_t at = a.poff[g];
+    const uint64_t cost = (uint16_t)a.gcost[g];
+    const ShortGroup sg(a, gs, ge);
+    for (uint32_t x = 0; x < kShort; ++x)
+        for (uint32_t y = 0; y < kShort; ++y)
+            if (sg.product(x, y)) {
+                const uint64_t cv = sg.v[x], rv = sg.v[y];
+                put(at++, (((cv >> 16) - a.c_begin) << a.rbits) | rv >> 16,
+                    ((rv & 0xffffull) << 48) | ((cv & 0xffffull) << 32) | cost);
+            }
+}
+
+// Groups of up to kSmallGroup products, a thread each, as in k_join_count.
+// The short ones of kTB neighbouring groups fill neighbouring places, which
+// are gathered in LDS and written in order; places of other groups are left
+// out there.  Before, the group of every eighth product was searched among all
+// groups: 1.06 ms per block of 17 million products, most of them dropped; now
+// 136 us for the 3.9 million that are kept.
+constexpr uint32_t kStage = 1024;
+
+__global__ void __launch_bounds__(kTB) k_emit_small(EmitArgs a)
+{
+    __shared__ uint64_t key[kStage], val[kStage];
+    __shared__ uint16_t list[kGroupTile];
+    __shared__ uint32_t nlist;
     uint64_t drop = 0;
-    const uint64_t t0 =
-        ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) * kPerThread;
-    if (t0 < a.nprod) {
-        // group of product t0: last g with poff[g] <= t0 and a product
-        uint64_t lo = 0, hi = a.ngroups - 1;
-        while (lo < hi) {
-            const uint64_t mid = (lo + hi + 1) / 2;
-            if (a.poff[mid] <= t0)
-                lo = mid;
-            else
-                hi = mid - 1;
+    for (uint64_t t0 = (uint64_t)blockIdx.x * kGroupTile; t0 < a.ngroups;
+         t0 += (uint64_t)gridDim.x * kGroupTile) {
+        if (threadIdx.x == 0)
+            nlist = 0;
+        for (uint32_t i0 = 0; i0 < kGroupTile && t0 + i0 < a.ngroups;
+             i0 += kTB) {
+            const uint64_t g0 = t0 + i0, g = g0 + threadIdx.x;
+            const uint64_t g1 = g0 + kTB < a.ngroups ? g0 + kTB : a.ngroups;
+            const uint64_t base = a.poff[g0], n = a.poff[g1] - base;
+            const bool stage = n <= kStage;
+            if (stage)
+                for (uint32_t i = threadIdx.x; i < n; i += kTB)
+                    key[i] = ~0ull;
+            __syncthreads();
+            const uint64_t np = g < a.ngroups ? a.pcount[g] : 0;
+            if (np > 0 && np <= kSmallGroup) {
+                const uint64_t gs = a.cgstart[g], ge = a.cgend[g];
+                if (a.one_set && ge - gs <= kShort)
+                    emit_short(a, g, gs, ge,
+                               [&](uint64_t at, uint64_t k, uint64_t v) {
+                                   if (stage) {
+                                       key[at - base] = k;
+                                       val[at - base] = v;
+                                   } else {
+                                       a.pkey[at] = k;
+                                       a.pval[at] = v;
+                                   }
+                               });
+                else
+                    list[atomicAdd(&nlist, 1u)] = (uint16_t)(i0 + threadIdx.x);
+            }
+            __syncthreads();
+            if (stage)
+                for (uint32_t i = threadIdx.x; i < n; i += kTB)
+                    if (key[i] != ~0ull) {
+                        a.pkey[base + i] = key[i];
+                        a.pval[base + i] = val[i];
+                    }
+            __syncthreads();
         }
-        uint64_t g = lo;
-        uint64_t local = t0 - a.poff[g];
-        int cost = -1;
-        uint64_t cost_g = ~0ull;
-        const uint64_t t1 = t0 + kPerThread < a.nprod ? t0 + kPerThread : a.nprod;
-        for (uint64_t t = t0; t < t1; ++t) {
-            while ((uint64_t)a.cn[g] * a.rn[g] <= local) {
-                local = 0;
-                ++g;
-            }
-            if (cost_g != g) {
-                cost = code_cost(a.gcode[g], a.alph, a.k);
-                cost_g = g;
-            }
-            const uint64_t bi = local / a.rn[g], ai = local % a.rn[g];
-            const uint64_t cv = a.cvals[a.ca[g] + bi];
-            const uint64_t rv = a.rvals[a.ra[g] + ai];
-            const uint64_t c = cv >> 16, r = rv >> 16;
-            const uint64_t R = r + a.row_base, C = c + a.col_base;
-            bool keep = true;
-            if (a.sym == PA_SYM_UPPER) {
-                keep = C > R;
-            } else if (a.sym == PA_SYM_EVEN_ODD) {
-                const bool ro = R & 1, co = C & 1;
-                keep = !(R == C || (R > C ? (ro ^ co) : !(ro ^ co)));
-            }
-            a.pkey[t] = keep ? ((c - a.c_begin) << a.rbits) | r : a.keymax;
-            a.pval[t] = ((rv & 0xffffull) << 48) | ((cv & 0xffffull) << 32) |
-                        (uint64_t)(uint16_t)(int16_t)cost;
-            drop += keep ? 0 : 1;
-            ++local;
+        for (uint32_t i = threadIdx.x; i < nlist; i += kTB) {
+            const uint64_t g = t0 + list[i];
+            drop += emit_group(a, g, 0, a.pcount[g], 1,
+                               [&](uint64_t at, uint64_t k, uint64_t v) {
+                                   a.pkey[at] = k;
+                                   a.pval[at] = v;
+                               });
         }
+        __syncthreads();
+    }
+    if (drop)
+        atomicAdd(a.ndrop, (unsigned long long)drop);
+}
+
+__global__ void __launch_bounds__(kTB) k_emit_large(EmitArgs a)
+{
+    auto put = [&](uint64_t at, uint64_t k, uint64_t v) {
+        a.pkey[at] = k;
+        a.pval[at] = v;
+    };
+    uint64_t drop = 0;
+    for (uint32_t k = blockIdx.x; k < *a.nlarge; k += gridDim.x) {
+        const uint64_t g = a.large[k];
+        drop += emit_group(a, g, threadIdx.x, a.pcount[g], kTB, put);
+    }
+    for (uint32_t k = 0; k < *a.nhuge; ++k) {
+        const uint64_t g = a.huge[k];
+        drop += emit_group(a, g,
+                           (uint64_t)blockIdx.x * kTB + threadIdx.x,
+                           a.pcount[g], (uint64_t)gridDim.x * kTB, put);
     }
     if (drop)
         atomicAdd(a.ndrop, (unsigned long long)drop);
@@ -471,10 +717,24 @@ int scan_flags(pa_ctx *c, KmerState *K, const uint32_t *in, uint64_t *out,
     return PA_OK;
 }
 
-template <class T> int d2h_value(pa_ctx *c, T *dst, const T *src, hipStream_t s)
+// Value i of src to the host's pinned words, ready after the next wait for
+// the stream (a copy to pageable memory costs 20 us more).
+template <class T> int d2h_start(pa_ctx *c, KmerState *K, int i, const T *src,
+                                 hipStream_t s)
 {
-    KCHK(c, hipMemcpyAsync(dst, src, sizeof(T), hipMemcpyDeviceToHost, s));
+    KCHK(c, hipMemcpyAsync(&K->host[i], src, sizeof(T), hipMemcpyDeviceToHost,
+                           s));
+    return PA_OK;
+}
+
+template <class T> int d2h_value(pa_ctx *c, KmerState *K, T *dst, const T *src,
+                                 hipStream_t s)
+{
+    int rc;
+    if ((rc = d2h_start(c, K, 0, src, s)))
+        return rc;
     KCHK(c, hipStreamSynchronize(s));
+    std::memcpy(dst, &K->host[0], sizeof(T));
     return PA_OK;
 }
 
@@ -501,7 +761,8 @@ int build_set(pa_ctx *c, KmerState *K, KmerSet &S, bool rows,
     S.stride = kc.stride;
     S.alph = kc.alphabet;
     S.gen = c->seq_gen;
-    S.nocc = S.ngroups = 0;
+    S.nocc = 0;
+    S.groups[0].built = S.groups[1].built = false;
     if (nslots == 0)
         return PA_OK;
     if ((rc = grow(c, K->slots, (nseq + 1) * 8)) ||
@@ -537,30 +798,47 @@ int build_set(pa_ctx *c, KmerState *K, KmerSet &S, bool rows,
                  P<uint64_t>(K->vals_a), P<uint64_t>(S.vals), nslots, 0, kbits,
                  s));
     uint64_t nbad = 0;
-    if ((rc = d2h_value(c, &nbad, P<uint64_t>(K->cnt), s)))
+    if ((rc = d2h_value(c, K, &nbad, P<uint64_t>(K->cnt), s)))
         return rc;
     S.nocc = nslots - nbad;
-    if (S.nocc == 0)
+    return PA_OK;
+}
+
+// Group table over the valid occurrences of a set; multi leaves out the codes
+// that occur once.
+int build_groups(pa_ctx *c, KmerState *K, KmerSet &S, bool multi,
+                 const KmerAlphabet &al, hipStream_t s)
+{
+    KmerGroups &T = S.groups[multi];
+    if (T.built)
         return PA_OK;
-    // group table over the valid occurrences
-    if ((rc = grow(c, K->heads, S.nocc * 4)) ||
-        (rc = grow(c, K->runid, S.nocc * 8)))
-        return rc;
-    hipLaunchKernelGGL(k_group_heads, dim3(nblocks(S.nocc)), dim3(kTB), 0, s,
-                       P<uint32_t>(S.keys), S.nocc, P<uint32_t>(K->heads));
-    if ((rc = scan_flags(c, K, P<uint32_t>(K->heads), P<uint64_t>(K->runid),
-                         S.nocc, true, s)))
-        return rc;
-    if ((rc = d2h_value(c, &S.ngroups, P<uint64_t>(K->runid) + S.nocc - 1, s)))
-        return rc;
-    if ((rc = grow(c, S.gstart, S.ngroups * 8)) ||
-        (rc = grow(c, S.gcode, S.ngroups * 4)))
-        return rc;
-    hipLaunchKernelGGL(k_group_table, dim3(nblocks(S.nocc)), dim3(kTB), 0, s,
-                       P<uint32_t>(S.keys), P<uint32_t>(K->heads),
-                       P<uint64_t>(K->runid), S.nocc, P<uint64_t>(S.gstart),
-                       P<uint32_t>(S.gcode));
-    KCHK(c, hipGetLastError());
+    T.n = 0;
+    int rc;
+    if (S.nocc) {
+        if ((rc = grow(c, K->heads, S.nocc * 4)) ||
+            (rc = grow(c, K->runid, S.nocc * 8)))
+            return rc;
+        hipLaunchKernelGGL(k_group_heads, dim3(nblocks(S.nocc)), dim3(kTB), 0,
+                           s, P<uint32_t>(S.keys), S.nocc, multi,
+                           P<uint32_t>(K->heads));
+        if ((rc = scan_flags(c, K, P<uint32_t>(K->heads), P<uint64_t>(K->runid),
+                             S.nocc, true, s)) ||
+            (rc = d2h_value(c, K, &T.n, P<uint64_t>(K->runid) + S.nocc - 1, s)))
+            return rc;
+    }
+    if (T.n) {
+        if ((rc = grow(c, T.start, T.n * 8)) ||
+            (rc = grow(c, T.end, T.n * 8)) ||
+            (rc = grow(c, T.code, T.n * 4)) || (rc = grow(c, T.cost, T.n * 2)))
+            return rc;
+        hipLaunchKernelGGL(k_group_table, dim3(nblocks(S.nocc)), dim3(kTB), 0,
+                           s, P<uint32_t>(S.keys), P<uint32_t>(K->heads),
+                           P<uint64_t>(K->runid), S.nocc, multi, al, S.k,
+                           P<uint64_t>(T.start), P<uint64_t>(T.end),
+                           P<uint32_t>(T.code), P<int16_t>(T.cost));
+        KCHK(c, hipGetLastError());
+    }
+    T.built = true;
     return PA_OK;
 }
 
@@ -595,21 +873,32 @@ int generate(pa_ctx *c, KmerState *K, const pa_kmer_config &kc, uint64_t cb,
         return rc;
     KmerSet &R = K->rows;
     *n = 0;
-    if (C.ngroups == 0 || R.nocc == 0 || cb >= ce)
+    const uint64_t up_off = kc.col_base - kc.row_base;
+    // a lone occurrence of a code meets only itself, and the symmetric rules
+    // drop that: 14 million groups of 60,000 sequences become 3.7 million
+    const bool multi = shared && kc.symmetric != PA_SYM_NONE && up_off == 0;
+    if ((rc = build_groups(c, K, C, multi, al, s)))
+        return rc;
+    KmerGroups &T = C.groups[multi];
+    if (T.n == 0 || R.nocc == 0 || cb >= ce)
         return PA_OK;
-    const uint64_t G = C.ngroups;
+    const uint64_t G = T.n;
     if ((rc = grow(c, K->pcount, (G + 1) * 8)) ||
         (rc = grow(c, K->poff, (G + 1) * 8)) ||
-        (rc = grow(c, K->gscr, G * 24)))
+        (rc = grow(c, K->gscr, G * 32)) || (rc = grow(c, K->cnt, 64)))
         return rc;
-    // per group: first column / row occurrence (u64), their counts (u32)
     uint64_t *pcount = P<uint64_t>(K->pcount);
-    uint64_t *ca = P<uint64_t>(K->gscr), *ra = ca + G;
-    uint32_t *cn = (uint32_t *)(ra + G), *rn = cn + G;
-    JoinArgs ja{P<uint64_t>(C.gstart), P<uint32_t>(C.gcode), P<uint64_t>(C.vals),
-                G, C.nocc, P<uint32_t>(R.keys), R.nocc, P<uint64_t>(R.gstart),
-                shared, cb, ce, ca, ra, cn, rn, pcount};
-    hipLaunchKernelGGL(k_join_count, dim3(nblocks(G)), dim3(kTB), 0, s, ja);
+    JoinGroup *grp = P<JoinGroup>(K->gscr);
+    uint32_t *large = (uint32_t *)(grp + G), *huge = large + G;
+    // counters: dropped products (u64), large and huge groups
+    uint32_t *ngr = P<uint32_t>(K->cnt) + 2;
+    KCHK(c, hipMemsetAsync(K->cnt.p, 0, 64, s));
+    JoinArgs ja{P<uint64_t>(T.start), P<uint64_t>(T.end), P<uint32_t>(T.code),
+                P<uint64_t>(C.vals), G, P<uint32_t>(R.keys), R.nocc, shared,
+                shared && up_off == 0, cb, ce, grp, pcount, P<uint64_t>(R.vals),
+                kc.symmetric, up_off, large, huge, ngr, ngr + 1};
+    hipLaunchKernelGGL(k_join_count, dim3(nblocks(G, kGroupTile)), dim3(kTB), 0,
+                       s, ja);
     KCHK(c, hipGetLastError());
     {
         size_t tmp = 0;
@@ -624,9 +913,13 @@ int generate(pa_ctx *c, KmerState *K, const pa_kmer_config &kc, uint64_t cb,
                                                  P<uint64_t>(K->poff), G + 1,
                                                  s));
     }
-    uint64_t nprod = 0;
-    if ((rc = d2h_value(c, &nprod, P<uint64_t>(K->poff) + G, s)))
+    if ((rc = d2h_start(c, K, 0, P<uint64_t>(K->poff) + G, s)) ||
+        (rc = d2h_start(c, K, 1, (uint64_t *)ngr, s)))
         return rc;
+    KCHK(c, hipStreamSynchronize(s));
+    const uint64_t nprod = K->host[0];
+    const uint32_t nlarge = (uint32_t)K->host[1];
+    const uint32_t nhuge = (uint32_t)(K->host[1] >> 32);
     if (nprod == 0)
         return PA_OK;
     const uint64_t ncols_blk = ce - cb;
@@ -638,18 +931,27 @@ int generate(pa_ctx *c, KmerState *K, const pa_kmer_config &kc, uint64_t cb,
     const uint64_t keymax = (1ull << (rbits + cbits)) - 1ull;   // unused key
     if ((rc = grow(c, K->pkey, nprod * 8)) || (rc = grow(c, K->pval, nprod * 8)) ||
         (rc = grow(c, K->pkey2, nprod * 8)) ||
-        (rc = grow(c, K->pval2, nprod * 8)) || (rc = grow(c, K->cnt, 64)))
+        (rc = grow(c, K->pval2, nprod * 8)))
         return rc;
-    KCHK(c, hipMemsetAsync(K->cnt.p, 0, 64, s));
-    EmitArgs ea{P<uint64_t>(K->poff), G, nprod, ca, ra, cn, rn,
-                P<uint32_t>(C.gcode), P<uint64_t>(C.vals), P<uint64_t>(R.vals),
-                al, kc.k, kc.symmetric, kc.row_base, kc.col_base, cb, rbits,
+    EmitArgs ea{P<uint64_t>(K->poff), G, grp,
+                P<int16_t>(T.cost), P<uint64_t>(C.vals), P<uint64_t>(R.vals),
+                P<uint64_t>(T.start), P<uint64_t>(T.end),
+                shared && up_off == 0, kc.symmetric, kc.row_base,
+                kc.col_base, cb, ce, rbits,
                 keymax, P<uint64_t>(K->pkey), P<uint64_t>(K->pval),
-                (unsigned long long *)K->cnt.p};
-    hipLaunchKernelGGL(k_emit_products,
-                       dim3(nblocks((nprod + kPerThread - 1) / kPerThread)),
-                       dim3(kTB), 0, s, ea);
+                (unsigned long long *)K->cnt.p, pcount, up_off, large, huge,
+                ngr, ngr + 1};
+    hipLaunchKernelGGL(k_emit_small, dim3(nblocks(G, kGroupTile)), dim3(kTB), 0,
+                       s, ea);
+    if (nlarge || nhuge)
+        hipLaunchKernelGGL(k_emit_large,
+                           dim3(nhuge ? 1024u : std::min(nlarge, 1024u)),
+                           dim3(kTB), 0, s, ea);
     KCHK(c, hipGetLastError());
+    // the number of dropped products arrives while they are sorted
+    if ((rc = d2h_start(c, K, 0, P<uint64_t>(K->cnt), s)))
+        return rc;
+    KCHK(c, hipEventRecord(c->ev_fork[0], s));
     {
         size_t tmp = 0;
         KCHK(c, hipcub::DeviceRadixSort::SortPairs(
@@ -663,9 +965,8 @@ int generate(pa_ctx *c, KmerState *K, const pa_kmer_config &kc, uint64_t cb,
                      P<uint64_t>(K->pval), P<uint64_t>(K->pval2), nprod, 0,
                      rbits + cbits, s));
     }
-    uint64_t ndrop = 0;
-    if ((rc = d2h_value(c, &ndrop, P<uint64_t>(K->cnt), s)))
-        return rc;
+    KCHK(c, hipEventSynchronize(c->ev_fork[0]));
+    const uint64_t ndrop = K->host[0];
     const uint64_t np = nprod - ndrop;   // dropped products sort last
     if (np == 0)
         return PA_OK;
@@ -677,7 +978,7 @@ int generate(pa_ctx *c, KmerState *K, const pa_kmer_config &kc, uint64_t cb,
                          np, true, s)))
         return rc;
     uint64_t nruns = 0;
-    if ((rc = d2h_value(c, &nruns, P<uint64_t>(K->runid) + np - 1, s)))
+    if ((rc = d2h_value(c, K, &nruns, P<uint64_t>(K->runid) + np - 1, s)))
         return rc;
     if ((rc = grow(c, K->rstart, nruns * 8)) ||
         (rc = grow(c, K->keep, nruns * 4 + 8)) ||
@@ -698,11 +999,11 @@ int generate(pa_ctx *c, KmerState *K, const pa_kmer_config &kc, uint64_t cb,
     if ((rc = scan_flags(c, K, P<uint32_t>(K->keep), P<uint64_t>(K->kpos),
                          nruns, false, s)))
         return rc;
-    uint64_t last = 0;
-    uint32_t lastkeep = 0;
-    if ((rc = d2h_value(c, &last, P<uint64_t>(K->kpos) + nruns - 1, s)) ||
-        (rc = d2h_value(c, &lastkeep, P<uint32_t>(K->keep) + nruns - 1, s)))
+    if ((rc = d2h_start(c, K, 0, P<uint64_t>(K->kpos) + nruns - 1, s)) ||
+        (rc = d2h_start(c, K, 1, P<uint32_t>(K->keep) + nruns - 1, s)))
         return rc;
+    KCHK(c, hipStreamSynchronize(s));
+    const uint64_t last = K->host[0], lastkeep = (uint32_t)K->host[1];
     const uint64_t nout = last + lastkeep;
     hipLaunchKernelGGL(k_compact, dim3(nblocks(nruns)), dim3(kTB), 0, s,
                        P<pa_pair>(K->pkey), P<uint32_t>(K->keep),
@@ -738,6 +1039,8 @@ extern "C" int pa_kmer_candidates(pa_ctx *c, const pa_kmer_config *kc,
     if (!c->kmer)
         c->kmer = new KmerState();
     KmerState *K = c->kmer;
+    if (!K->host)
+        KCHK(c, hipHostMalloc((void **)&K->host, 64, hipHostMallocDefault));
     hipStream_t s = c->st;
     int rc;
     if (!(K->have_last && same_cfg(K->last, *kc) && K->last_cb == c_begin &&
