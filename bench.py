@@ -137,8 +137,8 @@ def roofline(kstats, st, step_ms_total, tuning=None, traffic_key=None):
         tn = tuning or {}
         chain = ["k_xdrop_coop"] if tn.get("xd_coop") else []
         chain.append("k_xdrop_pl<%d>" % tn.get("xd_ring", 16))
-        chain += {0: [], 1: ["k_xdrop_band<8>", "k_xdrop_band<16>"],
-                  2: ["k_xdrop_band<16>"]}[tn.get("xd_wave", 1)]
+        chain += {0: [], 1: ["k_xdrop_band<4>", "k_xdrop_band<8>"],
+                  2: ["k_xdrop_band<8>"]}[tn.get("xd_wave", 1)]
         chain.append("k_xdrop_pl<0>")
         xk = "X-drop stage: " + " -> ".join(chain)
         cands.append(dict(kernel=xk, ms=st["ms_xdrop"],

@@ -1,27 +1,40 @@
 // k_xdrop_wave.hip -- gapped X-drop seed extension with one 16-lane row of a
-// wave per work item (four items per wave), for the items whose band
-// outgrows the per-lane kernel's LDS rings (k_xdrop.hip).  Same algorithm,
-// step for step, as k_xdrop_pl and the oracle's or_xdrop_one (SeqAn's
-// one-direction GappedXDrop as called at
+// wave per work item (four items per wave), for bands wider than the other
+// kernels hold.  Same algorithm, step for step, as k_xdrop_pl and the oracle's
+// or_xdrop_one (SeqAn's one-direction GappedXDrop as called at
 // src/align/SeqanXdropAligner.cpp:281-283), so extents and evaluated-cell
 // counts are bit-identical.
 //
-// The cells of one anti-diagonal depend only on the two before it, so the 16
-// lanes of an item evaluate 16 consecutive columns at once.  The item's three
-// live anti-diagonals stay in registers: lane j holds, for each of kChunks
-// chunks c, column base + 16c + j of each (a window of kWin columns starting
-// at `base`).  The value of column col - 1 comes from the neighbouring lane
-// through DPP row_shr:1, whose first lane keeps the DPP "old" operand, lane 15
-// of the chunk below rotated in with row_ror:1.  The window moves up a chunk
-// when the oldest anti-diagonal's range has left its first chunk; an item
-// whose band outgrows the window is handed on to the global-ring kernel
-// through the overflow list.  The anti-diagonal's best score is a row
-// maximum (row_ror 1, 2, 4, 8) and the band update two ballots (the first
-// column from the left and the last from the right that stay live).  Query
-// residues sit in registers per column; database residues are loaded two
-// anti-diagonals ahead and turned into substitution scores one ahead, so no
-// step waits on memory.  A row that finishes its item takes the next one
-// from a range its wave claims with one queue atomic.
+// The cells of one anti-diagonal depend only on the two before it, so all of
+// them are evaluated at once.  A lane holds a block of BL neighbouring columns,
+// two 16-bit values a register, and the 16 lanes a window of W = 16 BL
+// columns; column c sits at place c mod W, and a lane whose block the band has
+// left behind takes the block W columns further.  So nothing is moved when the
+// band moves, and column c - 1 is a register shift, or one DPP rotation at a
+// block's first column.
+//   - Values are kept as v + X in int16, the undefined cell as -32768: a cell
+//     kept on anti-diagonal d is at least best - X, so a defined value is not
+//     negative, "undefined" is its sign, saturating sums of an undefined cell
+//     stay undefined, and the limit in these units is the best score itself.
+//     An item whose best score nears the type's range, or whose band nears
+//     the window (W - 3 BL columns), is handed on through the overflow list:
+//     from the 128-column to the 256-column kernel, then to the rings in
+//     global memory.
+//   - Outside the range [minCol, maxCol) of an anti-diagonal the recurrence
+//     gives undefined cells by itself: the columns that the update of minCol
+//     passes are undefined on both anti-diagonals it reads, and so are those
+//     from two past the last defined one.  Only where minCol or maxCol was set
+//     by the ends of the segments, and in the first steps, where column 0 and
+//     row 0 hold gap scores, are the columns masked.
+//   - A lane's database residues move up one column a step (a byte shift); the
+//     one that enters comes from a ring in LDS, and so do the query residues
+//     of a new block.  The rings are filled every kSteps steps with what was
+//     loaded kSteps steps before.  A lane takes its new block at least BL + 2
+//     steps before the band gets there, when its residues are in place.
+// Bound by instructions, about 190 per step of four items; a column per lane
+// in 32-bit values (up to eight chunks of 16 columns) took over 450.  60,001
+// pairs, log-normal lengths to 3,000, X = 49, gap -2: the two windows 9.2 + 4.2
+// -> 4.7 + 1.3 ms.
 #include <limits.h>
 
 #include "pa_internal.h"
@@ -29,17 +42,17 @@
 namespace pa {
 namespace {
 
-constexpr int32_t kUndef = INT_MIN / 4;
-constexpr int kW = 16;                // lanes per item
 constexpr uint32_t kClaim = 4;        // items claimed per queue atomic
-// window of the main pass (128 columns) and of the pass that takes its
-// overflow (256 columns; few items, so its register use does not matter)
-constexpr int kBandChunks = 8;
-constexpr int kWideChunks = 16;
+constexpr int kSteps = 16;            // anti-diagonals between ring refills
+// registers per lane and anti-diagonal: windows of 128 and 256 columns
+constexpr int kBandRegs = 4;
+constexpr int kWideRegs = 8;
+constexpr uint32_t kUndef2 = 0x80008000u;
+constexpr int kUndef = -32768;
 
 struct WaveArgs {
     const XdTask *tasks;
-    const uint32_t *list;   // work items (k = 2 * task + dir)
+    const uint32_t *list;   // work items (k = 2 * task + dir), NULL = 0..count
     const uint32_t *count;
     uint32_t *queue;
     const int8_t *mat;
@@ -48,157 +61,175 @@ struct WaveArgs {
     uint32_t *ovf_list, *ovf_count;
 };
 
+typedef short s2v __attribute__((ext_vector_type(2)));
+typedef unsigned short u2v __attribute__((ext_vector_type(2)));
+// a register's two values stored over int16 places
+typedef uint32_t __attribute__((may_alias)) u32a;
+
+__device__ inline s2v sv(uint32_t x) { return __builtin_bit_cast(s2v, x); }
+__device__ inline uint32_t uv(s2v x) { return __builtin_bit_cast(uint32_t, x); }
+__device__ inline uint32_t pk_add(uint32_t a, uint32_t b)
+{
+    return uv(__builtin_elementwise_add_sat(sv(a), sv(b)));
+}
+__device__ inline uint32_t pk_sub(uint32_t a, uint32_t b)
+{
+    return uv(__builtin_elementwise_sub_sat(sv(a), sv(b)));
+}
+__device__ inline uint32_t pk_max(uint32_t a, uint32_t b)
+{
+    return uv(__builtin_elementwise_max(sv(a), sv(b)));
+}
+__device__ inline uint32_t pk_minu(uint32_t a, uint32_t b)
+{
+    return __builtin_bit_cast(
+        uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u2v, a),
+                                            __builtin_bit_cast(u2v, b)));
+}
+// all ones where negative
+__device__ inline uint32_t pk_neg(uint32_t a) { return uv(sv(a) >> (short)15); }
+__device__ inline uint32_t splat(int x)
+{
+    return __builtin_amdgcn_perm((uint32_t)x, (uint32_t)x, 0x01000100u);
+}
+
 // lane j of each 16-lane row reads lane j - K (mod 16) of its row (every
 // lane has a source, so no "old" operand: the compiler can fold the move
 // into the instruction that uses it)
 template <int K> __device__ inline int32_t ror(int32_t v)
 {
-    return __builtin_amdgcn_mov_dpp(v, 0x120 + K, 0xf, 0xf, false);
+    return __builtin_amdgcn_mov_dpp(v, 0x120 + K, 0xf, 0xf, true);
 }
 
-// Column col - 1 of the lanes' columns of a chunk: lanes 1..15 take lane
-// j - 1 of `cur`, lane 0 keeps the DPP "old" operand, lane 15 of `below`.
-__device__ inline int32_t left_of(int32_t cur, int32_t below)
+__device__ inline int row_max(int v)
 {
-    return __builtin_amdgcn_update_dpp(ror<1>(below), cur, 0x111, 0xf, 0xf,
-                                       false);
+    v = max(v, ror<1>(v));
+    v = max(v, ror<2>(v));
+    v = max(v, ror<4>(v));
+    v = max(v, ror<8>(v));
+    return v;
 }
 
-__device__ inline int32_t row_max(int32_t v)
+__device__ inline int row_min(int v)
 {
-    int32_t o = ror<1>(v);
-    v = o > v ? o : v;
-    o = ror<2>(v);
-    v = o > v ? o : v;
-    o = ror<4>(v);
-    v = o > v ? o : v;
-    o = ror<8>(v);
-    return o > v ? o : v;
+    v = min(v, ror<1>(v));
+    v = min(v, ror<2>(v));
+    v = min(v, ror<4>(v));
+    v = min(v, ror<8>(v));
+    return v;
 }
 
-__device__ inline int32_t row_min(int32_t v)
+// kEmpty: nothing to extend; kOut: handed on
+enum : int { kNeed = 0, kRun = 1, kDone = 2, kEmpty = 3, kOut = 4 };
+
+// The longest items are chains of thousands of steps, and the caller waits for
+// them: these waves issue ahead of those of another batch's DP that they share
+// a SIMD with.
+__device__ inline void band_first_issue()
 {
-    int32_t o = ror<1>(v);
-    v = o < v ? o : v;
-    o = ror<2>(v);
-    v = o < v ? o : v;
-    o = ror<4>(v);
-    v = o < v ? o : v;
-    o = ror<8>(v);
-    return o < v ? o : v;
+#ifdef __HIP_DEVICE_COMPILE__
+    __builtin_amdgcn_s_setprio(3);
+#endif
 }
 
-// maximum over the wave of a non-negative value
-__device__ inline int wave_max(int v)
-{
-    const int r = row_max(v);
-    const int a = __builtin_amdgcn_readlane(r, 0);
-    const int b = __builtin_amdgcn_readlane(r, 16);
-    const int c = __builtin_amdgcn_readlane(r, 32);
-    const int d = __builtin_amdgcn_readlane(r, 48);
-    const int ab = a > b ? a : b, cd = c > d ? c : d;
-    return ab > cd ? ab : cd;
-}
-
-// Writes the half of XdOut that item k (direction k & 1) owns.
-__device__ inline void wave_write(const WaveArgs &a, uint32_t k, int32_t score,
-                                  int col, int row, bool upd, uint32_t nc,
-                                  uint16_t flags)
-{
-    const XdTask T = a.tasks[k >> 1];
-    XdOut PA_GLOBAL &o = glb(a.out)[T.id];
-    const int beg_h = (int)T.beg_h, beg_v = (int)T.beg_v;
-    if ((k & 1) == 0) {
-        o.beg_h = upd ? beg_h - row : beg_h;
-        o.beg_v = upd ? beg_v - col : beg_v;
-        o.score_left = score;
-        o.cells_left = nc;
-        o.flags_left = flags;
-    } else {
-        const int end_h = beg_h + a.seed_len, end_v = beg_v + a.seed_len;
-        o.end_h = upd ? end_h + row : end_h;
-        o.end_v = upd ? end_v + col : end_v;
-        o.score_right = score;
-        o.cells_right = nc;
-        o.flags_right = flags;
-    }
-}
-
-enum : int { kIdle = 0, kRun = 1, kDone = 2 };
-
-// NCH chunks of 16 columns per lane: a window of 16 * NCH columns.
-template <int NCH>
+template <int NR>
 __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
 {
-    constexpr int kChunks = NCH;
-    constexpr int kWin = kW * kChunks;
+    band_first_issue();
+    constexpr int BL = 2 * NR;         // columns per lane
+    constexpr int W = 16 * BL;         // columns of the window
+    constexpr int QR = 4 * W, DR = 2 * W;   // residues per ring
+    constexpr int WL = W - 3 * BL;     // widest written range
     __shared__ int8_t mat[32 * 32];
-    const int lane = threadIdx.x, j = lane & (kW - 1), g = lane / kW;
+    __shared__ uint8_t rings[4 * (QR + DR)];
+    __shared__ int16_t dump[4 * 3 * W];   // three anti-diagonals at an end
+    const int lane = threadIdx.x, j = lane & 15, row = lane >> 4;
     for (int i = lane; i < 32 * 32; i += 64)
         mat[i] = a.mat[i];
+    // (residue codes are below 32: a slot not yet stored must be, too)
+    for (int i = lane; i < 4 * (QR + DR); i += 64)
+        rings[i] = 0;
     __syncthreads();
     const uint32_t n = *a.count;
-    const int gap = a.gap, X = a.X;
+    const int X = a.X, gap = max(a.gap, -32000);
+    const uint32_t GAP = splat(gap);
+    const int best_max = 32000 - X;
+    uint8_t *const qring = rings + row * (QR + DR);
+    uint8_t *const dring = qring + QR;
+    int16_t *const dmp = dump + row * 3 * W;
 
-    // Item of this lane's row; the same in all 16 lanes of the row.
-    int state = kIdle;
+    // row-uniform state of the current item
+    int state = kNeed;
     uint32_t k = 0;
-    const uint8_t PA_GLOBAL *qb = nullptr;
-    const uint8_t PA_GLOBAL *db = nullptr;
-    int qstep = 1, dstep = 1, cols = 2, rows = 2;
-    int d = 0, minCol = 0, maxCol = 0, best = 0, base = 0;
+    int cols = 0, rows = 0, d = 0, minCol = 0, maxCol = 0, best = 0;
     int off1 = 0, off2 = 0, off3 = 0, l1 = 0, l2 = 0, l3 = 0;
+    bool right = false, invalid = false;
     uint32_t nc = 0;
-    // this lane's column base + kW*c + j of anti-diagonals d-2, d-1, d
-    int32_t A1[kChunks], A2[kChunks], A3[kChunks];
-    int q[kChunks];             // query residue of the column
-    int32_t sc[kChunks];        // substitution score of the next step's cell
-    int B0[kChunks], B1[kChunks];   // database residues, loaded ahead
-    // column - 1 of A2 in this lane's columns, saved by each step: the next
-    // step's column - 1 of A1 (its diagonal input); kept by the 128-column
-    // pass only (the 256-column pass is at its register limit)
-    constexpr bool kKeepDL = NCH <= 8;
-    int32_t DL[kKeepDL ? kChunks : 1];
+    int64_t dgap = 0;       // d * gap, while a border cell is kept
+    bool edge = false;      // one may be
+    int masked = 0;         // steps that still need masks (INT_MAX: all)
+    const uint8_t PA_GLOBAL *qb = nullptr, *db = nullptr;
+    int qstep = 1;          // column c at qb[qstep * c], row r at db[qstep * r]
+    // rings: columns below qfill and rows below dfill are stored, the next W
+    // columns (BL a lane) and 16 rows are on their way
+    int qfill = 0, dfill = 0, dpre = 0;
+    uint64_t qpre[NR / 4];
+    // this lane's block: columns c0 + 2 r + h in half h of register r, values
+    // of anti-diagonals d (P), d-1 (O), d-2 (Z) and column - 1 of d-1 (LD)
+    int c0 = 0;
+    uint32_t P[NR], O[NR], Z[NR], LD[NR];
+    uint32_t Q[NR];         // query residues * 32
+    uint32_t R[NR / 2];     // database residues of anti-diagonal d + 1
+    int S0[NR], S1[NR];     // and its scores (joined where they are used, so
+                            // that no step waits for its own lookups)
+    int nb = 0;             // residue that enters for d + 2
 #pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
-        A1[c] = A2[c] = A3[c] = kUndef;
-        q[c] = 0;
-        sc[c] = 0;
-        B0[c] = B1[c] = 0;
-        if (kKeepDL)
-            DL[c] = kUndef;
+    for (int r = 0; r < NR; ++r) {
+        P[r] = O[r] = Z[r] = LD[r] = kUndef2;
+        Q[r] = 0;
+        S0[r] = S1[r] = 0;
+        R[r / 2] = 0;
+        qpre[r / 4] = 0;
     }
-    // DL does not hold this row's values (new item, or the window moved)
-    bool fresh = true;
-    int cw_prev = -1;   // chunks the previous step computed
     uint32_t cbase = 0, cend = 0;   // claimed, not yet handed out
-    // highest chunk any running row reaches in the coming step (set at the
-    // end of each step; a new item starts in chunk 0)
-    int cw_next = 0;
 
-    auto qres = [&](int col) {   // query residue of column col (clamped)
-        col = col < 1 ? 1 : (col > cols - 1 ? cols - 1 : col);
-        return (int)qb[qstep > 0 ? col : -col];
+    // residues of columns c .. c + 7 (0 past the end: up to seven bytes beside
+    // the segment are read, which the store's margins hold)
+    auto q_load8 = [&](int c) -> uint64_t {
+        typedef uint64_t __attribute__((aligned(1))) u64u;
+        if (c >= cols)
+            return 0;
+        if (qstep > 0)
+            return *(const u64u PA_GLOBAL *)(qb + c) & 0x1f1f1f1f1f1f1f1full;
+        return __builtin_bswap64(*(const u64u PA_GLOBAL *)(qb - c - 7)) &
+               0x1f1f1f1f1f1f1f1full;
     };
-    auto dres = [&](int row) {   // database residue of row (clamped)
-        row = row < 1 ? 1 : (row > rows - 1 ? rows - 1 : row);
-        return (int)db[dstep > 0 ? row : -row];
+    auto d_load = [&](int r) {
+        return r >= 1 && r < rows ? (int)db[qstep > 0 ? r : -r] : 0;
     };
-    // group value of column x of anti-diagonal array A (x in the window)
-    auto at = [&](const int32_t *A, int x) {
-        int32_t v = INT_MIN;
+    // query residues of the block as pairs, times 32
+    auto set_q = [&](const uint64_t *w) {
 #pragma unroll
-        for (int c = 0; c < kChunks; ++c)
-            v = base + kW * c + j == x ? A[c] : v;
-        return row_max(v);
+        for (int r = 0; r < NR; ++r) {
+            const uint32_t x = (uint32_t)(w[r / 4] >> (16 * (r % 4)));
+            Q[r] = ((x & 0xffu) | ((x & 0xff00u) << 8)) << 5;
+        }
+    };
+    auto scores = [&]() {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            // bytes 2r, 2r+1 as two halves
+            const uint32_t sel = r % 2 ? 0x0c030c02u : 0x0c010c00u;
+            const uint32_t ad =
+                Q[r] | __builtin_amdgcn_perm(0u, R[r / 2], sel);
+            S0[r] = mat[ad & 0xffffu];
+            S1[r] = mat[ad >> 16];
+        }
     };
 
-    // One half of the loop: claims for idle rows, then one anti-diagonal of
-    // every running item.  LOAD receives the database residues of the step
-    // after next, LOOK holds those of the next step (loaded a half before).
-    auto half = [&](int *LOAD, int *LOOK) {
-        // ---- claims (wave-uniform block; every lane runs it) -----------
-        uint64_t need = __ballot(state == kIdle && j == 0);
+    for (;;) {
+        // ---- hand out items to rows that need one (wave-uniform)
+        uint64_t need = __ballot(state == kNeed && j == 0);
         while (need) {
             if (cbase >= cend) {
                 uint32_t b = atomicAdd(a.queue, lane == 0 ? kClaim : 0u);
@@ -208,281 +239,318 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
             }
             const uint32_t cnt = (uint32_t)__popcll(need);
             const uint32_t take = min(cnt, cend - cbase);
-            // rank of this row among the rows asking
-            const uint64_t mine = 1ull << (g * kW);
-            const uint32_t rank = (uint32_t)__popcll(need & (mine - 1ull));
-            const bool asks = (need & mine) != 0;
-            if (asks && rank < take) {
+            const uint32_t rank =
+                (uint32_t)__popcll(need & ((1ull << (16 * row)) - 1ull));
+            const bool mine =
+                ((need >> (16 * row)) & 1ull) != 0 && rank < take;
+            if (mine) {
                 const uint32_t idx = cbase + rank;
                 if (idx >= n) {
                     state = kDone;
+                    cols = rows = 0;   // nothing more to load
                 } else {
-                    k = glb(a.list)[idx];
+                    k = a.list ? glb(a.list)[idx] : idx;
                     const XdTask T = a.tasks[k >> 1];
                     const uint8_t PA_GLOBAL *h = glb_addr<const uint8_t>(T.h_off);
                     const uint8_t PA_GLOBAL *v = glb_addr<const uint8_t>(T.v_off);
                     const int beg_h = (int)T.beg_h, beg_v = (int)T.beg_v;
-                    if ((k & 1) == 0) {
+                    right = (k & 1) != 0;
+                    if (!right) {   // query V[0, beg_v), database H[0, beg_h)
                         cols = beg_v + 1;
                         rows = beg_h + 1;
-                        qb = v + (cols - 1);
+                        qb = v + beg_v;
+                        db = h + beg_h;
                         qstep = -1;
-                        db = h + (rows - 1);
-                        dstep = -1;
-                    } else {
+                    } else {        // suffixes after the seed
                         cols = (int)T.nv - beg_v - a.seed_len + 1;
                         rows = (int)T.nh - beg_h - a.seed_len + 1;
                         qb = v + beg_v + a.seed_len - 1;
-                        qstep = 1;
                         db = h + beg_h + a.seed_len - 1;
-                        dstep = 1;
+                        qstep = 1;
                     }
-                    // item_init: anti-diagonals 0 (A2) and 1 (A3); the
-                    // step rotates them into A1 and A2
                     d = 1;
                     minCol = 1;
                     maxCol = 2;
-                    best = 0;
-                    base = 0;
                     off1 = off2 = off3 = 0;
                     l1 = 0;
                     l2 = 1;
                     l3 = 2;
+                    best = 0;
                     nc = 0;
-                    const int32_t g1 = -gap > X ? kUndef : gap;
-#pragma unroll
-                    for (int c = 0; c < kChunks; ++c) {
-                        const int col = kW * c + j;
-                        A2[c] = col == 0 ? 0 : kUndef;
-                        A3[c] = col <= 1 ? g1 : kUndef;
-                        q[c] = qres(col);
-                        // scores of step 2 (rows 2 - col) and residues of
-                        // step 3 (rows 3 - col)
-                        sc[c] = mat[q[c] * 32 + dres(2 - col)];
-                        LOOK[c] = dres(3 - col);
-                    }
-                    fresh = true;
+                    dgap = gap;
+                    edge = -gap <= X;
+                    masked = 3;
+                    invalid = (T.pad & kXdInvalid) != 0;
                     state = kRun;
+                    if (invalid || rows <= 1 || cols <= 1) {
+                        state = kEmpty;
+                    } else {
+                        // anti-diagonal 0: column 0 = 0; anti-diagonal 1:
+                        // columns 0 and 1 = gap (undefined when -gap > X)
+                        const uint32_t z = (uint32_t)X;
+                        const uint32_t g1 = -gap > X ? kUndef2 : splat(gap + X);
+#pragma unroll
+                        for (int r = 0; r < NR; ++r)
+                            P[r] = O[r] = LD[r] = Z[r] = kUndef2;
+                        if (j == 0) {
+                            O[0] = 0x80000000u | z;
+                            P[0] = g1;
+                            LD[0] = (z << 16) | 0x8000u;
+                        }
+                        c0 = j * BL;
+                        uint64_t w[NR / 4];
+#pragma unroll
+                        for (int q = 0; q < NR / 4; ++q) {
+                            w[q] = q_load8(c0 + 8 * q);
+                            qpre[q] = q_load8(W + c0 + 8 * q);
+                        }
+                        set_q(w);
+                        qfill = W;
+                        dring[1 + j] = (uint8_t)d_load(1 + j);
+                        dring[17 + j] = (uint8_t)d_load(17 + j);
+                        dfill = 33;
+                        dpre = d_load(33 + j);
+                        // anti-diagonal 2: column 1, row 1 only
+#pragma unroll
+                        for (int q = 0; q < NR / 2; ++q)
+                            R[q] = 0;
+                        if (j == 0)
+                            R[0] = (uint32_t)d_load(2) |
+                                   ((uint32_t)d_load(1) << 8);
+                        nb = j == 0 ? d_load(3) : 0;
+                        scores();
+                    }
                 }
             }
             cbase += take;
             for (uint32_t t = 0; t < take; ++t)
-                need &= need - 1;
+                need &= need - 1;   // the rows served
         }
+        if (!__ballot(state != kDone))
+            break;
 
-        // ---- one anti-diagonal of each running item ---------------------
-        // Every lane runs this part (the DPP moves, ballots and row maxima
-        // need whole rows, and the emulation of the tests needs the whole
-        // wave): rows without an item compute on stale registers, which the
-        // next claim resets, and only memory accesses and state changes are
-        // guarded by `run`.
-        bool run = state == kRun;
-        ++d;
+        // ---- rings for the next kSteps anti-diagonals.  Blocks are taken up
+        // to W - 1 columns above minCol - 1, which passes maxCol by no more
+        // than kSteps; rows enter at most BL columns below minCol, two
+        // anti-diagonals ahead.
+        if (qfill < minCol + kSteps + WL + W) {
 #pragma unroll
-        for (int c = 0; c < kChunks; ++c) {
-            A1[c] = A2[c];
-            A2[c] = A3[c];
-        }
-        l1 = l2;
-        l2 = l3;
-        off1 = off2;
-        off2 = off3;
-        off3 = minCol - 1;
-        l3 = maxCol + 1 - off3;
-        const int maxCol0 = maxCol;
-        if (run && maxCol0 - base >= kWin) {
-            // the band left the window: restart in the global-ring kernel
-            if (j == 0) {
-                const uint32_t pos = atomicAdd(a.ovf_count, 1u);
-                a.ovf_list[pos] = k;
-                wave_write(a, k, 0, 0, 0, false, 0, 1);
+            for (int q = 0; q < NR / 4; ++q) {
+                *(uint64_t *)(qring + ((qfill + j * BL + 8 * q) & (QR - 1))) =
+                    qpre[q];
+                qpre[q] = q_load8(qfill + W + j * BL + 8 * q);
             }
-            state = kIdle;
-            run = false;
+            qfill += W;
         }
-        const bool cond = (long)d * gap > (long)best - X;
-        const int32_t lim = best - X;
-        const int32_t dgap = d * gap;
-        int32_t adbest = dgap;
-        // the chunks any running row reads or writes this step: columns up
-        // to its maxCol0 (the others hold columns no step reads)
-        const int cw = cw_next;
-        // The diagonal input (column - 1 of A1) is the left input the
-        // previous step computed (column - 1 of its A2), unless a running
-        // row started an item or moved its window since, or the chunk is
-        // new this step.
-        const bool stale = __ballot(run && fresh) != 0;
-        // The new minCol is the first column c in [minCol, maxCol0] that
-        // does not satisfy (A3[c] undefined, c - 1 in A2's range, A2[c-1]
-        // undefined), or maxCol0 + 1 when all do; the new maxCol is one past
-        // the last column x in [off3, maxCol0) with A3[x] or A2[x] defined
-        // (off3 when none), plus one.  Each lane keeps its own candidates;
-        // one row minimum and maximum per step combine them.  x = col -
-        // minCol turns the ranges into single unsigned comparisons.
-        const int w = maxCol0 - minCol;
-        const int ecol0 = cond && off3 == 0 ? 0 : -1;   // edge columns
-        const int ecol1 = cond && d == maxCol0 ? maxCol0 : -1;
-        const int dlim = off2 + 1 + l2;   // c - 1 in A2's range: c < dlim
-        int32_t lo = INT_MAX, hi = INT_MIN;
+        if (dfill < d - minCol + kSteps + BL + 4) {
+            dring[(dfill + j) & (DR - 1)] = (uint8_t)dpre;
+            dfill += 16;
+            dpre = d_load(dfill + j);
+        }
+        // ---- kSteps anti-diagonals, or until a row's item ends.  Rows
+        // without an item compute on (their results go nowhere).
+        bool fin = state != kDone && !(state == kRun && minCol < maxCol);
+        uint64_t any = __ballot(fin);
+        for (int st = 0; st < kSteps && !any; ++st) {
+            const bool ovf = maxCol - minCol + 2 > WL || best > best_max;
+            const int noff3 = minCol - 1;
+            const int nl3 = maxCol + 1 - noff3;
+            ++d;
+            // column - 1
+            uint32_t L[NR], V[NR], m[NR];
+            L[0] = __builtin_amdgcn_alignbit(P[0], (uint32_t)ror<1>((int)P[NR - 1]), 16);
 #pragma unroll
-        for (int c = 0; c < kChunks; ++c) {
-            if (c > cw)
-                break;
-            const int col = base + kW * c + j;
-            const int x = col - minCol;
-            const int32_t u = A2[c];
-            const int32_t l = left_of(u, c ? A2[c - 1] : kUndef);
-            int32_t dl;
-            if (!kKeepDL || stale || c > cw_prev)
-                dl = left_of(A1[c], c ? A1[c - 1] : kUndef);
-            else
-                dl = DL[c];
-            if constexpr (kKeepDL)
-                DL[c] = l;
-            int32_t tmp = (l > u ? l : u) + gap;
-            const int32_t dg = dl + sc[c];
-            tmp = dg > tmp ? dg : tmp;
-            const bool inb = (uint32_t)x < (uint32_t)w;
-            const int32_t val = tmp < lim ? kUndef : tmp;
-            const bool edge = col == ecol0 || col == ecol1;
-            const int32_t a3 = inb ? val : (edge ? dgap : kUndef);
-            A3[c] = a3;
-            adbest = inb && val > adbest ? val : adbest;
-            const bool u3 = a3 == kUndef;
-            if ((uint32_t)x <= (uint32_t)w && !(u3 && col < dlim && l == kUndef))
-                lo = col < lo ? col : lo;
-            if ((uint32_t)(x + 1) < (uint32_t)(w + 1) && !(u3 && u == kUndef))
-                hi = col + 1;
+            for (int r = 1; r < NR; ++r)
+                L[r] = __builtin_amdgcn_alignbit(P[r], P[r - 1], 16);
+            const uint32_t BEST = splat(best);
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                const uint32_t sc = __builtin_amdgcn_perm(
+                    (uint32_t)S1[r], (uint32_t)S0[r], 0x05040100u);
+                V[r] = pk_max(pk_add(pk_max(P[r], L[r]), GAP),
+                              pk_add(LD[r], sc));
+                m[r] = pk_neg(pk_sub(V[r], BEST));
+            }
+            if (__ballot(masked > 0 && state == kRun)) {
+                const uint32_t lo = splat(c0 - minCol);
+                const uint32_t w1 = splat(maxCol - minCol - 1);
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    const uint32_t x =
+                        pk_add(lo, (uint32_t)(2 * r) | ((2 * r + 1) << 16));
+                    m[r] |= pk_neg(x) | pk_neg(pk_sub(w1, x));
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < NR; ++r)
+                V[r] = (m[r] & kUndef2) | (V[r] & ~m[r]);
+            uint32_t ab = V[0];
+#pragma unroll
+            for (int r = 1; r < NR; ++r)
+                ab = pk_max(ab, V[r]);
+            // cells of column 0 and row 0, while the gap to them is kept: d *
+            // gap falls and the limit does not, so once it is not, never again
+            if (__ballot(edge && state == kRun)) {
+                dgap += gap;
+                edge = edge && dgap > (int64_t)best - X;
+                if (edge) {
+                    const uint32_t e = (uint32_t)((int)dgap + X) & 0xffffu;
+                    masked = 3;
+                    if (c0 == 0 && noff3 == 0)
+                        V[0] = (V[0] & 0xffff0000u) | e;
+                    const int x = d - c0;
+                    if (d == maxCol && x >= 0 && x < BL) {
+#pragma unroll
+                        for (int r = 0; r < NR; ++r) {
+                            if (x == 2 * r)
+                                V[r] = (V[r] & 0xffff0000u) | e;
+                            if (x == 2 * r + 1)
+                                V[r] = (V[r] & 0xffffu) | (e << 16);
+                        }
+                    }
+                }
+            }
+            // minCol: the first column defined here or, at column - 1, on the
+            // anti-diagonal before; maxCol: two past the last column below it
+            // that is defined on either
+            uint32_t f = ~0u, g = ~0u;
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                const uint32_t at = (uint32_t)(2 * r) | ((2 * r + 1) << 16);
+                f = pk_minu(f, pk_neg(pk_max(V[r], L[r])) | at);
+                g = pk_max(g, pk_neg(pk_max(V[r], P[r])) | at);
+            }
+            const int fl = min((int)(f & 0xffffu), (int)(f >> 16));
+            const int gl = max((int)(int16_t)g, (int)g >> 16);
+            const int lo = row_min(c0 + fl);
+            const int hi = row_max(gl < 0 ? -1 : c0 + gl);
+            const int adb = row_max(max((int)(int16_t)ab, (int)ab >> 16)) - X;
+            nc += (uint32_t)(maxCol - minCol);
+            best = max(best, adb);
+            // scores of the next anti-diagonal
+#pragma unroll
+            for (int q = NR / 2 - 1; q > 0; --q)
+                R[q] = __builtin_amdgcn_alignbit(R[q], R[q - 1], 24);
+            R[0] = (R[0] << 8) | (uint32_t)nb;
+            nb = dring[(d + 2 - c0) & (DR - 1)];
+            scores();
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                Z[r] = O[r];
+                O[r] = P[r];
+                P[r] = V[r];
+                LD[r] = L[r];
+            }
+            off1 = off2;
+            off2 = off3;
+            off3 = noff3;
+            l1 = l2;
+            l2 = l3;
+            l3 = nl3;
+            const int nmin = min(max(lo, minCol), maxCol + 1);
+            const int nmax = max(min(hi, maxCol - 1) + 1, noff3) + 1;
+            if (masked < INT_MAX)
+                masked = nmin < d + 2 - rows || nmax > cols
+                             ? INT_MAX
+                             : max(masked - 1, 0);
+            minCol = max(nmin, d + 2 - rows);
+            maxCol = min(nmax, cols);
+            const bool up = state == kRun && c0 + BL < minCol;
+            if (__ballot(up)) {
+                if (up) {
+                    c0 += W;
+                    uint64_t w[NR / 4];
+#pragma unroll
+                    for (int q = 0; q < NR / 4; ++q)
+                        w[q] = *(const uint64_t *)(qring + ((c0 + 8 * q) &
+                                                            (QR - 1)));
+                    set_q(w);
+                }
+            }
+            state = ovf && state == kRun ? kOut : state;
+            fin = state != kDone && (state != kRun || minCol >= maxCol);
+            any = __ballot(fin);
         }
-        fresh = false;
-        cw_prev = cw;
-        nc += (uint32_t)(maxCol0 - minCol);
-        adbest = row_max(adbest);
-        best = adbest > best ? adbest : best;
-        lo = row_min(lo);
-        hi = row_max(hi);
-        int nmin = lo == INT_MAX ? maxCol0 + 1 : lo;
-        int nmax = hi == INT_MIN ? off3 : hi;
-        ++nmax;
-        if (nmin < d + 2 - rows)
-            nmin = d + 2 - rows;
-        if (nmax > cols)
-            nmax = cols;
-        minCol = nmin;
-        maxCol = nmax;
-        const bool ended = run && minCol >= maxCol;
-        if (__ballot(ended)) {
-            // item_end: the "longest extension" end point
+        if (!any)
+            continue;
+
+        // ---- finish rows whose band emptied (or that never started): the
+        // "longest extension" end point, from the last computed column of the
+        // last anti-diagonal, then the end of d-1, else the best of d-2
+        {
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                *(u32a *)(dmp + j * BL + 2 * r) = P[r];
+                *(u32a *)(dmp + W + j * BL + 2 * r) = O[r];
+                *(u32a *)(dmp + 2 * W + j * BL + 2 * r) = Z[r];
+            }
+            any = __ballot(fin);
             int lcol = l3 + off3 - 2;
             int lrow = d - lcol;
-            int32_t ls = at(A3, lcol);
-            const int32_t v2 = at(A2, l2 + off2 - 2);
-            const int32_t v3 = at(A2, l2 + off2 - 3);
+            int ls = dmp[lcol & (W - 1)];
+            const int c2a = l2 + off2 - 2, c2b = l2 + off2 - 3;
+            const int v2a = dmp[W + (c2a & (W - 1))];
+            const int v2b = dmp[W + (c2b & (W - 1))];
             if (ls == kUndef) {
-                if (v2 != kUndef) {
-                    lcol = l2 + off2 - 2;
+                if (v2a != kUndef) {
+                    lcol = c2a;
                     lrow = d - 1 - lcol;
-                    ls = v2;
-                } else if (l2 > 2 && v3 != kUndef) {
-                    lcol = l2 + off2 - 3;
+                    ls = v2a;
+                } else if (l2 > 2 && v2b != kUndef) {
+                    lcol = c2b;
                     lrow = d - 1 - lcol;
-                    ls = v3;
+                    ls = v2b;
                 }
             }
-            // the first maximum above kUndef of anti-diagonal d - 2: the
-            // largest value, and among equal values the smallest column
-            int32_t bv = kUndef;
-            int bc = INT_MAX;
-#pragma unroll
-            for (int c = 0; c < kChunks; ++c) {
-                const int col = base + kW * c + j;
-                if (col >= off1 && col < off1 + l1 && A1[c] > bv) {
-                    bv = A1[c];
-                    bc = col;
+            // first maximum of anti-diagonal d-2 over columns [off1, off1+l1)
+            int m1 = INT_MIN, cm = INT_MAX;
+            for (int x = j; x < W; x += 16) {
+                const int col = off1 + x;
+                const int v = x < l1 ? (int)dmp[2 * W + (col & (W - 1))] : INT_MIN;
+                if (v > m1) {
+                    m1 = v;
+                    cm = col;
                 }
             }
-            // row reduction of (value, column)
-            int32_t ov = ror<1>(bv), oc = ror<1>(bc);
-            if (ov > bv || (ov == bv && oc < bc)) {
-                bv = ov;
-                bc = oc;
-            }
-            ov = ror<2>(bv);
-            oc = ror<2>(bc);
-            if (ov > bv || (ov == bv && oc < bc)) {
-                bv = ov;
-                bc = oc;
-            }
-            ov = ror<4>(bv);
-            oc = ror<4>(bc);
-            if (ov > bv || (ov == bv && oc < bc)) {
-                bv = ov;
-                bc = oc;
-            }
-            ov = ror<8>(bv);
-            oc = ror<8>(bc);
-            if (ov > bv || (ov == bv && oc < bc)) {
-                bv = ov;
-                bc = oc;
-            }
-            if (ls == kUndef && bv > kUndef) {
-                ls = bv;
-                lcol = bc;
+            const int mm = row_max(m1);
+            cm = row_min(m1 == mm ? cm : INT_MAX);
+            if (ls == kUndef && l1 > 0 && mm > kUndef) {
+                ls = mm;
+                lcol = cm;
                 lrow = d - 2 - lcol;
             }
-            if (ended && j == 0)
-                wave_write(a, k, ls, lcol, lrow, ls != kUndef, nc, 0);
-        }
-        if (ended) {
-            state = kIdle;
-            run = false;
-        }
-        // move the window up while its first chunk is below the oldest
-        // range the next steps read (A1 of the next step starts at off2)
-        while (run && base + kW <= off2) {
-#pragma unroll
-            for (int c = 0; c < kChunks - 1; ++c) {
-                A1[c] = A1[c + 1];
-                A2[c] = A2[c + 1];
-                A3[c] = A3[c + 1];
-                q[c] = q[c + 1];
-                LOOK[c] = LOOK[c + 1];
+            if (fin && j == 0) {
+                const XdTask T = a.tasks[k >> 1];
+                XdOut PA_GLOBAL &o = glb(a.out)[T.id];
+                const bool upd = state != kEmpty && ls != kUndef;
+                const int beg_h = (int)T.beg_h, beg_v = (int)T.beg_v;
+                const uint16_t fg = state == kOut ? 1 : 0;
+                // (score kUndef of the other kernels where nothing is defined)
+                const int score = state == kEmpty || state == kOut ? 0
+                                  : ls == kUndef ? INT_MIN / 4
+                                                 : ls - X;
+                if (state == kOut) {
+                    const uint32_t pos = atomicAdd(a.ovf_count, 1u);
+                    a.ovf_list[pos] = k;
+                }
+                if (!right) {
+                    o.beg_h = invalid ? 0 : (upd ? beg_h - lrow : beg_h);
+                    o.beg_v = invalid ? 0 : (upd ? beg_v - lcol : beg_v);
+                    o.score_left = score;
+                    o.cells_left = nc;
+                    o.flags_left = fg;
+                } else {
+                    const int end_h = beg_h + a.seed_len;
+                    const int end_v = beg_v + a.seed_len;
+                    o.end_h = invalid ? 0 : (upd ? end_h + lrow : end_h);
+                    o.end_v = invalid ? 0 : (upd ? end_v + lcol : end_v);
+                    o.score_right = score;
+                    o.cells_right = nc;
+                    o.flags_right = fg;
+                }
             }
-            base += kW;
-            fresh = true;
-            const int col = base + kW * (kChunks - 1) + j;
-            A1[kChunks - 1] = A2[kChunks - 1] = A3[kChunks - 1] = kUndef;
-            q[kChunks - 1] = qres(col);
-            LOOK[kChunks - 1] = dres(d + 1 - col);
+            state = fin ? kNeed : state;
         }
-        // scores of the next step from the residues loaded a half ago, and
-        // the residues of the step after, for the chunks the next steps can
-        // reach (the band's top moves up at most one column per step)
-        // (the next step computes chunks up to the reach, the one after at
-        // most one chunk more: its band's top is at most two columns higher)
-        const int reach = wave_max(run ? (maxCol - base) / kW : 0);
-        cw_next = min(kChunks - 1, reach);
-        const int pw = min(kChunks - 1, reach);
-        if (run) {
-#pragma unroll
-            for (int c = 0; c < kChunks; ++c) {
-                if (c > pw + 1)
-                    break;
-                const int col = base + kW * c + j;
-                if (c <= pw)
-                    sc[c] = mat[q[c] * 32 + LOOK[c]];
-                LOAD[c] = dres(d + 2 - col);
-            }
-        }
-    };
-
-    for (;;) {
-        half(B0, B1);
-        if (!__ballot(state != kDone))
-            break;
-        half(B1, B0);
-        if (!__ballot(state != kDone))
-            break;
     }
 }
 
@@ -498,10 +566,10 @@ hipError_t launch_xdrop_wave(const XdTask *tasks, const uint32_t *list,
     WaveArgs a{tasks, list, count, queue, mat, gap, xdrop, seed_len,
                out, ovf_list, ovf_count};
     if (wide)
-        hipLaunchKernelGGL(k_xdrop_band<kWideChunks>, dim3(grid), dim3(64), 0,
+        hipLaunchKernelGGL(k_xdrop_band<kWideRegs>, dim3(grid), dim3(64), 0,
                            s, a);
     else
-        hipLaunchKernelGGL(k_xdrop_band<kBandChunks>, dim3(grid), dim3(64), 0,
+        hipLaunchKernelGGL(k_xdrop_band<kBandRegs>, dim3(grid), dim3(64), 0,
                            s, a);
     return hipGetLastError();
 }
@@ -513,10 +581,10 @@ int xdrop_wave_occupancy(int wide)
         int n = 0;
         if (wide)
             hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &n, k_xdrop_band<kWideChunks>, 64, 0);
+                &n, k_xdrop_band<kWideRegs>, 64, 0);
         else
             hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &n, k_xdrop_band<kBandChunks>, 64, 0);
+                &n, k_xdrop_band<kBandRegs>, 64, 0);
         cache[wide ? 1 : 0] = n > 0 ? n : 1;
     }
     return cache[wide ? 1 : 0];

@@ -807,9 +807,16 @@ int run_xdrop(pa_ctx *c, const pa_pair *d_pairs, uint64_t n, hipStream_t s)
     const bool thin = c->cfg.xdrop / -c->cfg.xdrop_gap <= 5;
     const bool small16 = thin && !c->tune.xd_coop && ni <= kXdSmall;
     const bool two = thin && !c->tune.xd_coop && !small16;
+    // Wider bands outgrow 16 columns in most items: the band kernels take all
+    // of them, those that may extend far first (60,001 pairs, X = 49, gap -2:
+    // per-lane pass 0.87 ms and 5.5 ms for its overflow, unsorted; 4.7 ms for
+    // all).
+    const bool all_band = !thin && !c->tune.xd_coop && c->tune.xd_wave == 1 &&
+                      c->cfg.xdrop <= 30000;
     uint32_t *const order = lng + ni;
-    if (two)
-        HIPCHK(c, sort_reach(P<XdTask>(c->xdt), nt, c->cfg.seed_len, kXdLong,
+    if (two || all_band)
+        HIPCHK(c, sort_reach(P<XdTask>(c->xdt), nt, c->cfg.seed_len,
+                             all_band ? UINT32_MAX : kXdLong,
                              ctr + C_HIST, ctr + C_FILL, order,
                              ctr + C_XDN, lng, ctr + C_XDLONG, s));
     auto coop = [&](const uint32_t *list, uint32_t *count, uint32_t *queue,
@@ -827,7 +834,7 @@ int run_xdrop(pa_ctx *c, const pa_pair *d_pairs, uint64_t n, hipStream_t s)
         c->stats.launches++;
         return PA_OK;
     };
-    {
+    if (!all_band) {
         Scope t(c, 1, s);
         const int grid = xd_grid(c, ni);
         if (small16) {
@@ -875,6 +882,11 @@ int run_xdrop(pa_ctx *c, const pa_pair *d_pairs, uint64_t n, hipStream_t s)
     // list the pass before last consumed (`lng` is free once the per-lane
     // kernel is done).
     uint32_t *last = ovf, *last_n = ctr + C_XDOVF, *last_q = ctr + C_XDOVFQ;
+    if (all_band) {
+        last = order;
+        last_n = ctr + C_XDN;
+        last_q = ctr + C_XDQ;
+    }
     // one band pass: items of `last` in, overflow to `to`
     auto band = [&](int wide, uint32_t *to, uint32_t *to_n,
                     uint32_t *to_q) -> int {
