@@ -81,6 +81,12 @@ def rocprof_name(kernel):
     mode = kernel[len("k_dp<"):].split(".")[0]
     if mode in linear:
         return linear[mode]
+    m = re.match(r"k_dp<(sw|swt|nwt)\.all\.r8\.(i16|i32)>", kernel)
+    if m:
+        return "void pa::k_dp_all<%s, %s>" % (
+            {"sw": "true, false", "swt": "true, true",
+             "nwt": "false, true"}[m.group(1)],
+            "true" if m.group(2) == "i16" else "false")
     m = re.match(r"k_dp<(sw|swt|nwt)\.c\d\.l(\d+)r(\d+)\.(i16|i32)>", kernel)
     if not m:
         return None

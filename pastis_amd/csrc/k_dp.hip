@@ -345,9 +345,7 @@ template <int L> __device__ inline uint64_t group_max_u64(uint64_t v)
 // the LDS of byte profiles, and are compiled for three waves per SIMD, so
 // that twelve one-wave workgroups fit a CU.
 template <int R, int L, bool LOCAL, bool TRACE, bool I16>
-__global__ __launch_bounds__(64)
-PA_WAVES_PER_EU(rows_nib(R) && I16 ? 3 : 1)
-void k_dp(DpArgs a)
+__device__ __forceinline__ void dp_run(const DpArgs &a, uint32_t *prof32)
 {
     typedef Ops<I16> O;
     typedef typename O::V V;
@@ -364,7 +362,6 @@ void k_dp(DpArgs a)
     constexpr int RB = L == 64 ? 64 : 4 * L;
     constexpr int SH = TRACE ? 2 : 0;
     constexpr int NEG = TRACE ? O::kNegTraced : O::kNeg;
-    HIP_DYNAMIC_SHARED(uint32_t, prof32)
     const int lane = threadIdx.x;
     const int gl = lane % L;     // lane within the task
     const int grp = lane / L;    // task slot of the wave
@@ -382,6 +379,8 @@ void k_dp(DpArgs a)
     // below every real cell) and tag every diagonal 2.
     const int nbase = TRACE ? 4 * a.nib_min + 2 : a.nib_min;
     const uint32_t count = *a.count;
+    if (count == 0)   // no claim: 2,048 waves' atomics on one word take 25 us
+        return;
     const int open = a.gap_open * (1 << SH);
     const int ext = a.gap_ext * (1 << SH);
     const int gmax = open > ext ? open : ext;
@@ -398,7 +397,10 @@ void k_dp(DpArgs a)
 
     // tasks claimed by this wave and not yet started: [cbase, cend)
     uint32_t cbase = 0, cend = 0;
-    const uint32_t chunk = a.chunk;
+    // Several rounds per atomic only where every wave gets some: 20,000 pairs
+    // at 32 tasks a claim left 190 of 3,072 waves with all of a class's work.
+    const uint32_t chunk =
+        count / (G * 4u) >= a.chunk * gridDim.x ? a.chunk : 1u;
     for (;;) {
         // One queue atomic claims `chunk` tasks.  Every lane takes part in
         // the atomic (only lane 0 adds): a lane-0-only branch ahead of the
@@ -860,6 +862,8 @@ void k_dp(DpArgs a)
                 if (valid && sc >= lim && gl == 0) {
                     const uint32_t pos = atomicAdd(a.sat_count, 1u);
                     a.sat_list[pos] = tid;
+                    a.tflags[tid] |= 1;
+                    atomicAdd(a.reruns, 1ull);
                 }
             }
         } else {
@@ -878,6 +882,32 @@ void k_dp(DpArgs a)
         if (valid)
             a.out[tid] = o;
     }
+}
+
+template <int R, int L, bool LOCAL, bool TRACE, bool I16>
+__global__ __launch_bounds__(64)
+PA_WAVES_PER_EU(rows_nib(R) && I16 ? 3 : 1)
+void k_dp(DpArgs a)
+{
+    HIP_DYNAMIC_SHARED(uint32_t, prof32)
+    dp_run<R, L, LOCAL, TRACE, I16>(a, prof32);
+}
+
+// All classes in their default shapes: a wave that finds a class's queue empty
+// goes on with the next, so that no class ends with the chip waiting for its
+// longest tasks.  In launches of their own each of the four took about as long
+// as one task of 3,000 columns: 20,003 local pairs of log-normal lengths to
+// 3,000 5.7 -> 1.5 ms, 120,002 global infixes 5.2 -> 4.2 ms.
+template <bool LOCAL, bool TRACE, bool I16>
+__global__ __launch_bounds__(64)
+PA_WAVES_PER_EU(I16 ? 3 : 1)
+void k_dp_all(DpAllArgs a)
+{
+    HIP_DYNAMIC_SHARED(uint32_t, prof32)
+    dp_run<8, 64, LOCAL, TRACE, I16>(a.cls[3], prof32);
+    dp_run<8, 32, LOCAL, TRACE, I16>(a.cls[2], prof32);
+    dp_run<8, 16, LOCAL, TRACE, I16>(a.cls[1], prof32);
+    dp_run<8, 8, LOCAL, TRACE, I16>(a.cls[0], prof32);
 }
 
 }  // namespace
@@ -929,16 +959,12 @@ struct ResWin {
 };
 
 template <int R, int L, bool LOCAL, bool STAGE>
-__global__ __launch_bounds__(kTbThreads) void k_traceback(TbArgs a)
+__device__ __forceinline__ void tb_run(const TbArgs &a, uint32_t tid,
+                                       uint32_t *stage)
 {
     constexpr int RUNW = 2 * R;   // 32-bit words of one lane run (8R bytes)
     // one run per thread; the odd stride spreads threads over the banks
-    __shared__ uint32_t stage[STAGE ? kTbThreads * (RUNW + 1) : 1];
     uint32_t *run = stage + (STAGE ? threadIdx.x * (RUNW + 1) : 0);
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= *a.count)
-        return;
-    const uint32_t tid = glb(a.list)[k];
     const DpTask T = a.tasks[tid];
     DpOut o = a.out[tid];
     const uint8_t PA_GLOBAL *qs = glb_addr<const uint8_t>(T.q_off);
@@ -1079,6 +1105,45 @@ __global__ __launch_bounds__(kTbThreads) void k_traceback(TbArgs a)
     a.out[tid] = o;
 }
 
+template <int R, int L, bool LOCAL, bool STAGE>
+__global__ __launch_bounds__(kTbThreads) void k_traceback(TbArgs a)
+{
+    __shared__ uint32_t stage[STAGE ? kTbThreads * (2 * R + 1) : 1];
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < *a.count)
+        tb_run<R, L, LOCAL, STAGE>(a, glb(a.list)[k], stage);
+}
+
+// The walks of all bins in the default shapes, the longest class first: they
+// are chains of dependent loads, so the launch takes as long as its longest
+// walk (the same batches: 1.2 -> 1.0 and 1.9 -> 1.2 ms, with the last class on
+// a second stream before).
+template <bool LOCAL, bool STAGE>
+__global__ __launch_bounds__(kTbThreads) void k_traceback_all(TbAllArgs a)
+{
+    __shared__ uint32_t stage[STAGE ? kTbThreads * 17 : 1];
+    uint32_t blk = blockIdx.x;
+    for (int i = 0; i < a.bins; ++i) {
+        const uint32_t n = *a.count[i];
+        const uint32_t nb = (n + kTbThreads - 1) / kTbThreads;
+        if (blk >= nb) {
+            blk -= nb;
+            continue;
+        }
+        const uint32_t k = blk * kTbThreads + threadIdx.x;
+        if (k >= n)
+            return;
+        const uint32_t tid = glb(a.list[i])[k];
+        switch (a.bins == 8 ? i / 2 : i) {
+        case 0: tb_run<8, 64, LOCAL, STAGE>(a.tb, tid, stage); break;
+        case 1: tb_run<8, 32, LOCAL, STAGE>(a.tb, tid, stage); break;
+        case 2: tb_run<8, 16, LOCAL, STAGE>(a.tb, tid, stage); break;
+        default: tb_run<8, 8, LOCAL, STAGE>(a.tb, tid, stage); break;
+        }
+        return;
+    }
+}
+
 template <int R, int L, bool LC, bool T, bool I>
 hipError_t launch_one(const DpArgs &a, int grid, hipStream_t s)
 {
@@ -1148,7 +1213,50 @@ hipError_t launch_traceback_c(const TbArgs &a, bool stage, int grid,
     return hipGetLastError();
 }
 
+// profiles of one wave in the default shapes (R = 8)
+constexpr size_t kAllLds = (size_t)kProfChars * (rows_nib(8) ? 64 : 128) * 8;
+
+template <bool LC, bool T, bool I>
+hipError_t launch_all(const DpAllArgs &a, int grid, hipStream_t s)
+{
+    hipLaunchKernelGGL((k_dp_all<LC, T, I>), dim3(grid), dim3(64), kAllLds, s,
+                       a);
+    return hipGetLastError();
+}
+
 }  // namespace
+
+hipError_t launch_dp_all(const DpAllArgs &a, bool local, bool trace, bool i16,
+                         int grid, hipStream_t s)
+{
+    if (local && trace)
+        return i16 ? launch_all<true, true, true>(a, grid, s)
+                   : launch_all<true, true, false>(a, grid, s);
+    if (local)
+        return i16 ? launch_all<true, false, true>(a, grid, s)
+                   : launch_all<true, false, false>(a, grid, s);
+    return i16 ? launch_all<false, true, true>(a, grid, s)
+               : launch_all<false, true, false>(a, grid, s);
+}
+
+hipError_t launch_traceback_all(const TbAllArgs &a, bool stage, uint32_t ntasks,
+                                hipStream_t s)
+{
+    const dim3 g((ntasks + kTbThreads - 1) / kTbThreads + (uint32_t)a.bins),
+        b(kTbThreads);
+    if (a.tb.local) {
+        if (stage)
+            hipLaunchKernelGGL((k_traceback_all<true, true>), g, b, 0, s, a);
+        else
+            hipLaunchKernelGGL((k_traceback_all<true, false>), g, b, 0, s, a);
+    } else {
+        if (stage)
+            hipLaunchKernelGGL((k_traceback_all<false, true>), g, b, 0, s, a);
+        else
+            hipLaunchKernelGGL((k_traceback_all<false, false>), g, b, 0, s, a);
+    }
+    return hipGetLastError();
+}
 
 hipError_t launch_dp(int shape, bool local, bool trace, bool i16,
                      const DpArgs &a, int grid, hipStream_t s)

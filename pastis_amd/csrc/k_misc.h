@@ -17,9 +17,6 @@ constexpr int kBuckets = 64;
 constexpr int kMaxBins = kLinClasses > kBins ? kLinClasses : kBins;
 
 hipError_t fill_u32(uint32_t *p, uint32_t v, uint32_t n, hipStream_t s);
-// *dst += *src (one thread; a device-side counter)
-hipError_t accumulate(const uint32_t *src, unsigned long long *dst,
-                      hipStream_t s);
 // Codes (at codes + kSeqPad, sentinels around them) and k-mer letters (in
 // place) of the total bytes at raw; both buffers hold 64 bytes more.
 hipError_t encode_set(uint8_t *raw, uint8_t *codes, uint64_t total,
@@ -73,9 +70,6 @@ hipError_t empty_out(const DpTask *tasks, uint32_t a, uint32_t b, int local,
 hipError_t trace_chunks(const uint64_t *toffs, uint32_t n, uint64_t cap,
                         int nchunks, uint32_t *ranges, uint64_t *bases,
                         uint32_t *err, hipStream_t s);
-hipError_t mark_flags(const uint32_t *list, const uint32_t *count,
-                      uint32_t max_n, uint8_t *flags, uint8_t bit,
-                      hipStream_t s);
 // err (optional, device): when nonzero the batch's trace did not fit the
 // captured chunks of a graph, and every result is PA_FLAG_NOTRACE
 hipError_t finalize_sw(const DpTask *tasks, const DpOut *dp,

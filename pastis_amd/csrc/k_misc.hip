@@ -32,12 +32,6 @@ inline int stride_blocks(uint64_t n)
     return (int)(b < 2048 ? (b > 0 ? b : 1) : 2048);
 }
 
-__global__ void k_accumulate(const uint32_t *src, unsigned long long *dst)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0 && *src)
-        atomicAdd(dst, (unsigned long long)*src);
-}
-
 __global__ void k_fill_u32(uint32_t *p, uint32_t v, uint32_t n)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -464,14 +458,6 @@ __global__ void k_empty_out(const DpTask *__restrict__ tasks, uint32_t a,
     out[i] = o;
 }
 
-__global__ void k_mark(const uint32_t *list, const uint32_t *count,
-                       uint8_t *flags, uint8_t bit)
-{
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < *count)
-        flags[list[k]] |= bit;
-}
-
 __device__ inline float identity_of(uint32_t matches, uint32_t cols)
 {
     return (float)(100.0 * (double)(float)matches / (double)(float)cols);
@@ -624,13 +610,6 @@ hipError_t fill_u32(uint32_t *p, uint32_t v, uint32_t n, hipStream_t s)
     if (!n)
         return hipSuccess;
     hipLaunchKernelGGL(k_fill_u32, dim3(blocks(n, 256)), dim3(256), 0, s, p, v, n);
-    return hipGetLastError();
-}
-
-hipError_t accumulate(const uint32_t *src, unsigned long long *dst,
-                      hipStream_t s)
-{
-    hipLaunchKernelGGL(k_accumulate, dim3(1), dim3(64), 0, s, src, dst);
     return hipGetLastError();
 }
 
@@ -804,17 +783,6 @@ hipError_t trace_chunks(const uint64_t *toffs, uint32_t n, uint64_t cap,
 {
     hipLaunchKernelGGL(k_trace_chunks, dim3(1), dim3(64), 0, s, toffs, n, cap,
                        nchunks, ranges, bases, err);
-    return hipGetLastError();
-}
-
-hipError_t mark_flags(const uint32_t *list, const uint32_t *count,
-                      uint32_t max_n, uint8_t *flags, uint8_t bit,
-                      hipStream_t s)
-{
-    if (!max_n)
-        return hipSuccess;
-    hipLaunchKernelGGL(k_mark, dim3(blocks(max_n, 256)), dim3(256), 0, s, list,
-                       count, flags, bit);
     return hipGetLastError();
 }
 

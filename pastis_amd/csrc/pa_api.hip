@@ -178,6 +178,15 @@ void resolve_timers(pa_ctx *c)
             c->klin[t.kind - 5].ms += ms;
             c->klin[t.kind - 5].launches++;
             break;
+        case 8:
+        case 9:
+        case 10:
+        case 11:
+        case 12:
+        case 13:
+            c->kall[(t.kind - 8) / 3][(t.kind - 8) % 3].ms += ms;
+            c->kall[(t.kind - 8) / 3][(t.kind - 8) % 3].launches++;
+            break;
         default: c->stats.ms_total += ms; break;
         }
         c->free_events.push_back(t.a);
@@ -560,6 +569,8 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
         args.bnd_stride = 2u * (c->max_clen + 2);
         args.gap_open = c->cfg.gap_open;
         args.gap_ext = c->cfg.gap_ext;
+        args.tflags = P<uint8_t>(c->tflags);
+        args.reruns = (unsigned long long *)P<uint64_t>(c->cells) + 2;
         TbArgs tb{};
         tb.codes = nullptr;
         tb.tasks = P<DpTask>(c->tasks);
@@ -588,6 +599,64 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
             }
             return PA_OK;
         };
+        // The default shapes: all classes in one launch, and so their walks.
+        // (Walks beside the DP need the classes one by one.)
+        if (!split && !beside &&
+            std::equal(c->shapes.shape, c->shapes.shape + kClasses,
+                       kDefaultShapes.shape)) {
+            auto all = [&](bool i16, const uint32_t *list0, uint32_t *count0,
+                           uint32_t *queue0, int step) -> int {
+                DpAllArgs aa;
+                int grid = INT_MAX;
+                for (int rcl = 0; rcl < kClasses; ++rcl) {
+                    DpArgs &x = aa.cls[rcl];
+                    x = args;
+                    x.chunk = rcl <= 2 ? 4u : 1u;
+                    x.pmat = rows_nib(shape_rows(c->shapes.shape[rcl]))
+                                 ? pmat_nib
+                                 : pmat_byte;
+                    x.list = list0 + (size_t)(step * rcl) * nt;
+                    x.count = count0 + step * rcl;
+                    x.queue = queue0 + step * rcl;
+                    x.sat_list = sat + (size_t)rcl * nt;
+                    x.sat_count = ctr + C_SAT + rcl;
+                    grid = std::min(grid, dp_grid(c, b - a, rcl, local, trace,
+                                                  i16));
+                }
+                Scope k(c, (i16 ? 8 : 11) + dmode, s);
+                HIPCHK(c, launch_dp_all(aa, local, trace, i16, grid, s));
+                c->stats.launches++;
+                return PA_OK;
+            };
+            {
+                Scope sc(c, kind, s);
+                // global tasks that may leave the int16 range
+                if (nw == 2 && (rc = all(false, lists + nt, ctr + C_BIN + 1,
+                                         ctr + C_BINQ + 1, 2)))
+                    return rc;
+                if ((rc = all(true, lists, ctr + C_BIN, ctr + C_BINQ, 2)))
+                    return rc;
+                // local tasks whose int16 DP saturated
+                if (local && (rc = all(false, sat, ctr + C_SAT, ctr + C_SATQ,
+                                       1)))
+                    return rc;
+            }
+            if (trace) {
+                TbAllArgs ta{};
+                ta.tb = tb;
+                for (int cls = kClasses - 1; cls >= 0; --cls)
+                    for (int w = 0; w < nw; ++w) {
+                        const int bin = 2 * cls + w;
+                        ta.list[ta.bins] = lists + (size_t)bin * nt;
+                        ta.count[ta.bins++] = ctr + C_BIN + bin;
+                    }
+                Scope sc(c, 3, s);
+                HIPCHK(c, launch_traceback_all(ta, c->tune.tb_stage != 0,
+                                               b - a, s));
+                c->stats.launches++;
+            }
+            continue;
+        }
         {
             Scope sc(c, kind, s);
             // DP of class rcl's bin w (0: int16, 1: int32)
@@ -641,14 +710,7 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
                                                     false),
                                             s));
                     }
-                    HIPCHK(c, mark_flags(args.list, args.count, b - a,
-                                         P<uint8_t>(c->tflags), 1, s));
-                    // tasks re-run in int32 (pa_stats.rerun_pairs)
-                    HIPCHK(c, accumulate(args.count,
-                                         (unsigned long long *)P<uint64_t>(
-                                             c->cells) + 2,
-                                         s));
-                    c->stats.launches += 3;
+                    c->stats.launches++;
                 }
                 if (split) {
                     // this class's trace is complete: it is traced back on
@@ -1920,6 +1982,9 @@ int pa_reset_stats(pa_ctx *c)
         HIPCHK(c, hipMemset(c->cells.p, 0, 32));
     for (auto &k : c->klin)
         k = pa_ctx::KStat{};
+    for (auto &m : c->kall)
+        for (auto &k : m)
+            k = pa_ctx::KStat{};
     HIPCHK(c, hipMemset(c->bincells.p, 0,
                         2 * kModes * kBins * sizeof(uint64_t)));
     return PA_OK;
@@ -1979,6 +2044,24 @@ int pa_get_kernel_stats(pa_ctx *c, pa_kernel_stat *out, int cap, int *n)
         }
         ++k;
     }
+    for (int w = 0; w < 2; ++w)
+        for (int m = 0; m < 3; ++m) {
+            if (!c->kall[w][m].launches)
+                continue;
+            if (k < cap) {
+                // (the int32 re-runs of saturated local tasks count as the
+                // int16 cells they repeat)
+                pa_kernel_stat &o = out[k];
+                std::memset(&o, 0, sizeof(o));
+                std::snprintf(o.name, sizeof(o.name), "%s.all.r8.%s", mname[m],
+                              w ? "i32" : "i16");
+                o.launches = c->kall[w][m].launches;
+                o.ms = c->kall[w][m].ms;
+                for (int b = w; b < kBins; b += 2)
+                    o.cells += cells[m * kBins + b];
+            }
+            ++k;
+        }
     *n = k;
     return PA_OK;
 }

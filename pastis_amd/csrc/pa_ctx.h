@@ -97,6 +97,7 @@ struct pa_ctx {
         double ms = 0;
     } kstat[3][pa::kBins + pa::kClasses];   // DP mode x (bins, int32 re-runs)
     KStat klin[3];   // linear-gap kernels, all classes, by DP mode
+    KStat kall[2][3];   // affine, all classes: int16 / int32, by DP mode
     std::vector<Timer> pending;
     std::vector<hipEvent_t> free_events;
     pa_stats stats{};

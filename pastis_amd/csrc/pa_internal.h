@@ -126,8 +126,10 @@ struct DpArgs {
     uint32_t bnd_stride;       // int32 entries per workgroup
     uint32_t *sat_list;        // tasks that saturated (int16 kernels)
     uint32_t *sat_count;
+    uint8_t *tflags;           // and their flag, 1
+    unsigned long long *reruns;// and their number (pa_stats.rerun_pairs)
     int32_t gap_open, gap_ext;
-    uint32_t chunk;            // tasks claimed per queue atomic (>= 1)
+    uint32_t chunk;            // most tasks claimed per queue atomic (>= 1)
     int32_t nib_min;           // 4-bit profiles: the score of nibble 0
 };
 
@@ -142,6 +144,17 @@ struct TbArgs {
     const uint64_t *trace_base;   // as DpArgs::trace_base
     DpOut *out;
     int local;
+};
+
+// The four row classes in the default shapes, in one launch.
+struct DpAllArgs {
+    DpArgs cls[4];
+};
+struct TbAllArgs {
+    TbArgs tb;                 // without list and count
+    const uint32_t *list[8];   // bins, the longest class first
+    const uint32_t *count[8];
+    int bins;                  // 4 (no int32 bins) or 8
 };
 
 // DP kernel shapes: L lanes per task (G = 64 / L tasks per wave, one per
@@ -406,6 +419,10 @@ hipError_t launch_dp(int shape, bool local, bool trace, bool i16,
 // Traceback of tasks traced by the DP kernels of one shape; stage: copy each
 // lane run (8R bytes) the walk enters into LDS with wide loads instead of
 // loading one byte per step.
+hipError_t launch_dp_all(const DpAllArgs &a, bool local, bool trace, bool i16,
+                         int grid, hipStream_t s);
+hipError_t launch_traceback_all(const TbAllArgs &a, bool stage, uint32_t ntasks,
+                                hipStream_t s);
 hipError_t launch_traceback(const TbArgs &a, int shape, bool stage, int grid,
                             hipStream_t s);
 // X-drop with one 16-lane row of a wave per work item (k_xdrop_coop.hip);

@@ -46,7 +46,7 @@ constexpr uint64_t kValidate = 1u << 23;
 constexpr int kReps = 2;
 
 struct Times {
-    double dp = 0, cls[kClasses] = {0, 0, 0, 0}, trace = 0, xdrop = 0;
+    double dp = 0, trace = 0, xdrop = 0;
     double wall = 0;   // host time of the whole call, synchronised
 };
 
@@ -79,8 +79,6 @@ public:
             return rc;
         Times b;
         b.dp = b.trace = b.xdrop = b.wall = INFINITY;
-        for (int k = 0; k < kClasses; ++k)
-            b.cls[k] = INFINITY;
         for (int r = 0; r < kReps; ++r) {
             if ((rc = pa_reset_stats(c_)))
                 return rc;
@@ -97,13 +95,6 @@ public:
             b.dp = std::min(b.dp, st.ms_sw + st.ms_nw);
             b.trace = std::min(b.trace, st.ms_trace);
             b.xdrop = std::min(b.xdrop, st.ms_xdrop);
-            for (int k = 0; k < kClasses; ++k) {
-                double ms = 0;
-                for (int m = 0; m < 3; ++m)
-                    ms += c_->kstat[m][2 * k].ms + c_->kstat[m][2 * k + 1].ms +
-                          c_->kstat[m][kBins + k].ms;
-                b.cls[k] = std::min(b.cls[k], ms);
-            }
         }
         *best = b;
         ++runs_;
@@ -194,7 +185,8 @@ int search(Tuner &tu, bool xdrop, bool lin, pa_tuning &t)
         }
     }
 
-    // 3. the kernel shape of each class
+    // 3. the kernel shape of each class (by all classes' DP: the default
+    // shapes run in one launch, others class by class)
     for (int k = 0; k < kClasses; ++k)
         for (int sh = 0; sh < kShapes; ++sh) {
             if (lin || sh == t.dp_shape[k])
@@ -204,8 +196,7 @@ int search(Tuner &tu, bool xdrop, bool lin, pa_tuning &t)
             Times tm;
             if ((rc = tu.measure(cand, &tm)))
                 return rc;
-            if (better(tm.cls[k] + tm.trace, cur.cls[k] + cur.trace, tm,
-                       cur)) {
+            if (better(tm.dp + tm.trace, cur.dp + cur.trace, tm, cur)) {
                 t = cand;
                 cur = tm;
             }
