@@ -922,7 +922,6 @@ void k_dp_all(DpAllArgs a)
 namespace pa {
 namespace {
 
-
 // R and L are fixed per launch (one launch per DP class, whose kernel
 // shape wrote the trace), so the layout arithmetic divides by constants.
 // Global traces of byte-profile kernels mark a diagonal step between equal
@@ -930,13 +929,13 @@ namespace {
 // no residue loads; those of 4-bit-profile kernels (rows_nib) tag every
 // diagonal 2 and the walk compares the residues, as local walks do.
 //
-// STAGE: the walk reads the trace one lane run at a time: the kTraceSeg
-// records of one lane in one segment (8R contiguous bytes, 8R-aligned) are
-// loaded with wide loads into the thread's slot in LDS when the walk enters
-// them, and the codes are read from there.  Diagonal and horizontal moves
-// step back one record inside the run, vertical moves stay in the record,
-// so a run serves several steps.  Without STAGE each step loads its byte
-// from global memory.
+// STAGE: the walk reads the trace through windows of two lane runs (the
+// kTraceSeg records of one lane in one segment, 8R contiguous bytes, 8R-aligned)
+// that are copied into the thread's slot in LDS with wide loads.  All walks of
+// a wave load their windows together: one run each, loaded when its walk
+// entered it, left some walk of the wave waiting in nearly every step (20,003
+// local walks to 3,000 residues 1.02 -> 0.73 ms, 120,002 global ones 1.19 ->
+// 0.70 ms).  Without STAGE each step loads its byte from global memory.
 
 // Residues of one sequence as the walk reads them (backwards, mostly one
 // position per diagonal step): the aligned 8-byte word holding the last one
@@ -964,7 +963,7 @@ __device__ __forceinline__ void tb_run(const TbArgs &a, uint32_t tid,
 {
     constexpr int RUNW = 2 * R;   // 32-bit words of one lane run (8R bytes)
     // one run per thread; the odd stride spreads threads over the banks
-    uint32_t *run = stage + (STAGE ? threadIdx.x * (RUNW + 1) : 0);
+    uint32_t *run = stage + (STAGE ? threadIdx.x * (2 * RUNW + 1) : 0);
     const DpTask T = a.tasks[tid];
     DpOut o = a.out[tid];
     const uint8_t PA_GLOBAL *qs = glb_addr<const uint8_t>(T.q_off);
@@ -1012,90 +1011,139 @@ __device__ __forceinline__ void tb_run(const TbArgs &a, uint32_t tid,
             }
         }
     };
-    uint32_t cur_run = 0xffffffffu;   // byte offset of the staged run
-    ResWin qwin{qs}, twin{ts};
     int matches = 0, cols = 0, runs = 0;
     int last = 0;   // 1 diagonal, 2 vertical, 3 horizontal
     int state = 0;  // 0 H, 1 E (horizontal), 2 F (vertical)
-    if (LOCAL && o.score <= 0) {
-        i = j = 0;
-    } else {
+    bool more = i > 0 && j > 0 && !(LOCAL && o.score <= 0);
+    // One step on a cell's code; same: the residues at (i, j) are equal.
+    // Returns what moved: 1 i, 2 j, 0 neither (a change of state), -1 the
+    // restart of a local alignment.
+    auto step = [&](int c, bool same) -> int {
+        if (state == 0) {
+            const int src = c & 3;
+            if (LOCAL && src == 3)
+                return -1;
+            if (src < 2) {
+                state = src == 1 ? 2 : 1;
+                return 0;
+            }
+            ++cols;
+            matches += LOCAL || rows_nib(R) ? same : src == 3;
+            last = 1;
+            --i;
+            --j;
+            up();
+            return 3;
+        }
+        ++cols;
+        if (state == 1) {
+            runs += last != 3;
+            last = 3;
+            state = (c >> 3) & 1 ? 1 : 0;   // E extended
+            --j;
+            return 2;
+        }
+        runs += last != 2;
+        last = 2;
+        state = (c >> 2) & 1 ? 2 : 0;   // F extended
+        --i;
+        up();
+        return 1;
+    };
+    // record of (step t, lane l); row r, half h of a record sits in byte
+    // 4*(r/4) + 2*(r%2) + h, high nibble when (r/2) is odd
+    if constexpr (!STAGE) {
+        ResWin qwin{qs}, twin{ts};
+        while (more) {
+            const uint32_t t1 = (uint32_t)(j + 2 * l + h) - 1u;
+            const uint32_t byte =
+                glb(trg)[pbase + (t1 / kTraceSeg) * seg_bytes +
+                         (uint32_t)l * RUN + (t1 % kTraceSeg) * R +
+                         4u * (r >> 2) + 2u * (r & 1) + (uint32_t)h];
+            const int c = (int)((r & 2) ? (byte >> 4) : (byte & 15u));
+            const bool diag = state == 0 && (c & 3) >= 2;
+            more = step(c, diag && (LOCAL || rows_nib(R)) &&
+                               qwin.at(i - 1) == twin.at(j - 1)) >= 0 &&
+                   i > 0 && j > 0;
+        }
+    }
+    // Staged: windows of two lane runs (the segment the walk stands in and the
+    // one before) and 16 residues of either sequence, loaded by all walks of
+    // the wave together, then walked until every walk has left its own (as in
+    // the linear-gap walks).
+    if constexpr (STAGE)
+    while (more) {
+        const int seg = (j + 2 * l + h - 1) / (int)kTraceSeg;
+        const uint32_t off =
+            pbase + (uint32_t)seg * seg_bytes + (uint32_t)l * RUN;
+        // generic pointers: vector-struct loads from the global address
+        // space do not compile
+        const uint4 *s1 = (const uint4 *)(trg + off);
+        const uint4 *s0 = (const uint4 *)(trg + (seg ? off - seg_bytes : off));
+        uint4 x[RUNW / 2];
+#pragma unroll
+        for (int q = 0; q < RUNW / 4; ++q) {
+            x[q] = s0[q];
+            x[RUNW / 4 + q] = s1[q];
+        }
+        // residues i - 16 .. i - 1 and j - 16 .. j - 1, the next one on top
+        // (those before a sequence's start lie in the store and are not used)
+        uint64_t q0 = 0, q1 = 0, t0 = 0, t1 = 0;
+        if (LOCAL || rows_nib(R)) {
+            typedef uint64_t __attribute__((aligned(1))) u64u;
+            q0 = *(const u64u PA_GLOBAL *)(qs + i - 16);
+            q1 = *(const u64u PA_GLOBAL *)(qs + i - 8);
+            t0 = *(const u64u PA_GLOBAL *)(ts + j - 16);
+            t1 = *(const u64u PA_GLOBAL *)(ts + j - 8);
+        }
+#pragma unroll
+        for (int q = 0; q < RUNW / 2; ++q) {
+            run[4 * q + 0] = x[q].x;
+            run[4 * q + 1] = x[q].y;
+            run[4 * q + 2] = x[q].z;
+            run[4 * q + 3] = x[q].w;
+        }
+        const int tb = (seg - 1) * (int)kTraceSeg;   // step of the first record
+        const int lw = l, iw = i - 16 > 0 ? i - 16 : 0;
+        const int jw = j - 16 > 0 ? j - 16 : 0;
         for (;;) {
-            if (i == 0 || j == 0) {
-                if (LOCAL)
-                    break;
-                // global boundary: a single gap run to the origin
-                if (i > 0) {
-                    cols += i;
-                    runs += last != 2;
-                    i = 0;
-                } else if (j > 0) {
-                    cols += j;
-                    runs += last != 3;
-                    j = 0;
-                }
+            const int at = j + 2 * l + h - 1 - tb;
+            if (at < 0)
+                break;
+            const uint32_t bi = (uint32_t)at * R + 4u * (r >> 2) +
+                                2u * (r & 1) + (uint32_t)h;
+            const uint32_t byte = (run[bi >> 2] >> (8u * (bi & 3u))) & 0xffu;
+            const int moved = step((int)((r & 2) ? (byte >> 4) : (byte & 15u)),
+                                   (q1 ^ t1) >> 56 == 0);
+            if (moved < 0) {
+                more = false;
                 break;
             }
-            // record of (step t, lane l); row r, half h of a record sits in
-            // byte 4*(r/4) + 2*(r%2) + h, high nibble when (r/2) is odd
-            const uint32_t t1 = (uint32_t)(j + 2 * l + h) - 1u;
-            const uint32_t run_off =
-                pbase + (t1 / kTraceSeg) * seg_bytes + (uint32_t)l * RUN;
-            const uint32_t bi = (t1 % kTraceSeg) * R + 4u * (r >> 2) +
-                                2u * (r & 1) + (uint32_t)h;
-            uint32_t byte;
-            if (STAGE) {
-                if (run_off != cur_run) {
-                    cur_run = run_off;
-                    // generic pointer: vector-struct loads from the global
-                    // address space do not compile
-                    const uint4 *src = (const uint4 *)(trg + run_off);
-#pragma unroll
-                    for (int q = 0; q < RUNW / 4; ++q) {
-                        const uint4 x = src[q];
-                        run[4 * q + 0] = x.x;
-                        run[4 * q + 1] = x.y;
-                        run[4 * q + 2] = x.z;
-                        run[4 * q + 3] = x.w;
-                    }
-                }
-                byte = (run[bi >> 2] >> (8u * (bi & 3u))) & 0xffu;
-            } else {
-                byte = glb(trg)[run_off + bi];
+            if (moved & 1) {
+                q1 = (q1 << 8) | (q0 >> 56);
+                q0 <<= 8;
             }
-            const int c = (int)((r & 2) ? (byte >> 4) : (byte & 15u));
-            if (state == 0) {
-                const int src = c & 3;
-                if (LOCAL && src == 3)
-                    break;  // restart
-                if (src >= 2) {
-                    ++cols;
-                    if (LOCAL || rows_nib(R))
-                        matches += qwin.at(i - 1) == twin.at(j - 1);
-                    else
-                        matches += src == 3;
-                    last = 1;
-                    --i;
-                    up();
-                    --j;
-                } else {
-                    state = src == 1 ? 2 : 1;
-                }
-            } else if (state == 1) {
-                ++cols;
-                runs += last != 3;
-                last = 3;
-                state = (c >> 3) & 1 ? 1 : 0;   // E extended
-                --j;
-            } else {
-                ++cols;
-                runs += last != 2;
-                last = 2;
-                state = (c >> 2) & 1 ? 2 : 0;   // F extended
-                --i;
-                up();
+            if (moved & 2) {
+                t1 = (t1 << 8) | (t0 >> 56);
+                t0 <<= 8;
             }
+            if (i <= iw || j <= jw || l != lw)
+                break;
         }
+        more = more && i > 0 && j > 0;
+    }
+    if (LOCAL) {
+        if (o.score <= 0)
+            i = j = 0;
+    } else if (i > 0) {
+        // border: a single gap run to the origin
+        cols += i;
+        runs += last != 2;
+        i = 0;
+    } else if (j > 0) {
+        cols += j;
+        runs += last != 3;
+        j = 0;
     }
     o.q_beg = i;
     o.t_beg = j;
@@ -1108,7 +1156,7 @@ __device__ __forceinline__ void tb_run(const TbArgs &a, uint32_t tid,
 template <int R, int L, bool LOCAL, bool STAGE>
 __global__ __launch_bounds__(kTbThreads) void k_traceback(TbArgs a)
 {
-    __shared__ uint32_t stage[STAGE ? kTbThreads * (2 * R + 1) : 1];
+    __shared__ uint32_t stage[STAGE ? kTbThreads * (4 * R + 1) : 1];
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k < *a.count)
         tb_run<R, L, LOCAL, STAGE>(a, glb(a.list)[k], stage);
@@ -1117,11 +1165,11 @@ __global__ __launch_bounds__(kTbThreads) void k_traceback(TbArgs a)
 // The walks of all bins in the default shapes, the longest class first: they
 // are chains of dependent loads, so the launch takes as long as its longest
 // walk (the same batches: 1.2 -> 1.0 and 1.9 -> 1.2 ms, with the last class on
-// a second stream before).
+// a second stream before; the windows of tb_run make them 0.73 and 0.70).
 template <bool LOCAL, bool STAGE>
 __global__ __launch_bounds__(kTbThreads) void k_traceback_all(TbAllArgs a)
 {
-    __shared__ uint32_t stage[STAGE ? kTbThreads * 17 : 1];
+    __shared__ uint32_t stage[STAGE ? kTbThreads * 33 : 1];
     uint32_t blk = blockIdx.x;
     for (int i = 0; i < a.bins; ++i) {
         const uint32_t n = *a.count[i];
