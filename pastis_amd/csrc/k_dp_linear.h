@@ -598,7 +598,7 @@ constexpr uint32_t kLinDone = 0xffffffffu;
 // (35,000 x 35,000 residues: 320 ms) while the chip was idle.  Items are
 // claimed in order, a task's passes one after the other, and an item waits
 // only for items claimed before it (its predecessor's columns, the last
-// reader of its boundary slot), so the first unfinished item always runs.
+// owner and reader of its boundary slot), so the first unfinished item always runs.
 template <class P, bool MULTI, bool PIPE>
 __device__ inline void lin_run(const LinArgs &a, uint32_t *prof,
                                const uint32_t PA_GLOBAL *list, uint32_t count,
@@ -684,8 +684,14 @@ __device__ inline void lin_run(const LinArgs &a, uint32_t *prof,
             if (lane == 0)
                 lin_put(prog + k0 % S, lin_progress(k0, cols));
         };
-        if (PIPE && k0 >= S)   // the slot's last reader is done with it
+        if (PIPE && k0 >= S) {
+            // The slot's last owner and its reader are done with it.  (The
+            // reader may be the first pass of another task, which waits for
+            // nobody, so its end does not imply the owner's: an owner still
+            // running would set the progress word back under this item.)
+            wait(k0 - S, kLinDone);
             wait(k0 - S + 1, kLinDone);
+        }
         uint64_t value = 0;
         uint32_t avail = 0;    // columns the pass before has published
 
