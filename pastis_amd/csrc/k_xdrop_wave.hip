@@ -151,9 +151,8 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
         rings[i] = 0;
     __syncthreads();
     const uint32_t n = *a.count;
-    const int X = a.X, gap = max(a.gap, -32000);
+    const int gap = max(a.gap, -32000);
     const uint32_t GAP = splat(gap);
-    const int best_max = 32000 - X;
     uint8_t *const qring = rings + row * (QR + DR);
     uint8_t *const dring = qring + QR;
     int16_t *const dmp = dump + row * 3 * W;
@@ -161,6 +160,7 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
     // row-uniform state of the current item
     int state = kNeed;
     uint32_t k = 0;
+    int X = 0, best_max = 0;
     int cols = 0, rows = 0, d = 0, minCol = 0, maxCol = 0, best = 0;
     int off1 = 0, off2 = 0, off3 = 0, l1 = 0, l2 = 0, l3 = 0;
     bool right = false, invalid = false;
@@ -268,6 +268,13 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
                         db = h + beg_h + a.seed_len - 1;
                         qstep = 1;
                     }
+                    // No cell lies more below the best score than the gaps of
+                    // its anti-diagonal and 31 (the largest matrix score) per
+                    // row or column: a larger X drops nothing either.
+                    X = (int)min((int64_t)a.X,
+                                 31ll * min(cols, rows) + 1 -
+                                     (int64_t)(cols + rows) * gap);
+                    best_max = a.gap < -32000 ? -1 : 32000 - X;
                     d = 1;
                     minCol = 1;
                     maxCol = 2;
