@@ -467,16 +467,17 @@ typedef struct pa_tuning {
                                128, 256, 512 */
     int32_t dp_shape[4];    /* pa_dp_shape of each row class; default
                                L8R8, L16R8, L32R8, L64R8 */
-    int32_t tb_stage;       /* 1 (default): the traceback copies each lane
-                               run of the trace it enters into LDS with wide
-                               loads; 0: one byte load per step */
+    int32_t tb_stage;       /* 1 (default): the traceback copies the lane
+                               runs of the trace it stands in into LDS with
+                               wide loads; 0: one byte load per step */
     int32_t xd_wave;        /* X-drop items whose band outgrows the
                                per-lane kernel's rings continue with 16
                                lanes per item: 1 (default) in a 128-column
                                window, then a 256-column one; 2: the
                                256-column window only; 0: none.  What is
                                left runs with global-memory rings, one lane
-                               per item */
+                               per item.  With 1 (and xd_coop 0), items start
+                               there where X / -gap exceeds 5 */
     int32_t tb_overlap;     /* 1: each class's tracebacks run on a second
                                stream beside the next classes' DP; 2: those
                                of all classes but the last beside the last
