@@ -141,8 +141,10 @@ def roofline(kstats, st, step_ms_total, tuning=None, traffic_key=None):
         # overflow lists, the last ones taking only the items that outgrow
         # the earlier ones' windows
         tn = tuning or {}
-        chain = ["k_xdrop_coop"] if tn.get("xd_coop") else []
-        chain.append("k_xdrop_pl<%d>" % tn.get("xd_ring", 16))
+        # (bands of more than about ten columns start in the band kernels)
+        pl = "k_xdrop_pl<%d>" % tn.get("xd_ring", 16)
+        chain = ["k_xdrop_coop", pl] if tn.get("xd_coop") else \
+            ["(thin bands) k_xdrop_coop beside " + pl]
         chain += {0: [], 1: ["k_xdrop_band<4>", "k_xdrop_band<8>"],
                   2: ["k_xdrop_band<8>"]}[tn.get("xd_wave", 1)]
         chain.append("k_xdrop_pl<0>")
