@@ -599,13 +599,12 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
             }
             return PA_OK;
         };
-        // The default shapes: all classes in one launch, and so their walks.
-        // (Walks beside the DP need the classes one by one, and a workspace of
+        // The default shapes and row edges within a pass: all classes in one
+        // launch, and so their walks.  (Walks beside the DP need the classes one by one, and a workspace of
         // fixed size holds the boundary rows of fewer waves the fewer lanes a
         // task takes: each class then has the grid that fits it.)
         if (!split && !beside && c->slot_cap == 0 &&
-            std::equal(c->shapes.shape, c->shapes.shape + kClasses,
-                       kDefaultShapes.shape)) {
+            dp_one_launch(c->shapes)) {
             auto all = [&](bool i16, const uint32_t *list0, uint32_t *count0,
                            uint32_t *queue0, int step) -> int {
                 DpAllArgs aa;

@@ -146,7 +146,7 @@ struct TbArgs {
     int local;
 };
 
-// The four row classes in the default shapes, in one launch.
+// The four row classes in one launch (dp_one_launch).
 struct DpAllArgs {
     DpArgs cls[4];
 };
@@ -199,9 +199,9 @@ __host__ __device__ constexpr int shape_byte_fallback(int sh)
 // take 2L steps per pass and the last pass rounds the rows up to 2RL); wide
 // ones cost fewer boundary rows, profile builds and loop overhead per cell
 // on long tasks.  The defaults (kDefaultShapes) are
-//   0: qlen <= 128: 16 lanes x 4 rows, 128 rows per pass (one pass);
+//   0: qlen <= 128:  8 lanes x 8 rows, 128 rows per pass (one pass);
 //   1: qlen <= 256: 16 lanes x 8 rows, 256 rows per pass (one pass);
-//   2: qlen <= 512: 64 lanes x 4 rows, 512 rows per pass (one pass);
+//   2: qlen <= 512: 32 lanes x 8 rows, 512 rows per pass (one pass);
 //   3: longer:      64 lanes x 8 rows, 1024 rows per pass.
 struct DpShapes {
     uint32_t edge[3];
@@ -210,6 +210,21 @@ struct DpShapes {
 constexpr DpShapes kDefaultShapes = {{128, 256, 512},
                                      {kShapeL8R8, kShapeL16R8, kShapeL32R8,
                                       kShapeL64R8}};
+
+// The classes may share a launch (DpAllArgs): the default shapes, with one
+// pass for every task below the last class.  A task of several passes keeps
+// its boundary row at workgroup * slots + slot, and the slots per workgroup
+// differ between classes: were there such tasks in two classes, workgroups
+// that are in different classes at the same time would share rows.
+inline bool dp_one_launch(const DpShapes &sh)
+{
+    for (int c = 0; c < 4; ++c)
+        if (sh.shape[c] != kDefaultShapes.shape[c] ||
+            (c < 3 && sh.edge[c] > 2u * (uint32_t)shape_rows(sh.shape[c]) *
+                                       (uint32_t)shape_lanes(sh.shape[c])))
+            return false;
+    return true;
+}
 
 __host__ __device__ inline int dp_class(uint32_t qlen, const DpShapes &sh)
 {

@@ -9,9 +9,14 @@
 //         uint8 codes[offsets[nseq]]; pa_pair pairs[npairs]
 // output: pa_result results[npairs], then (X-drop mode) pa_extent of seed 0
 //         and of seed 1 for every pair, then the uint64 X-drop cell count.
+// EMU_DEV runs the batch through pa_align_dev instead (which takes pairs that
+// the host entry points refuse) and leaves out the extents; EMU_SCORES=<entry>
+// runs pa_sw_scores_<entry> (dev or noalloc) and writes pa_score scores[npairs]
+// instead; EMU_STATS=<file> receives the kernel launches that pa_stats counts.
 // Mode 2 runs the k-mer candidate generation instead (see kmer_mode).
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <vector>
 
 #include "../../include/pastis_hip.h"
@@ -72,6 +77,48 @@ int kmer_mode(const int32_t *h, const std::vector<uint64_t> &offs,
     std::fclose(f);
     pa_device_free(c, d);
     pa_destroy(c);
+    return 0;
+}
+
+int write_stats(pa_ctx *c)
+{
+    const char *path = std::getenv("EMU_STATS");
+    if (!path)
+        return 0;
+    pa_stats st;
+    if (pa_get_stats(c, &st))
+        return 1;
+    FILE *f = std::fopen(path, "w");
+    if (!f)
+        return 2;
+    std::fprintf(f, "%llu\n", (unsigned long long)st.launches);
+    std::fclose(f);
+    return 0;
+}
+
+int scores_run(pa_ctx *c, const std::vector<pa_pair> &pairs, const char *entry,
+               const char *outp)
+{
+    const uint64_t np = pairs.size();
+    std::vector<pa_score> sc(np);
+    void *dp = nullptr, *ds = nullptr;
+    int rc;
+    if ((rc = pa_device_alloc(c, np * sizeof(pa_pair), &dp)) ||
+        (rc = pa_device_alloc(c, np * sizeof(pa_score), &ds)) ||
+        (rc = pa_memcpy_h2d(c, dp, pairs.data(), np * sizeof(pa_pair))) ||
+        (rc = (std::strcmp(entry, "noalloc") == 0
+                   ? pa_sw_scores_noalloc
+                   : pa_sw_scores_dev)(c, (const pa_pair *)dp, np,
+                                       (pa_score *)ds, nullptr)) ||
+        (rc = pa_memcpy_d2h(c, sc.data(), ds, np * sizeof(pa_score))))
+        return fail("pa_sw_scores", rc, c);
+    FILE *f = std::fopen(outp, "wb");
+    if (!f)
+        return 2;
+    std::fwrite(sc.data(), sizeof(pa_score), np, f);
+    std::fclose(f);
+    pa_device_free(c, dp);
+    pa_device_free(c, ds);
     return 0;
 }
 
@@ -136,14 +183,36 @@ int main(int argc, char **argv)
     if ((rc = pa_load_seqs(c, PA_SIDE_BOTH, codes.data(), offs.data(), nseq,
                            PA_ENC_CODES)))
         return fail("pa_load_seqs", rc, c);
+    const char *scores = std::getenv("EMU_SCORES");
+    const bool dev = std::getenv("EMU_DEV") != nullptr;
+    if (scores) {
+        rc = scores_run(c, pairs, scores, argv[2]);
+        const int st = write_stats(c);
+        pa_destroy(c);
+        return rc ? rc : st;
+    }
     std::vector<pa_result> res(np);
-    if ((rc = pa_align(c, pairs.data(), np, res.data())))
+    if (dev) {
+        void *dp = nullptr, *dr = nullptr;
+        if ((rc = pa_device_alloc(c, np * sizeof(pa_pair), &dp)) ||
+            (rc = pa_device_alloc(c, np * sizeof(pa_result), &dr)) ||
+            (rc = pa_memcpy_h2d(c, dp, pairs.data(), np * sizeof(pa_pair))) ||
+            (rc = pa_align_dev(c, (const pa_pair *)dp, np, (pa_result *)dr,
+                               nullptr)) ||
+            (rc = pa_memcpy_d2h(c, res.data(), dr, np * sizeof(pa_result))))
+            return fail("pa_align_dev", rc, c);
+        pa_device_free(c, dp);
+        pa_device_free(c, dr);
+    } else if ((rc = pa_align(c, pairs.data(), np, res.data()))) {
         return fail("pa_align", rc, c);
+    }
+    if ((rc = write_stats(c)))
+        return rc;
     FILE *out = std::fopen(argv[2], "wb");
     if (!out)
         return 2;
     std::fwrite(res.data(), sizeof(pa_result), np, out);
-    if (cfg.mode == PA_MODE_XDROP) {
+    if (cfg.mode == PA_MODE_XDROP && !dev) {
         std::vector<pa_extent> ext(np);
         for (int s = 0; s < cfg.seed_cnt; ++s) {
             if ((rc = pa_xdrop_extents(c, pairs.data(), np, s, ext.data())))

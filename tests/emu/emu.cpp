@@ -3,6 +3,7 @@
 
 #include <cstdio>
 #include <mutex>
+#include <string>
 
 namespace emu {
 thread_local dim3 tIdx, bIdx, bDim, gDim;
@@ -46,6 +47,20 @@ uint64_t wave_ballot(bool p)
 }
 
 void block_sync() { g_block->arrive_and_wait(); }
+
+void log_launch(const char *name, dim3 g, dim3 b)
+{
+    const char *path = std::getenv("EMU_LAUNCHES");
+    if (!path)
+        return;
+    // a template kernel is passed as "(name<...>)", in parentheses or not
+    std::string n(name[0] == '(' ? name + 1 : name);
+    n = n.substr(0, n.find_first_of("<)"));
+    if (FILE *f = std::fopen(path, "a")) {
+        std::fprintf(f, "%s %u %u\n", n.c_str(), g.x, b.x);
+        std::fclose(f);
+    }
+}
 
 void launch_impl(dim3 g, dim3 b, size_t shmem, void (*body)(void *), void *arg)
 {

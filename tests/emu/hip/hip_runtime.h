@@ -77,10 +77,15 @@ void launch_impl(dim3 g, dim3 b, size_t shmem, void (*body)(void *),
 
 template <class F> void trampoline(void *p) { (*(F *)p)(); }
 
+// One line per launch, "kernel workgroups threads", appended to the file that
+// EMU_LAUNCHES names.
+void log_launch(const char *name, dim3 g, dim3 b);
+
 template <class K, class... A>
-void launch(K kernel, dim3 g, dim3 b, size_t shmem, A... args)
+void launch(const char *name, K kernel, dim3 g, dim3 b, size_t shmem, A... args)
 {
     auto f = [=]() { kernel(args...); };
+    log_launch(name, g, b);
     launch_impl(g, b, shmem, &trampoline<decltype(f)>, (void *)&f);
 }
 }  // namespace emu
@@ -91,7 +96,7 @@ void launch(K kernel, dim3 g, dim3 b, size_t shmem, A... args)
 #define gridDim emu::gDim
 
 #define hipLaunchKernelGGL(kernel, grid, block, shmem, stream, ...) \
-    emu::launch(kernel, dim3(grid), dim3(block), (size_t)(shmem), __VA_ARGS__)
+    emu::launch(#kernel, kernel, dim3(grid), dim3(block), (size_t)(shmem), __VA_ARGS__)
 
 inline void __syncthreads() { emu::block_sync(); }
 inline void __threadfence() { std::atomic_thread_fence(std::memory_order_seq_cst); }

@@ -1,0 +1,68 @@
+"""Which kernels a call launches, on the CPU emulation of tests/test_emu.py.
+
+The emulation runs workgroups one after the other, so a race between two of
+them changes no result here; these tests look at the launches instead.
+"""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from helpers import oracle_params, pairs_of, rand_seq, seqset
+from oracle import oracle as orc
+from pastis_amd._lib import PAIR_DTYPE, RESULT_DTYPE
+from test_emu import driver  # noqa: F401  (the built driver, a fixture)
+
+
+def run(driver, tmp_path, codes, offs, pairs, mode=0, xdrop=0, gap_model=0,
+        shapes=None, **env):
+    """Results (pa_result) and the launches as (kernel, workgroups)."""
+    inp, outp, log = (tmp_path / n for n in ("in.bin", "out.bin", "log.txt"))
+    log.unlink(missing_ok=True)
+    hdr = np.array([mode, -11, -2, 6, xdrop, 2, gap_model, 0], np.int32)
+    with open(inp, "wb") as f:
+        f.write(hdr.tobytes())
+        f.write(np.array([len(offs) - 1, len(pairs)], np.uint64).tobytes())
+        f.write(np.ascontiguousarray(offs, np.uint64).tobytes())
+        f.write(np.ascontiguousarray(codes, np.uint8).tobytes())
+        f.write(np.ascontiguousarray(pairs, PAIR_DTYPE).tobytes())
+    e = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:abort_on_error=1",
+             UBSAN_OPTIONS="print_stacktrace=1", EMU_LAUNCHES=str(log), **env)
+    if shapes is not None:
+        e["EMU_SHAPES"] = ",".join(str(v) for v in shapes)
+    r = subprocess.run([driver, str(inp), str(outp)], env=e,
+                       capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stderr[-4000:]
+    launches = [(n, int(g)) for n, g, _ in
+                (ln.split() for ln in open(log))]
+    return outp.read_bytes(), launches
+
+
+# Default shapes: 128, 256 and 512 rows a pass in the classes below the last.
+# A task of several passes keeps a boundary row at workgroup * slots + slot,
+# and the classes have 8, 4, 2 and 1 slots a workgroup, so in one launch the
+# second workgroup of class 2 (rows 2 and 3) and workgroups 2 and 3 of class 3
+# would share rows if both classes held such tasks.
+@pytest.mark.parametrize("edges,one", [
+    ((128, 256, 512), True), ((64, 200, 400), True),
+    ((129, 256, 512), False), ((128, 257, 512), False),
+    ((128, 256, 513), False), ((128, 256, 768), False),
+    ((128, 384, 768), False)])
+def test_affine_one_launch_only_with_one_pass_below_the_last_class(
+        driver, tmp_path, edges, one):
+    rng = np.random.default_rng(5)
+    seqs = [rand_seq(rng, n) for n in (600, 1030, 300, 12)]
+    codes, offs = seqset(seqs)
+    pairs = pairs_of([(0, 3), (1, 3), (2, 3)])
+    raw, launches = run(driver, tmp_path, codes, offs, pairs, gap_model=1,
+                        shapes=(5, 1, 4, 3) + edges + (1, 0))
+    got = np.frombuffer(raw, RESULT_DTYPE)
+    ref = orc.sfa_batch(codes, offs, pairs["r"], pairs["c"],
+                        oracle_params("as_documented"))
+    for f in ("score", "matches", "cols", "gap_opens"):
+        assert np.array_equal(got[f].astype(np.int64),
+                              ref[f].astype(np.int64)), f
+    names = [n for n, _ in launches]
+    assert ("k_dp_all" in names) == one
+    assert ("k_traceback_all" in names) == one
