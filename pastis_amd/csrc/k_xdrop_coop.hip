@@ -183,6 +183,12 @@ __global__ __launch_bounds__(256) void k_xdrop_coop(CoopArgs a)
                             db = h + beg_h + a.seed_len - 1;
                             qstep = 1;
                         }
+                        // the rings load up to cols and rows whatever the
+                        // item's state, and the seed of an invalid task may
+                        // lie anywhere
+                        invalid = (T.pad & kXdInvalid) != 0;
+                        if (invalid)
+                            cols = rows = 0;
                         // anti-diagonal 0: column 0 = 0; anti-diagonal 1:
                         // columns 0 and 1 = gap (undefined when -gap > X)
                         const int g1 = -gap > X ? kUndef : gap;
@@ -200,7 +206,7 @@ __global__ __launch_bounds__(256) void k_xdrop_coop(CoopArgs a)
                         dgap = gap;
                         edge = -gap <= X;
                         state = kRun;
-                        if ((T.pad & kXdInvalid) || rows <= 1 || cols <= 1) {
+                        if (rows <= 1 || cols <= 1) {
                             state = 3;   // finished without an update
                         } else {
                             const int f = 1 + j;
@@ -217,7 +223,6 @@ __global__ __launch_bounds__(256) void k_xdrop_coop(CoopArgs a)
                             qv = q_load(max(j, 1)) << 5;
                             sc = mat[qv | d_load(1)];
                         }
-                        invalid = (T.pad & kXdInvalid) != 0;
                     }
                 }
                 cbase += take;

@@ -268,6 +268,11 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
                         db = h + beg_h + a.seed_len - 1;
                         qstep = 1;
                     }
+                    // the rings load up to cols and rows whatever the item's
+                    // state, and the seed of an invalid task may lie anywhere
+                    invalid = (T.pad & kXdInvalid) != 0;
+                    if (invalid)
+                        cols = rows = 0;
                     // No cell lies more below the best score than the gaps of
                     // its anti-diagonal and 31 (the largest matrix score) per
                     // row or column: a larger X drops nothing either.
@@ -287,9 +292,8 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
                     dgap = gap;
                     edge = -gap <= X;
                     masked = 3;
-                    invalid = (T.pad & kXdInvalid) != 0;
                     state = kRun;
-                    if (invalid || rows <= 1 || cols <= 1) {
+                    if (rows <= 1 || cols <= 1) {
                         state = kEmpty;
                     } else {
                         // anti-diagonal 0: column 0 = 0; anti-diagonal 1:

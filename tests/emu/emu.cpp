@@ -3,6 +3,7 @@
 
 #include <cstdio>
 #include <mutex>
+#include <sanitizer/asan_interface.h>
 #include <string>
 
 namespace emu {
@@ -93,17 +94,34 @@ void launch_impl(dim3 g, dim3 b, size_t shmem, void (*body)(void *), void *arg)
 }
 }  // namespace emu
 
+// Device memory lies between margins that the address sanitizer reports, wide
+// enough that an access a sequence's length off does not reach other memory.
+constexpr size_t kMargin = (size_t)1 << 17;
+
 hipError_t hipMalloc(void **p, size_t n)
 {
-    *p = std::malloc(n ? n : 1);
-    if (!*p)
+    n = (n + 7) & ~(size_t)7;
+    char *m = (char *)std::malloc(n + 2 * kMargin + 16);
+    if (!m) {
+        *p = nullptr;
         return hipErrorOutOfMemory;
-    std::memset(*p, 0xa5, n);
+    }
+    std::memcpy(m, &n, sizeof(n));
+    std::memset(m + kMargin, 0xa5, n);
+    ASAN_POISON_MEMORY_REGION(m + 8, kMargin - 8);
+    ASAN_POISON_MEMORY_REGION(m + kMargin + n, kMargin);
+    *p = m + kMargin;
     return hipSuccess;
 }
 hipError_t hipFree(void *p)
 {
-    std::free(p);
+    if (!p)
+        return hipSuccess;
+    char *m = (char *)p - kMargin;
+    size_t n;
+    std::memcpy(&n, m, sizeof(n));
+    ASAN_UNPOISON_MEMORY_REGION(m, n + 2 * kMargin);
+    std::free(m);
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned)

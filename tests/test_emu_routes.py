@@ -66,3 +66,38 @@ def test_affine_one_launch_only_with_one_pass_below_the_last_class(
     names = [n for n, _ in launches]
     assert ("k_dp_all" in names) == one
     assert ("k_traceback_all" in names) == one
+
+
+# Seeds far past the end of their sequences, and pairs outside the sets, in
+# the kernels that take a small batch first: 16 lanes per item as called, the
+# band kernels as documented, among good pairs or alone.  The sanitizers report
+# a read outside the store.
+@pytest.mark.parametrize("alone", [False, True])
+@pytest.mark.parametrize("gap_model", [0, 1])
+def test_pairs_that_do_not_fit_read_no_residues(driver, tmp_path, gap_model,
+                                                alone):
+    rng = np.random.default_rng(9)
+    codes, offs = seqset([rand_seq(rng, 40) for _ in range(3)])
+    far = [1 << k for k in range(15, 11, -1)] + list(range(3000, 40, -61))
+    rc = [(2, 2)] * len(far) + [(7, 2), (2, 9), (0, 1), (1, 2)]
+    seeds = [[f, f, f, f + 1] for f in far] + [[900, 900, 900, 900]] * 2 + \
+        [[10, 12, 10, 12], [3, 4, 3, 4]]
+    pairs = pairs_of(rc, seeds)
+    if alone:
+        pairs = pairs[:-2]
+    raw, launches = run(driver, tmp_path, codes, offs, pairs, mode=1,
+                        xdrop=49, gap_model=gap_model, EMU_DEV="1")
+    assert ("k_xdrop_band" if gap_model else "k_xdrop_coop") in \
+        [n for n, _ in launches]
+    got = np.frombuffer(raw, RESULT_DTYPE)
+    for f in ("score", "matches", "cols", "score_aln"):
+        assert not got[f][:len(far) + 2].any(), f
+    if alone:
+        return
+    good = pairs[-2:]
+    ref = orc.sxa_batch(codes, offs, good["r"], good["c"], good["seed"],
+                        oracle_params(["as_called", "as_documented"]
+                                      [gap_model]))
+    for f in ("score", "matches", "cols", "gap_opens"):
+        assert np.array_equal(got[f][-2:].astype(np.int64),
+                              ref[f].astype(np.int64)), f
