@@ -538,10 +538,7 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
                 Scope k(c, 5 + dmode, s);
                 // progress words of the pipelined items: none yet
                 HIPCHK(c, fill_u32((uint32_t *)la.prog, 0, 2 * ll.slots, s));
-                HIPCHK(c, launch_dp_linear(la, local, trace, (int)grid,
-                                           (int)std::min(
-                                               grid, (uint32_t)c->ncu),
-                                           s));
+                HIPCHK(c, launch_dp_linear(la, local, trace, (int)grid, s));
             }
             if (trace) {
                 Scope sc(c, 3, s);

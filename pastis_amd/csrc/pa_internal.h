@@ -388,7 +388,7 @@ struct LinArgs {
     int32_t gap, nib_min;
 };
 hipError_t launch_dp_linear(const LinArgs &a, bool local, bool trace, int grid,
-                            int rerun_grid, hipStream_t s);
+                            hipStream_t s);
 int dp_linear_occupancy(bool local, bool trace);
 hipError_t launch_traceback_linear(const LinArgs &a, bool local,
                                    uint32_t ntasks, hipStream_t s);

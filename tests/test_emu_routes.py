@@ -101,3 +101,24 @@ def test_pairs_that_do_not_fit_read_no_residues(driver, tmp_path, gap_model,
     for f in ("score", "matches", "cols", "gap_opens"):
         assert np.array_equal(got[f][-2:].astype(np.int64),
                               ref[f].astype(np.int64)), f
+
+
+def _equal_scores(tmp_path, driver, codes, offs, pairs, **env):
+    raw, launches = run(driver, tmp_path, codes, offs, pairs, **env)
+    got = np.frombuffer(raw, RESULT_DTYPE)
+    ref = orc.sfa_batch(codes, offs, pairs["r"], pairs["c"],
+                        oracle_params("as_called"))
+    for f in ("score", "matches", "cols", "gap_opens"):
+        assert np.array_equal(got[f].astype(np.int64),
+                              ref[f].astype(np.int64)), f
+    return launches
+
+
+def test_linear_rerun_has_the_grid_of_the_first_run(driver, tmp_path):
+    """Every task of a batch may leave int16, and the int32 run of them is
+    then the longer one."""
+    rng = np.random.default_rng(10)
+    codes, offs = seqset([rand_seq(rng, 12) for _ in range(6)])
+    pairs = pairs_of([(r, c) for r in range(6) for c in range(6)])
+    grids = dict(_equal_scores(tmp_path, driver, codes, offs, pairs))
+    assert grids["k_sw_linear_rerun"] == grids["k_sw_linear"] > 2
