@@ -22,7 +22,7 @@
 // limits): about 0.2 us for four items a wave, a quarter of what the per-lane
 // kernel of k_xdrop.hip takes for its 64.  So it runs where the per-lane
 // kernel would leave the chip waiting for single lanes: all items of a small
-// batch, and the items of a large one that may go on for long (run_xdrop).
+// batch, and the items of a larger one that may go on for long (xd_route).
 // An item whose written range would exceed 16 columns stops and goes to the
 // overflow list; the band kernels recompute it from scratch.  A row whose
 // item ends takes the next item of the queue at once, so the four rows of a

@@ -98,14 +98,6 @@ enum {
 
 constexpr int kModes = 3;           // DP modes of the kernel statistics
 constexpr int kMaxWgPerCu = 32;     // one-wave workgroups per CU (8 per SIMD)
-// X-drop work items of a batch small enough for 16 lanes per item, and the
-// reach (xd_reach) from which an item of a larger batch gets 16 lanes.  A lane
-// alone takes 0.7 us an anti-diagonal in an idle chip and 3 us beside five
-// other waves, a row of 16 lanes 0.2 us: 1,204 items 1.60 -> 0.28 ms, and in
-// 1.6 M items, where the longest took 8.3 ms, both kernels now end together
-// after 3.3 ms (reaches of 768 and more: 5.4 and 3.5 ms).
-constexpr uint64_t kXdSmall = 65536;
-constexpr uint32_t kXdLong = 512;
 constexpr int kXdWideLanes = 65536;  // lanes of the wide (global scratch) re-run
 constexpr int kXdGraphLanes = 4096;  // its lanes in a captured batch
 
@@ -856,29 +848,16 @@ int run_xdrop(pa_ctx *c, const pa_pair *d_pairs, uint64_t n, hipStream_t s)
                              P<uint64_t>(c->roffs), P<uint64_t>(c->coffs),
                              c->rlen.size(), c->clen.size(),
                              P<XdTask>(c->xdt), s));
-    // Which kernel takes an item first.  Sixteen lanes per item take a fifth
-    // of the time per anti-diagonal that one lane takes, at four times the
-    // instructions: they run all items of a small batch (kXdSmall) and, in a
-    // larger one, those that may extend far (kXdLong), on the second stream
-    // beside the others, which start in the order of their reach so that the
-    // grid does not end on long ones.  Only while the bands fit 16 columns: a
-    // gap costs -xdrop_gap and an extension ends X below its best, so a band
-    // spans about 2 X / -xdrop_gap columns (9 as called, 49 as documented).
-    const bool thin = c->cfg.xdrop / -c->cfg.xdrop_gap <= 5;
-    const bool small16 = thin && !c->tune.xd_coop && ni <= kXdSmall;
-    const bool two = thin && !c->tune.xd_coop && !small16;
-    // Wider bands outgrow 16 columns in most items: the band kernels take all
-    // of them, those that may extend far first (60,001 pairs, X = 49, gap -2:
-    // per-lane pass 0.87 ms and 5.5 ms for its overflow, unsorted; 4.7 ms for
-    // all).
-    const bool all_band = !thin && !c->tune.xd_coop && c->tune.xd_wave == 1 &&
-                      c->cfg.xdrop <= 30000;
+    const XdRoute way = xd_route(ni, c->cfg.xdrop, c->cfg.xdrop_gap,
+                                 c->tune.xd_coop, c->tune.xd_wave);
     uint32_t *const order = lng + ni;
-    if (two || all_band)
+    if (way.sorted) {
+        Scope t(c, 1, s);
         HIPCHK(c, sort_reach(P<XdTask>(c->xdt), nt, c->cfg.seed_len,
-                             all_band ? UINT32_MAX : kXdLong,
-                             ctr + C_HIST, ctr + C_FILL, order,
-                             ctr + C_XDN, lng, ctr + C_XDLONG, s));
+                             way.split ? kXdLong : UINT32_MAX, ctr + C_HIST,
+                             ctr + C_FILL, order, ctr + C_XDN, lng,
+                             ctr + C_XDLONG, s));
+    }
     auto coop = [&](const uint32_t *list, uint32_t *count, uint32_t *queue,
                     uint64_t most, uint32_t *to, uint32_t *to_n,
                     hipStream_t cs) -> int {
@@ -894,10 +873,10 @@ int run_xdrop(pa_ctx *c, const pa_pair *d_pairs, uint64_t n, hipStream_t s)
         c->stats.launches++;
         return PA_OK;
     };
-    if (!all_band) {
+    if (!way.all_band) {
         Scope t(c, 1, s);
         const int grid = xd_grid(c, ni);
-        if (small16) {
+        if (way.small16) {
             if ((rc = coop(nullptr, ctr + C_XDN, ctr + C_XDQ, ni, ovf,
                            ctr + C_XDOVF, s)))
                 return rc;
@@ -916,21 +895,22 @@ int run_xdrop(pa_ctx *c, const pa_pair *d_pairs, uint64_t n, hipStream_t s)
             c->stats.launches++;
         } else {
             // both kernels append to the same overflow list
-            if (two) {
+            if (way.split) {
                 HIPCHK(c, hipEventRecord(c->ev_fork[0], s));
                 HIPCHK(c, hipStreamWaitEvent(c->st2, c->ev_fork[0], 0));
                 if ((rc = coop(lng, ctr + C_XDLONG, ctr + C_XDLONGQ, ni, ovf,
                                ctr + C_XDOVF, c->st2)))
                     return rc;
             }
-            HIPCHK(c, launch_xdrop(P<XdTask>(c->xdt), two ? order : nullptr,
+            HIPCHK(c, launch_xdrop(P<XdTask>(c->xdt),
+                                   way.sorted ? order : nullptr,
                                    ctr + C_XDN, ctr + C_XDQ,
                                    P<int8_t>(c->dmat), c->cfg.xdrop_gap,
                                    c->cfg.xdrop, c->cfg.seed_len, nullptr, 0,
                                    P<XdOut>(c->xdo), ovf, ctr + C_XDOVF, grid,
                                    c->tune.xd_ring, s));
             c->stats.launches++;
-            if (two) {
+            if (way.split) {
                 HIPCHK(c, hipEventRecord(c->ev_join, c->st2));
                 HIPCHK(c, hipStreamWaitEvent(s, c->ev_join, 0));
             }
@@ -942,7 +922,7 @@ int run_xdrop(pa_ctx *c, const pa_pair *d_pairs, uint64_t n, hipStream_t s)
     // list the pass before last consumed (`lng` is free once the per-lane
     // kernel is done).
     uint32_t *last = ovf, *last_n = ctr + C_XDOVF, *last_q = ctr + C_XDOVFQ;
-    if (all_band) {
+    if (way.all_band) {
         last = order;
         last_n = ctr + C_XDN;
         last_q = ctr + C_XDQ;

@@ -417,6 +417,53 @@ __host__ __device__ inline uint32_t xd_reach(const XdTask &t, int dir,
     return h < v ? h : v;
 }
 
+// X-drop work items of a batch small enough for 16 lanes per item, the reach
+// (xd_reach) from which an item of a larger batch gets 16 lanes, and the items
+// up to which a batch is split that way.
+constexpr uint64_t kXdSmall = 65536, kXdSplit = (uint64_t)4 << 20;
+constexpr uint32_t kXdLong = 512;
+
+// Which kernel takes an item first.  Sixteen lanes per item take a fifth of the
+// time per anti-diagonal that one lane takes (0.2 us; a lane 0.7 in an idle
+// chip, 3 beside five other waves), at four times the instructions.
+//   small16: all items of a small batch.
+//   split: the items of a larger one that may extend far, on the second stream
+//     beside the others.  Not in a full chip, where the instructions count and
+//     the longest item ends before the rest does.
+//   sorted: the one-lane kernel's items (with all_band: the band kernel's) in
+//     falling order of their reach, so that the grid does not end on long ones.
+//   all_band: 16 lanes and wide bands for all items.
+// The first two only while the bands fit 16 columns: a gap costs -xdrop_gap and
+// an extension ends X below its best, so a band spans about 2 X / -xdrop_gap
+// columns (9 as called, 49 as documented).  Wider bands outgrow 16 columns in
+// most items: the band kernels take all of them (60,001 pairs, X = 49, gap -2:
+// per-lane pass 0.87 ms and 5.5 ms for its overflow, unsorted; 4.7 ms for all).
+// Measured for the log-normal workload as called (30 % homologs, four items a
+// pair), the whole stage in ms:
+//   pairs          one lane, unsorted   sorted   split   16 lanes
+//       16,384                   4.42     5.11    2.30      1.43
+//       65,536                   5.73     6.03    2.42      2.27
+//      262,144                   7.14     7.02    4.07      5.41
+//      800,000                  10.99     9.75    9.25
+//    1,200,000                  13.67    12.28   12.94
+//    5,000,000                  42.70    40.08   45.22
+struct XdRoute {
+    bool small16, split, sorted, all_band;
+};
+inline XdRoute xd_route(uint64_t ni, int xdrop, int xdrop_gap, int xd_coop,
+                        int xd_wave)
+{
+    XdRoute r{};
+    if (xd_coop)
+        return r;
+    const bool thin = xdrop / -(int64_t)xdrop_gap <= 5;
+    r.small16 = thin && ni <= kXdSmall;
+    r.split = thin && !r.small16 && ni <= kXdSplit;
+    r.all_band = !thin && xd_wave == 1 && xdrop <= 30000;
+    r.sorted = (thin && !r.small16) || r.all_band;
+    return r;
+}
+
 // Seed extension result; the left direction writes beg_*, score_left,
 // cells_left, flags_left and the right direction the other half.
 struct XdOut {
