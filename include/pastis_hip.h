@@ -129,7 +129,7 @@ typedef struct pa_stats {
     double ms_nw;            /* device time of the global-alignment kernels */
     double ms_trace;         /* device time of the traceback kernels */
     double ms_total;         /* device time of whole calls (event to event) */
-    uint64_t launches;       /* kernel launches */
+    uint64_t launches;       /* launches of DP, X-drop and traceback kernels */
     uint64_t graph_captures; /* graphs captured by pa_sw_scores_graph */
 } pa_stats;
 

@@ -536,7 +536,8 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
                 Scope sc(c, 3, s);
                 HIPCHK(c, launch_traceback_linear(la, local, b - a, s));
             }
-            c->stats.launches += trace ? 2 : 1;
+            // k_lin_passes, the DP, its int32 run (local), the walks
+            c->stats.launches += 2 + (local ? 1 : 0) + (trace ? 1 : 0);
             continue;
         }
         DpArgs args{};

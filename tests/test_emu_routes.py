@@ -144,3 +144,22 @@ def test_xdrop_route(items, xdrop, gap, coop, wave, want):
                                            (items, xdrop, gap, coop, wave)],
                        capture_output=True, text=True, check=True)
     assert r.stdout.strip() == want
+
+
+# pa_stats counts the launches of the DP, X-drop and traceback kernels
+COUNTED = ("k_dp", "k_nw_", "k_sw_", "k_lin_", "k_xdrop", "k_traceback")
+
+
+@pytest.mark.parametrize("mode,gap_model,env", [
+    (0, 0, {}), (0, 1, {}), (1, 0, {}), (1, 1, {}),
+    (0, 0, {"EMU_SCORES": "dev"}), (0, 1, {"EMU_SCORES": "dev"})])
+def test_launches_are_counted(driver, tmp_path, mode, gap_model, env):
+    rng = np.random.default_rng(11)
+    codes, offs = seqset([rand_seq(rng, 14) for _ in range(3)])
+    pairs = pairs_of([(0, 1), (1, 2)], [[2, 2, 4, 4]] * 2)
+    stats = tmp_path / "stats.txt"
+    _, launches = run(driver, tmp_path, codes, offs, pairs, mode=mode,
+                      xdrop=49 if mode else 0, gap_model=gap_model,
+                      EMU_DEV="1", EMU_STATS=str(stats), **env)
+    assert int(stats.read_text()) == sum(n.startswith(COUNTED)
+                                         for n, _ in launches)
