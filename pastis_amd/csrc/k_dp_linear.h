@@ -1148,7 +1148,8 @@ __global__ __launch_bounds__(kTbThreads) void k_traceback_linear(LinArgs a)
 hipError_t launch_dp_linear(const LinArgs &a, bool local, bool trace, int grid,
                             hipStream_t s)
 {
-    hipLaunchKernelGGL(k_lin_passes, dim3(1), dim3(256), 0, s, a);
+    if (a.pipe_slots)
+        hipLaunchKernelGGL(k_lin_passes, dim3(1), dim3(256), 0, s, a);
     if (!local) {
         hipLaunchKernelGGL(k_nw_linear, dim3(grid), dim3(64), 0, s, a);
     } else if (trace) {

@@ -54,9 +54,9 @@ hipError_t bin_tasks(const DpTask *tasks, uint32_t a, uint32_t b,
                      uint32_t cap, uint32_t *counts, uint32_t *hist,
                      uint32_t *fill, unsigned long long *bin_cells,
                      hipStream_t s, const uint32_t *rng = nullptr);
-// The same for the linear-gap kernel: bin = lin_class, one list with the bins
+// The same for the linear-gap kernel: bin = lin_class (pipe), one list with the bins
 // one after the other, the last bin first; starts receives their places.
-hipError_t bin_linear(const DpTask *tasks, uint32_t a, uint32_t b,
+hipError_t bin_linear(const DpTask *tasks, uint32_t a, uint32_t b, bool pipe,
                       uint32_t *list, uint32_t *counts, uint32_t *starts,
                       uint32_t *hist, uint32_t *fill,
                       unsigned long long *bin_cells, hipStream_t s,

@@ -273,11 +273,12 @@ __device__ inline uint32_t task_steps(uint32_t qlen, uint32_t tlen,
     return (npass - 1) * (tlen + 2u * L - 1u) + tlen + 2u * (nl - 1u) + 1u;
 }
 
-// What bin_key needs: the class shapes and the int16 bounds (unused for the
-// linear-gap kernel's sort).
+// What bin_key needs: the class shapes and the int16 bounds, or for the
+// linear-gap kernel's sort whether passes are pipelined.
 struct BinArgs {
     DpShapes sh;
     int local, maxs, open, ext;
+    bool pipe;
 };
 
 // Bin and bucket of a task (-1: empty task).  Buckets are 1/8 of an octave
@@ -290,7 +291,7 @@ __device__ inline int bin_key(const DpTask &t, const BinArgs &a)
     int bin;
     uint32_t steps;
     if (LIN) {
-        bin = lin_class(t.qlen, t.tlen);
+        bin = lin_class(t.qlen, t.tlen, a.pipe);
         steps = (t.qlen - 1) / kLinRows * (t.tlen + 127u) + t.tlen +
                 2u * (lin_last_lanes(t.qlen) - 1u) + 1u;
     } else {
@@ -703,19 +704,21 @@ hipError_t bin_tasks(const DpTask *tasks, uint32_t a, uint32_t b,
                      uint32_t *fill, unsigned long long *bin_cells,
                      hipStream_t s, const uint32_t *rng)
 {
-    return bin_run<kBins>(tasks, a, b, BinArgs{sh, local, maxs, open, ext},
+    return bin_run<kBins>(tasks, a, b, BinArgs{sh, local, maxs, open, ext, false},
                           lists, cap, counts, nullptr, hist, fill, bin_cells,
                           s, rng);
 }
 
-hipError_t bin_linear(const DpTask *tasks, uint32_t a, uint32_t b,
+hipError_t bin_linear(const DpTask *tasks, uint32_t a, uint32_t b, bool pipe,
                       uint32_t *list, uint32_t *counts, uint32_t *starts,
                       uint32_t *hist, uint32_t *fill,
                       unsigned long long *bin_cells, hipStream_t s,
                       const uint32_t *rng)
 {
-    return bin_run<kLinClasses>(tasks, a, b, BinArgs{}, list, 0, counts,
-                                starts, hist, fill, bin_cells, s, rng);
+    BinArgs ba{};
+    ba.pipe = pipe;
+    return bin_run<kLinClasses>(tasks, a, b, ba, list, 0, counts, starts, hist,
+                                fill, bin_cells, s, rng);
 }
 
 hipError_t trace_sizes(const DpTask *tasks, uint64_t n, const DpShapes &sh,

@@ -240,7 +240,8 @@ int xd_grid(pa_ctx *c, uint64_t nitems)
 
 // Linear-gap kernels: persistent grid, boundary-row slots of the pipelined
 // class (any number from 2 on is correct; twice the grid never waits for a
-// slot) and their sizes in c->bnd: the progress words, then the rows.
+// slot; 0: no task is in that class) and their sizes in c->bnd: the progress
+// words, then the rows.
 struct LinLayout {
     uint32_t grid, slots, words;
     size_t prog_bytes() const { return (size_t)slots * 16; }
@@ -264,12 +265,14 @@ LinLayout lin_layout(pa_ctx *c, bool local, bool trace)
     l.grid = (uint32_t)(c->ncu * per_cu);
     l.slots = 2 * l.grid;
     l.words = (c->max_clen + 1u) / 2u + kLinBndPad;
-    if (c->slot_cap > 0) {   // a workspace of fixed size (pa_noalloc.hip)
-        const uint64_t fit = c->bnd.cap / ((size_t)l.words * 8 + 16);
-        l.slots = (uint32_t)std::max<uint64_t>(
-            2, std::min<uint64_t>(l.slots, fit / 8));
+    if (c->slot_cap > 0) {
+        // A workspace of fixed size, which calls share (pa_noalloc.hip): one
+        // that overlaps another takes its progress words away, and a pass
+        // must not wait for words that nobody writes.
+        l.slots = 0;
         l.grid = (uint32_t)std::max<uint64_t>(
-            1, std::min<uint64_t>(l.grid, fit - l.slots));
+            1, std::min<uint64_t>(l.grid,
+                                  c->bnd.cap / ((size_t)l.words * 8)));
     }
     return l;
 }
@@ -482,8 +485,8 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
         HIPCHK(c, fill_u32(ctr + C_LIN, 0, C_N - C_LIN, s));
         if (lin)
             HIPCHK(c, bin_linear(
-                          P<DpTask>(c->tasks), a, b, lists, ctr + C_LIN,
-                          ctr + C_LINS, ctr + C_HIST, ctr + C_FILL,
+                          P<DpTask>(c->tasks), a, b, ll.slots > 0, lists,
+                          ctr + C_LIN, ctr + C_LINS, ctr + C_HIST, ctr + C_FILL,
                           (unsigned long long *)P<uint64_t>(c->bincells) +
                               (kModes + dmode) * kBins,
                           s, rng));
@@ -529,7 +532,9 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
                 Scope sc(c, kind, s);
                 Scope k(c, 5 + dmode, s);
                 // progress words of the pipelined items: none yet
-                HIPCHK(c, fill_u32((uint32_t *)la.prog, 0, 2 * ll.slots, s));
+                if (ll.slots)
+                    HIPCHK(c, fill_u32((uint32_t *)la.prog, 0, 2 * ll.slots,
+                                       s));
                 HIPCHK(c, launch_dp_linear(la, local, trace, (int)grid, s));
             }
             if (trace) {
@@ -537,7 +542,8 @@ int run_dp(pa_ctx *c, uint64_t nt, bool local, bool trace, int kind,
                 HIPCHK(c, launch_traceback_linear(la, local, b - a, s));
             }
             // k_lin_passes, the DP, its int32 run (local), the walks
-            c->stats.launches += 2 + (local ? 1 : 0) + (trace ? 1 : 0);
+            c->stats.launches +=
+                1 + (ll.slots ? 1 : 0) + (local ? 1 : 0) + (trace ? 1 : 0);
             continue;
         }
         DpArgs args{};

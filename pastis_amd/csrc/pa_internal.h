@@ -328,9 +328,11 @@ __host__ __device__ inline int lin_lanes(int cls)
            : cls == 13 ? 32
                        : 64;
 }
-__host__ __device__ inline int lin_class(uint32_t qlen, uint32_t tlen)
+// pipe: the pipelined class may be used
+__host__ __device__ inline int lin_class(uint32_t qlen, uint32_t tlen,
+                                         bool pipe)
 {
-    if (qlen > kLinRows && tlen >= kLinPipeCols)
+    if (pipe && qlen > kLinRows && tlen >= kLinPipeCols)
         return kLinPipe;
     const uint32_t need = (qlen + 2u * kLinR - 1u) / (2u * kLinR);
     return need <= 10   ? (int)need - 1
@@ -374,8 +376,8 @@ struct LinArgs {
     uint8_t *trace;
     const uint64_t *trace_off;
     const uint64_t *trace_base; // as DpArgs::trace_base
-    // boundary rows of bnd_words words: pipe_slots for pipelined passes, then
-    // one per workgroup
+    // boundary rows of bnd_words words: pipe_slots for pipelined passes (0:
+    // no task is in their class), then one per workgroup
     uint64_t *bnd;
     uint32_t bnd_words;
     uint32_t pipe_slots;

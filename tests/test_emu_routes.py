@@ -11,7 +11,7 @@ import pytest
 
 from helpers import oracle_params, pairs_of, rand_seq, seqset
 from oracle import oracle as orc
-from pastis_amd._lib import PAIR_DTYPE, RESULT_DTYPE
+from pastis_amd._lib import PAIR_DTYPE, RESULT_DTYPE, SCORE_DTYPE
 from test_emu import EMU, OUT, driver  # noqa: F401  (driver: a fixture)
 
 
@@ -163,3 +163,26 @@ def test_launches_are_counted(driver, tmp_path, mode, gap_model, env):
                       EMU_DEV="1", EMU_STATS=str(stats), **env)
     assert int(stats.read_text()) == sum(n.startswith(COUNTED)
                                          for n, _ in launches)
+
+
+@pytest.mark.parametrize("entry", ["dev", "noalloc"])
+def test_passes_wait_for_one_another_only_on_a_workspace_of_ones_own(
+        driver, tmp_path, entry):
+    """pa_sw_scores_noalloc calls that overlap race on their common workspace:
+    their results may be wrong, but no wave may wait for progress that the
+    other call took away, so no task's passes are pipelined there."""
+    rng = np.random.default_rng(12)
+    seqs = [rand_seq(rng, n) for n in (2049, 2048, 30)]
+    seqs[1][500:900] = seqs[0][700:1100]
+    codes, offs = seqset(seqs)
+    pairs = pairs_of([(0, 1), (0, 2), (2, 1)])
+    raw, launches = run(driver, tmp_path, codes, offs, pairs,
+                        EMU_SCORES=entry)
+    got = np.frombuffer(raw, SCORE_DTYPE)
+    sc, ve, he = orc.sw_batch(codes, offs, pairs["r"], pairs["c"], -2, -11)
+    assert np.array_equal(got["score"], sc)
+    assert np.array_equal(got["r_end"].astype(np.int32), ve)
+    assert np.array_equal(got["c_end"].astype(np.int32), he)
+    names = [n for n, _ in launches]
+    assert "k_sw_linear" in names
+    assert ("k_lin_passes" in names) == (entry == "dev")
