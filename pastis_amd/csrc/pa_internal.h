@@ -424,6 +424,7 @@ __host__ __device__ inline uint32_t xd_reach(const XdTask &t, int dir,
 // up to which a batch is split that way.
 constexpr uint64_t kXdSmall = 65536, kXdSplit = (uint64_t)4 << 20;
 constexpr uint32_t kXdLong = 512;
+constexpr int64_t kXdBandItems = 120000;
 
 // Which kernel takes an item first.  Sixteen lanes per item take a fifth of the
 // time per anti-diagonal that one lane takes (0.2 us; a lane 0.7 in an idle
@@ -435,13 +436,21 @@ constexpr uint32_t kXdLong = 512;
 //   sorted: the one-lane kernel's items (with all_band: the band kernel's) in
 //     falling order of their reach, so that the grid does not end on long ones.
 //   all_band: 16 lanes and wide bands for all items.
-// The first two only while the bands fit 16 columns: a gap costs -xdrop_gap and
-// an extension ends X below its best, so a band spans about 2 X / -xdrop_gap
-// columns (9 as called, 49 as documented).  Wider bands outgrow 16 columns in
-// most items: the band kernels take all of them (60,001 pairs, X = 49, gap -2:
-// per-lane pass 0.87 ms and 5.5 ms for its overflow, unsorted; 4.7 ms for all).
-// Measured for the log-normal workload as called (30 % homologs, four items a
-// pair), the whole stage in ms:
+// 16 lanes hold 14 columns.  A gap costs -xdrop_gap and an extension ends X below
+// its best, so a band spans up to 2 X / -xdrop_gap columns (9 as called, 49 as
+// documented).  Bands of 10 fit in nearly every item.  Wider ones outgrow 16
+// columns in the more items the smaller the gap for the same ratio (bands end
+// on mismatches too): from 2 X = g (12 + g) on, g = -xdrop_gap, the band kernels
+// are faster whatever the batch, and up to 120,000 items, divided by what is
+// missing to that line, they are faster since the chip is not full.  The stage
+// in ms, one lane unsorted / split / all_band:
+//   X, gap      line    60,000 pairs        150,000             400,000
+//    66, -11    0.52    6.27  3.53  3.42     7.63  3.77  8.22    9.47  5.49 20.47
+//   100, -11    0.79    8.48  5.49  3.90    11.25  6.51  9.25   16.53 11.23 23.95
+//    40, -5     0.94   10.65  7.06  4.13    16.35 12.53  9.71   29.94 25.36 24.98
+//   130, -11    1.03   11.57  8.66  4.12    18.76 15.76  9.93   37.52 33.73 25.71
+//    20, -2     1.43   11.21  8.94  4.46    18.72 16.19 10.82   39.24 35.06 27.90
+// (log-normal workload, 30 % homologs, four items a pair).  As called:
 //   pairs          one lane, unsorted   sorted   split   16 lanes
 //       16,384                   4.42     5.11    2.30      1.43
 //       65,536                   5.73     6.03    2.42      2.27
@@ -458,11 +467,16 @@ inline XdRoute xd_route(uint64_t ni, int xdrop, int xdrop_gap, int xd_coop,
     XdRoute r{};
     if (xd_coop)
         return r;
-    const bool thin = xdrop / -(int64_t)xdrop_gap <= 5;
+    const int64_t g = -(int64_t)xdrop_gap;
+    const bool thin = xdrop / g <= 5;
+    if (!thin && (xd_wave != 1 || xdrop > 30000))
+        return r;
+    const int64_t line = g * (12 + g), missing = line - 2 * (int64_t)xdrop;
     r.small16 = thin && ni <= kXdSmall;
-    r.split = thin && !r.small16 && ni <= kXdSplit;
-    r.all_band = !thin && xd_wave == 1 && xdrop <= 30000;
-    r.sorted = (thin && !r.small16) || r.all_band;
+    r.all_band = !thin && (missing <= 0 ||
+                           (int64_t)ni * missing <= kXdBandItems * line);
+    r.split = !r.small16 && !r.all_band && ni <= kXdSplit;
+    r.sorted = !r.small16;
     return r;
 }
 

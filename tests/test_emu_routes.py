@@ -135,6 +135,14 @@ def test_linear_rerun_has_the_grid_of_the_first_run(driver, tmp_path):
     (4, 49, -2, 0, 1, "0 0 1 1"), (20000000, 49, -2, 0, 1, "0 0 1 1"),
     (20000000, 49, -2, 0, 2, "0 0 0 0"), (4, 30001, -2, 0, 1, "0 0 0 0"),
     (4, 2147483647, -2147483648, 0, 1, "1 0 0 0"),
+    # bands a little wider: the band kernels for all items took 20.5 ms of
+    # 400,000 pairs at X = 66, where one lane per item had taken 9.5
+    (240000, 66, -11, 0, 1, "0 0 1 1"), (1600000, 66, -11, 0, 1, "0 1 1 0"),
+    (20000000, 66, -11, 0, 1, "0 0 1 0"), (1600000, 100, -11, 0, 1, "0 1 1 0"),
+    (1600000, 130, -11, 0, 1, "0 0 1 1"), (1600000, 40, -5, 0, 1, "0 0 1 1"),
+    (2100000, 40, -5, 0, 1, "0 1 1 0"), (1600000, 200, -31, 0, 1, "0 1 1 0"),
+    (1600000, 66, -11, 0, 0, "0 0 0 0"),
+    (4000000000, 30000, -5999, 0, 1, "0 0 1 0"),
     (4, 49, -11, 1, 1, "0 0 0 0"), (20000000, 49, -2, 1, 1, "0 0 0 0")])
 def test_xdrop_route(items, xdrop, gap, coop, wave, want):
     rules = os.path.join(OUT, "rules")
