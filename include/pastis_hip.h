@@ -473,8 +473,8 @@ typedef struct pa_tuning {
     int32_t xd_wave;        /* X-drop items whose band outgrows the
                                per-lane kernel's rings continue with 16
                                lanes per item: 1 (default) in a 128-column
-                               window, then a 256-column one; 2: the
-                               256-column window only; 0: none.  What is
+                               window, then a 256-column and a 512-column
+                               one; 2: without the first; 0: none.  What is
                                left runs with global-memory rings, one lane
                                per item.  With 1 (and xd_coop 0), items start
                                there where X / -gap exceeds 5 */

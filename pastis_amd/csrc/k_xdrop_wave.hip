@@ -17,9 +17,12 @@
 //     negative, "undefined" is its sign, saturating sums of an undefined cell
 //     stay undefined, and the limit in these units is the best score itself.
 //     An item whose best score nears the type's range, or whose band nears
-//     the window (W - 3 BL columns), is handed on through the overflow list:
-//     from the 128-column to the 256-column kernel, then to the rings in
-//     global memory.
+//     the window (W - 3 BL columns: 104, 208 and 416), is handed on through
+//     the overflow list: from the 128-column to the 256-column and to the
+//     512-column kernel, then to the rings in global memory, where a lane has
+//     the item alone: 10,000 pairs of homologs of 800 residues took 56 ms
+//     there for two items of 40,000, and 300 of 2,500 residues 139 ms for
+//     eight of 1,200.
 //   - Outside the range [minCol, maxCol) of an anti-diagonal the recurrence
 //     gives undefined cells by itself: the columns that the update of minCol
 //     passes are undefined on both anti-diagonals it reads, and so are those
@@ -44,9 +47,8 @@ namespace {
 
 constexpr uint32_t kClaim = 4;        // items claimed per queue atomic
 constexpr int kSteps = 16;            // anti-diagonals between ring refills
-// registers per lane and anti-diagonal: windows of 128 and 256 columns
-constexpr int kBandRegs = 4;
-constexpr int kWideRegs = 8;
+// registers per lane and anti-diagonal: windows of 128, 256 and 512 columns
+constexpr int kBandRegs[3] = {4, 8, 16};
 constexpr uint32_t kUndef2 = 0x80008000u;
 constexpr int kUndef = -32768;
 
@@ -151,6 +153,8 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
         rings[i] = 0;
     __syncthreads();
     const uint32_t n = *a.count;
+    if (n == 0)
+        return;
     const int gap = max(a.gap, -32000);
     const uint32_t GAP = splat(gap);
     uint8_t *const qring = rings + row * (QR + DR);
@@ -576,29 +580,35 @@ hipError_t launch_xdrop_wave(const XdTask *tasks, const uint32_t *list,
 {
     WaveArgs a{tasks, list, count, queue, mat, gap, xdrop, seed_len,
                out, ovf_list, ovf_count};
-    if (wide)
-        hipLaunchKernelGGL(k_xdrop_band<kWideRegs>, dim3(grid), dim3(64), 0,
+    if (wide == 0)
+        hipLaunchKernelGGL(k_xdrop_band<kBandRegs[0]>, dim3(grid), dim3(64), 0,
+                           s, a);
+    else if (wide == 1)
+        hipLaunchKernelGGL(k_xdrop_band<kBandRegs[1]>, dim3(grid), dim3(64), 0,
                            s, a);
     else
-        hipLaunchKernelGGL(k_xdrop_band<kBandRegs>, dim3(grid), dim3(64), 0,
+        hipLaunchKernelGGL(k_xdrop_band<kBandRegs[2]>, dim3(grid), dim3(64), 0,
                            s, a);
     return hipGetLastError();
 }
 
 int xdrop_wave_occupancy(int wide)
 {
-    static int cache[2] = {0, 0};
-    if (!cache[wide ? 1 : 0]) {
+    static int cache[3] = {0, 0, 0};
+    if (!cache[wide]) {
         int n = 0;
-        if (wide)
+        if (wide == 0)
             hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &n, k_xdrop_band<kWideRegs>, 64, 0);
+                &n, k_xdrop_band<kBandRegs[0]>, 64, 0);
+        else if (wide == 1)
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &n, k_xdrop_band<kBandRegs[1]>, 64, 0);
         else
             hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &n, k_xdrop_band<kBandRegs>, 64, 0);
-        cache[wide ? 1 : 0] = n > 0 ? n : 1;
+                &n, k_xdrop_band<kBandRegs[2]>, 64, 0);
+        cache[wide] = n > 0 ? n : 1;
     }
-    return cache[wide ? 1 : 0];
+    return cache[wide];
 }
 
 }  // namespace pa

@@ -87,7 +87,9 @@ enum {
     C_XDWOVFQ = 33,     // their queue head
     C_XDW2OVF = 34,     // items left by the 256-column band kernel
     C_XDW2OVFQ = 35,    // their queue head
-    C_LIN = 36,         // linear-gap classes: list lengths, starts, queues
+    C_XDW3OVF = 36,     // items left by the 512-column band kernel
+    C_XDW3OVFQ = 37,    // their queue head
+    C_LIN = 38,         // linear-gap classes: list lengths, starts, queues
     C_LINS = C_LIN + kLinClasses,
     C_LINQ = C_LINS + kLinClasses,
     C_LINP = C_LINQ + kLinClasses,   // items of the pipelined class
@@ -924,8 +926,8 @@ int run_xdrop(pa_ctx *c, const pa_pair *d_pairs, uint64_t n, hipStream_t s)
         }
     }
     // items whose band outgrew the LDS rings: 16 lanes per item with a
-    // 128-column window, what outgrows it with a 256-column window, the
-    // rest with rings in global memory.  Each pass's overflow list is the
+    // 128-column window, what outgrows it with a 256-column and then a
+    // 512-column window, the rest with rings in global memory.  Each pass's overflow list is the
     // list the pass before last consumed (`lng` is free once the per-lane
     // kernel is done).
     uint32_t *last = ovf, *last_n = ctr + C_XDOVF, *last_q = ctr + C_XDOVFQ;
@@ -956,6 +958,10 @@ int run_xdrop(pa_ctx *c, const pa_pair *d_pairs, uint64_t n, hipStream_t s)
     if (c->tune.xd_wave &&
         (rc = band(1, last == ovf ? lng : ovf, ctr + C_XDW2OVF,
                    ctr + C_XDW2OVFQ)))
+        return rc;
+    if (c->tune.xd_wave &&
+        (rc = band(2, last == ovf ? lng : ovf, ctr + C_XDW3OVF,
+                   ctr + C_XDW3OVFQ)))
         return rc;
     if (c->g_chunks > 0) {
         // captured batch: no host synchronisation; the global-ring pass

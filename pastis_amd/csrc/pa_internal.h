@@ -512,8 +512,8 @@ hipError_t launch_xdrop_coop(const XdTask *tasks, const uint32_t *list,
                              uint32_t *ovf_count, int grid, hipStream_t s);
 int xdrop_coop_occupancy();
 // X-drop with 16 lanes per work item (k_xdrop_wave.hip), for the items whose
-// band outgrew the per-lane kernel's LDS rings: a 128-column window, or
-// 256 columns with `wide`; items whose band outgrows the window are appended
+// band outgrew the per-lane kernel's LDS rings: a window of 128 columns, 256
+// (wide 1) or 512 (wide 2); items whose band outgrows the window are appended
 // to ovf_list.
 hipError_t launch_xdrop_wave(const XdTask *tasks, const uint32_t *list,
                              const uint32_t *count, uint32_t *queue,

@@ -12,7 +12,7 @@
 // EMU_DEV runs the batch through pa_align_dev instead (which takes pairs that
 // the host entry points refuse) and leaves out the extents; EMU_SCORES=<entry>
 // runs pa_sw_scores_<entry> (dev or noalloc) and writes pa_score scores[npairs]
-// instead; EMU_STATS=<file> receives the kernel launches that pa_stats counts.
+// instead; EMU_XDGAP sets the X-drop gap; EMU_STATS=<file> receives the kernel launches that pa_stats counts.
 // Mode 2 runs the k-mer candidate generation instead (see kmer_mode).
 #include <cstdio>
 #include <cstdlib>
@@ -153,6 +153,8 @@ int main(int argc, char **argv)
     if (rc)
         return fail("pa_config_for_cli", rc, nullptr);
     cfg.mode = h[0];
+    if (const char *e = std::getenv("EMU_XDGAP"))
+        cfg.xdrop_gap = std::atoi(e);
     pa_ctx *c = nullptr;
     if ((rc = pa_create(&cfg, &c)))
         return fail("pa_create", rc, nullptr);

@@ -11,7 +11,8 @@ import pytest
 
 from helpers import oracle_params, pairs_of, rand_seq, seqset
 from oracle import oracle as orc
-from pastis_amd._lib import PAIR_DTYPE, RESULT_DTYPE, SCORE_DTYPE
+from pastis_amd._lib import (EXTENT_DTYPE, PAIR_DTYPE, RESULT_DTYPE,
+                             SCORE_DTYPE)
 from test_emu import EMU, OUT, driver  # noqa: F401  (driver: a fixture)
 
 
@@ -194,3 +195,33 @@ def test_passes_wait_for_one_another_only_on_a_workspace_of_ones_own(
     names = [n for n, _ in launches]
     assert "k_sw_linear" in names
     assert ("k_lin_passes" in names) == (entry == "dev")
+
+
+def _extents(codes, offs, pairs, gap, xdrop):
+    out = []
+    for p in pairs:
+        v = codes[int(offs[p["r"]]):int(offs[p["r"] + 1])]
+        h = codes[int(offs[p["c"]]):int(offs[p["c"] + 1])]
+        x = orc.xdrop_extend(h, v, int(p["seed"][1]), int(p["seed"][0]), 6,
+                             gap, xdrop)
+        out.append((x["beg_v"], x["end_v"], x["beg_h"], x["end_h"]))
+    return np.array(out)
+
+
+# Bands of some 250 columns: a few such items took most of a batch's time in
+# the kernel that has its rings in global memory, a lane for an item.
+def test_wide_bands_stay_in_lds(driver, tmp_path):
+    rng = np.random.default_rng(13)
+    a = rand_seq(rng, 420)
+    codes, offs = seqset([a, rand_seq(rng, 430), a.copy()])
+    pairs = pairs_of([(0, 1), (0, 2)], [[200, 204, 0, 0], [100, 100, 0, 0]])
+    raw, launches = run(driver, tmp_path, codes, offs, pairs, mode=1,
+                        xdrop=125, EMU_XDGAP="-1")
+    names = [n for n, _ in launches]
+    # (two calls: the alignment, and the extents of each seed)
+    assert names.count("k_xdrop_band") and "k_xdrop_pl" not in names
+    n = len(pairs)
+    ext = np.frombuffer(raw[n * RESULT_DTYPE.itemsize:][:n * 8], EXTENT_DTYPE)
+    have = np.stack([ext[f].astype(np.int64) for f in
+                     ("r_beg", "r_end", "c_beg", "c_end")], axis=1)
+    assert np.array_equal(have, _extents(codes, offs, pairs, -1, 125))
