@@ -12,12 +12,17 @@
 // left behind takes the block W columns further.  So nothing is moved when the
 // band moves, and column c - 1 is a register shift, or one DPP rotation at a
 // block's first column.
-//   - Values are kept as v + X in int16, the undefined cell as -32768: a cell
-//     kept on anti-diagonal d is at least best - X, so a defined value is not
-//     negative, "undefined" is its sign, saturating sums of an undefined cell
-//     stay undefined, and the limit in these units is the best score itself.
-//     An item whose best score nears the type's range, or whose band nears
-//     the window (W - 3 BL columns: 104, 208 and 416), is handed on through
+//   - Values are kept as v + X - base in int16, the undefined cell as -32768: a
+//     cell kept on anti-diagonal d is at least best - X, so a defined value is
+//     not negative, "undefined" is its sign, saturating sums of an undefined
+//     cell stay undefined, and the limit in these units is best - base.  base
+//     is 0 until the best score nears the type's range, and then moves up to
+//     it: the values of the last three anti-diagonals lie no more than 93 below
+//     the limit (31 a step, the largest matrix score).  Long homologs need it:
+//     300 pairs of 8,000 nearly equal residues were handed on from window to
+//     window to the last kernel below, 181 ms, now 8.5.
+//     An item whose band nears the window (W - 3 BL columns: 104, 208 and
+//     416), or for whose X the type has no room, is handed on through
 //     the overflow list: from the 128-column to the 256-column and to the
 //     512-column kernel, then to the rings in global memory, where a lane has
 //     the item alone: 10,000 pairs of homologs of 800 residues took 56 ms
@@ -47,6 +52,9 @@ namespace {
 
 constexpr uint32_t kClaim = 4;        // items claimed per queue atomic
 constexpr int kSteps = 16;            // anti-diagonals between ring refills
+// largest best - base + X; base follows the best score at this distance from
+// what the steps to the next refill may add, and needs room to do so
+constexpr int kTop = 32000, kStepTop = kTop - 31 * kSteps, kBelow = 128;
 // registers per lane and anti-diagonal: windows of 128, 256 and 512 columns
 constexpr int kBandRegs[3] = {4, 8, 16};
 constexpr uint32_t kUndef2 = 0x80008000u;
@@ -164,7 +172,7 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
     // row-uniform state of the current item
     int state = kNeed;
     uint32_t k = 0;
-    int X = 0, best_max = 0;
+    int X = 0, best_max = 0, base = 0;
     int cols = 0, rows = 0, d = 0, minCol = 0, maxCol = 0, best = 0;
     int off1 = 0, off2 = 0, off3 = 0, l1 = 0, l2 = 0, l3 = 0;
     bool right = false, invalid = false;
@@ -283,7 +291,8 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
                     X = (int)min((int64_t)a.X,
                                  31ll * min(cols, rows) + 1 -
                                      (int64_t)(cols + rows) * gap);
-                    best_max = a.gap < -32000 ? -1 : 32000 - X;
+                    best_max = a.gap < -32000 ? -1 : kTop - X;
+                    base = 0;
                     d = 1;
                     minCol = 1;
                     maxCol = 2;
@@ -362,12 +371,28 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
             dfill += 16;
             dpre = d_load(dfill + j);
         }
+        // ---- the base of the values, where they near the type's range
+        const bool rise = state == kRun && best_max > 0 &&
+                          best - base > max(kStepTop - X, 2 * kBelow);
+        if (__ballot(rise)) {
+            const int up = rise ? best - base - kBelow : 0;
+            const uint32_t UP = splat(up);
+            base += up;
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                P[r] = pk_sub(P[r], UP);
+                O[r] = pk_sub(O[r], UP);
+                Z[r] = pk_sub(Z[r], UP);
+                LD[r] = pk_sub(LD[r], UP);
+            }
+        }
         // ---- kSteps anti-diagonals, or until a row's item ends.  Rows
         // without an item compute on (their results go nowhere).
         bool fin = state != kDone && !(state == kRun && minCol < maxCol);
         uint64_t any = __ballot(fin);
         for (int st = 0; st < kSteps && !any; ++st) {
-            const bool ovf = maxCol - minCol + 2 > WL || best > best_max;
+            const bool ovf =
+                maxCol - minCol + 2 > WL || best - base > best_max;
             const int noff3 = minCol - 1;
             const int nl3 = maxCol + 1 - noff3;
             ++d;
@@ -377,7 +402,7 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
 #pragma unroll
             for (int r = 1; r < NR; ++r)
                 L[r] = __builtin_amdgcn_alignbit(P[r], P[r - 1], 16);
-            const uint32_t BEST = splat(best);
+            const uint32_t BEST = splat(best - base);
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
                 const uint32_t sc = __builtin_amdgcn_perm(
@@ -409,7 +434,8 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
                 dgap += gap;
                 edge = edge && dgap > (int64_t)best - X;
                 if (edge) {
-                    const uint32_t e = (uint32_t)((int)dgap + X) & 0xffffu;
+                    const uint32_t e =
+                        (uint32_t)((int)dgap + X - base) & 0xffffu;
                     masked = 3;
                     if (c0 == 0 && noff3 == 0)
                         V[0] = (V[0] & 0xffff0000u) | e;
@@ -439,7 +465,8 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
             const int gl = max((int)(int16_t)g, (int)g >> 16);
             const int lo = row_min(c0 + fl);
             const int hi = row_max(gl < 0 ? -1 : c0 + gl);
-            const int adb = row_max(max((int)(int16_t)ab, (int)ab >> 16)) - X;
+            const int adb =
+                row_max(max((int)(int16_t)ab, (int)ab >> 16)) - X + base;
             nc += (uint32_t)(maxCol - minCol);
             best = max(best, adb);
             // scores of the next anti-diagonal
@@ -543,7 +570,7 @@ __global__ __launch_bounds__(64) void k_xdrop_band(WaveArgs a)
                 // (score kUndef of the other kernels where nothing is defined)
                 const int score = state == kEmpty || state == kOut ? 0
                                   : ls == kUndef ? INT_MIN / 4
-                                                 : ls - X;
+                                                 : ls - X + base;
                 if (state == kOut) {
                     const uint32_t pos = atomicAdd(a.ovf_count, 1u);
                     a.ovf_list[pos] = k;

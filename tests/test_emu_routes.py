@@ -225,3 +225,24 @@ def test_wide_bands_stay_in_lds(driver, tmp_path):
     have = np.stack([ext[f].astype(np.int64) for f in
                      ("r_beg", "r_end", "c_beg", "c_end")], axis=1)
     assert np.array_equal(have, _extents(codes, offs, pairs, -1, 125))
+
+
+# An X that leaves 16-bit values room for a best score of 2,000: 16 lanes per
+# item to the end all the same, as for homologs of thousands of residues.
+def test_high_scores_stay_in_lds(driver, tmp_path):
+    rng = np.random.default_rng(14)
+    a = rand_seq(rng, 300, "WWWWCP")
+    b = a.copy()
+    b[::50] = rand_seq(rng, len(b[::50]))
+    codes, offs = seqset([a, b])
+    pairs = pairs_of([(0, 1)], [[20, 20, 0, 0]])
+    raw, launches = run(driver, tmp_path, codes, offs, pairs, mode=1,
+                        xdrop=29900, EMU_XDGAP="-1000")
+    assert "k_xdrop_pl" not in [n for n, _ in launches]
+    n = len(pairs)
+    assert np.frombuffer(raw[:n * RESULT_DTYPE.itemsize],
+                         RESULT_DTYPE)["score"].min() > 2600
+    ext = np.frombuffer(raw[n * RESULT_DTYPE.itemsize:][:n * 8], EXTENT_DTYPE)
+    have = np.stack([ext[f].astype(np.int64) for f in
+                     ("r_beg", "r_end", "c_beg", "c_end")], axis=1)
+    assert np.array_equal(have, _extents(codes, offs, pairs, -1000, 29900))
