@@ -5,6 +5,7 @@
 
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -46,8 +47,21 @@ struct pa_fasta {
 
 namespace {
 
+// The compacted stream: no longer than the input, so its bytes are stored
+// without a test.
+struct Stream {
+    std::unique_ptr<char[]> p;
+    size_t n = 0;
+
+    void reserve(size_t cap) { p.reset(new char[cap]); }
+    size_t size() const { return n; }
+    void push_back(char ch) { p[n++] = ch; }
+    void cut(size_t to) { n = to; }
+    const char *begin() const { return p.get(); }
+};
+
 struct FastaParser {
-    std::vector<char> S;      // the compacted stream
+    Stream S;
     std::vector<int64_t> id_start, seq_start;
     std::vector<uint64_t> rec;
     uint64_t nrec = 0;
@@ -67,9 +81,9 @@ struct FastaParser {
             seq_len + (seq_start.back() - id_start.back()) + 1;
         const int64_t to = pos() - count;   // a position
         if (to + front >= 0) {
-            S.resize((size_t)(to + front));
+            S.cut((size_t)(to + front));
         } else {
-            S.clear();
+            S.cut(0);
             front = -to;
         }
         id_start.pop_back();
@@ -82,26 +96,38 @@ struct FastaParser {
         bool in_name = false, in_seq = false;
         int64_t seq_len = 0;
         S.reserve(n);
-        // bytes of a sequence that need a look: the others are copied in runs
+        // Bytes of a sequence that need a look.  The others are copied in
+        // runs, the first 16 bytes of each as they are found, since runs can
+        // be short: 900,000 residues one a line take 3.7 ms, 8.1 with a call
+        // for each run, 3.4 byte by byte; 6 million, 80 a line, 4.2, 4.3, 16.
         bool look[256] = {};
         for (const char ch : {'>', '\n', '*', 'U', 'u'})
             look[(uint8_t)ch] = true;
         for (uint64_t i = 0; i < n; ++i) {
-            if (in_name || in_seq) {
+            if (in_name) {   // a header: everything up to its newline
+                const void *nl = std::memchr(b + i, '\n', n - i);
+                const uint64_t e = nl ? (uint64_t)((const char *)nl - b) : n;
+                std::memcpy(S.p.get() + S.n, b + i, e - i);
+                S.n += e - i;
+                i = e;
+            } else if (in_seq) {
+                char *to = S.p.get() + S.n;
+                const uint64_t near = std::min(n, i + 16);
                 uint64_t e = i;
-                if (in_name) {   // a header: everything up to its newline
-                    const void *nl = std::memchr(b + i, '\n', n - i);
-                    e = nl ? (uint64_t)((const char *)nl - b) : n;
-                } else {
+                for (; e < near && !look[(uint8_t)b[e]]; ++e)
+                    *to++ = b[e];
+                if (e == near) {
+                    const uint64_t from = e;
                     while (e < n && !look[(uint8_t)b[e]])
                         ++e;
-                    seq_len += (int64_t)(e - i);
+                    std::memcpy(to, b + from, e - from);
                 }
-                S.insert(S.end(), b + i, b + e);
-                if (e == n)
-                    break;
+                S.n += e - i;
+                seq_len += (int64_t)(e - i);
                 i = e;
             }
+            if (i == n)
+                break;
             char ch = b[i];
             const bool last = i + 1 >= n;
             if (ch == '>' && !in_name) {
