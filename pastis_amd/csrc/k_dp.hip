@@ -1088,6 +1088,7 @@ __device__ __forceinline__ void tb_run(const TbArgs &a, uint32_t tid,
         }
         // residues i - 16 .. i - 1 and j - 16 .. j - 1, the next one on top
         // (those before a sequence's start lie in the store and are not used)
+        static_assert(kWalkRes == 16, "two words of residues");
         uint64_t q0 = 0, q1 = 0, t0 = 0, t1 = 0;
         if (LOCAL || rows_nib(R)) {
             typedef uint64_t __attribute__((aligned(1))) u64u;

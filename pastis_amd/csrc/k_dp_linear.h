@@ -1065,6 +1065,7 @@ __global__ __launch_bounds__(kTbThreads) void k_traceback_linear(LinArgs a)
         }
         // residues i - 16 .. i - 1 and j - 16 .. j - 1, the next one on top
         // (those before a sequence's start lie in the store and are not used)
+        static_assert(kWalkRes == 16, "two words of residues");
         uint64_t q0 = lin_load8(qs + i - 16), q1 = lin_load8(qs + i - 8);
         uint64_t t0 = lin_load8(ts + j - 16), t1 = lin_load8(ts + j - 8);
 #pragma unroll

@@ -41,9 +41,12 @@ template <class T> __device__ inline T PA_GLOBAL *glb_addr(uint64_t a)
 constexpr int kAlpha = 25;
 constexpr int kSentinel = 25;
 constexpr int kProfChars = 26;
-// Sentinels ahead of the first sequence of a store (a kernel's window of
-// residues may start up to 7 bytes before a sequence).
+// Sentinels ahead of the first sequence of a store: the walks' window of
+// kWalkRes residues that end at a cell starts up to kWalkRes - 1 bytes before
+// a sequence, the other kernels' windows up to 7.
+constexpr int kWalkRes = 16;
 constexpr size_t kSeqPad = 64;
+static_assert(kSeqPad >= kWalkRes, "walk windows stay in the store");
 
 // One DP task: the row (V, lanes) and column (H, streamed) sequence spans.
 struct DpTask {
