@@ -87,15 +87,19 @@ enum {
     C_XDWOVFQ = 33,     // their queue head
     C_XDW2OVF = 34,     // items left by the 256-column band kernel
     C_XDW2OVFQ = 35,    // their queue head
-    C_XDW3OVF = 36,     // items left by the 512-column band kernel
-    C_XDW3OVFQ = 37,    // their queue head
-    C_LIN = 38,         // linear-gap classes: list lengths, starts, queues
+    // linear-gap classes: list lengths, starts, queues (two words further on,
+    // 100,000 pairs U[50,500] took 2.6 % longer, traced and score only: the
+    // queues and what the waves read of the classes share cache lines)
+    C_LIN = 36,
     C_LINS = C_LIN + kLinClasses,
     C_LINQ = C_LINS + kLinClasses,
     C_LINP = C_LINQ + kLinClasses,   // items of the pipelined class
     C_HIST,             // histogram of the counting sort
     C_FILL = C_HIST + kMaxBins * kBuckets,   // its running slots
-    C_N = C_FILL + kMaxBins * kBuckets
+    C_XDW3OVF = C_FILL + kMaxBins * kBuckets,   // items left by the 512-column
+                                                // band kernel
+    C_XDW3OVFQ,         // their queue head
+    C_N
 };
 
 constexpr int kModes = 3;           // DP modes of the kernel statistics
