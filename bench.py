@@ -145,8 +145,10 @@ def roofline(kstats, st, step_ms_total, tuning=None, traffic_key=None):
         pl = "k_xdrop_pl<%d>" % tn.get("xd_ring", 16)
         chain = ["k_xdrop_coop", pl] if tn.get("xd_coop") else \
             ["(thin bands) k_xdrop_coop beside " + pl]
-        chain += {0: [], 1: ["k_xdrop_band<4>", "k_xdrop_band<8>"],
-                  2: ["k_xdrop_band<8>"]}[tn.get("xd_wave", 1)]
+        chain += {0: [], 1: ["k_xdrop_band<4>", "k_xdrop_band<8>",
+                             "k_xdrop_band<16>"],
+                  2: ["k_xdrop_band<8>", "k_xdrop_band<16>"]}[
+                      tn.get("xd_wave", 1)]
         chain.append("k_xdrop_pl<0>")
         xk = "X-drop stage: " + " -> ".join(chain)
         cands.append(dict(kernel=xk, ms=st["ms_xdrop"],

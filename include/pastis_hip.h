@@ -412,10 +412,11 @@ int pa_synchronize(struct pa_ctx *ctx);
  * swt = local traced, nwt = global traced), row class (c0..c3, with the
  * class's current kernel shape, e.g. l64r8 = 64 lanes x 8 rows per lane)
  * and arithmetic (i16 packed, i32); "rerun" classes are the int32 re-runs
- * of saturated tasks.  Example: "nwt.c3.l64r8.i16".  "swl.r16.i16",
- * "swtl.r16.i16" and "nwl.r16.i16" are the same modes in the linear-gap
- * kernels, which run all their tasks in one launch.  cells are DP cells of
- * the tasks the class ran. */
+ * of saturated tasks.  Example: "nwt.c3.l64r8.i16".  In the default shapes the
+ * row classes run in one launch: "nwt.all.r8.i16", "nwt.all.r8.i32" (the re-runs
+ * of saturated local tasks among the latter).  "swl.r16.i16", "swtl.r16.i16"
+ * and "nwl.r16.i16" are the same modes in the linear-gap kernels, which run all
+ * their tasks in one launch.  cells are DP cells of the tasks the class ran. */
 typedef struct pa_kernel_stat {
     char name[24];
     uint64_t launches;
@@ -459,7 +460,8 @@ typedef struct pa_tuning {
                                kernel first (band up to 14 columns), the rest
                                to the one-lane-per-item kernels; 0 (default):
                                by size, 16 lanes per item in small batches
-                               and for far-reaching items, else one */
+                               and for the far-reaching items of batches that
+                               do not fill the chip, else one */
     int32_t dp_edge[3];     /* DP row classes: a task whose row span has
                                qlen rows is in the first class c with
                                qlen <= dp_edge[c], class 3 takes the rest;
@@ -477,7 +479,8 @@ typedef struct pa_tuning {
                                one; 2: without the first; 0: none.  What is
                                left runs with global-memory rings, one lane
                                per item.  With 1 (and xd_coop 0), items start
-                               there where X / -gap exceeds 5 */
+                               there where X / -gap exceeds 5, except in large
+                               batches where bands rarely exceed 14 columns */
     int32_t tb_overlap;     /* 1: each class's tracebacks run on a second
                                stream beside the next classes' DP; 2: those
                                of all classes but the last beside the last

@@ -24,7 +24,9 @@
 // No value leaves 0 .. 15, whatever the lengths, so no task needs int32; one
 // register per row holds the state and the borders are zeros.  A cell pair is
 //   z = max3(s, v, u); z1 = (z & ~3) | 1; u = z1 - v; v = z1 - u
-// (no half borrows, so plain 32-bit subtractions).
+// (no half borrows, so plain 32-bit subtractions).  Alignment by differences
+// is published (Suzuki and Kasahara, BMC Bioinformatics 19, 2018, for affine
+// gaps in SIMD lanes).
 //
 // Local (LinLocal): H and H + g (saturated at 0) per row; saturating
 // subtraction takes the place of the maximum with 0.  Scores that come near
@@ -35,16 +37,20 @@
 // global state zero before the first column and unchanged after the last, and
 // keeps local cells below the best one.
 //
-// What bounds it: VALU issue.  A step of 16 row pairs takes 125 instructions
-// in global mode, 7.8 per pair (4 recurrence, 2 score unpack, 1.25 code
-// packing), 165-185 in traced local mode and 105-125 in score-only mode,
-// against 22-28 per pair in the affine kernels, which carry E, F and H.
-// Measured, start -> now:
+// What bounds it: VALU instructions.  A step of 16 row pairs takes 125 in
+// global mode, 7.8 per pair (4 recurrence, 2 score unpack, 1.25 code packing),
+// 165-185 in traced local mode and 105-125 in score-only mode, against 22-28
+// per pair in the affine kernels, which carry E, F and H.  By the counters the
+// global kernel issues VALU in 81 % of the cycles with 96 % of the lanes on,
+// the traced local one in 76 % (90 %) and the score-only one in 75 % (87 %):
+// 26,624 bytes of LDS a wave hold it to six waves per CU, two SIMDs with one.
+// Measured, affine kernels -> these:
 //   400,000 pairs of the log-normal X-drop workload (30 % homologs), traced
 //     global DP 16.6 -> 5.0 ms (eight launches -> one);
-//   100,000 pairs U[50,500], traced local DP 6.9 -> 2.4 ms, score only
-//     4.9 -> 1.6 ms;
-//   100,000 pairs with a tail to 35,000 residues, score only, 466 -> 14 ms.
+//   100,000 pairs U[50,500], traced local DP 6.9 -> 2.6 ms, score only
+//     4.9 -> 1.7 ms;
+//   100,000 pairs with a tail to 35,000 residues, score only, a pass alone
+//     180-470 -> 14 ms (one pass among others 5-12, by the longest pair).
 #pragma once
 
 namespace pa {
@@ -595,7 +601,9 @@ constexpr uint32_t kLinDone = 0xffffffffu;
 // PIPE: every pass of a task is an item of its own, so that the passes of a
 // long task run on as many waves, each a few hundred columns behind the one
 // before: without it the longest task of a batch ran its passes on one wave
-// (35,000 x 35,000 residues: 320 ms) while the chip was idle.  Items are
+// (35,000 x 35,000 residues: 320 ms) while the chip was idle.  (The grid has
+// no more workgroups than the batch tasks, so a single task gains nothing:
+// 20,000 x 20,000 residues 66 ms.)  Items are
 // claimed in order, a task's passes one after the other, and an item waits
 // only for items claimed before it (its predecessor's columns, the last
 // owner and reader of its boundary slot), so the first unfinished item always runs.
@@ -1014,7 +1022,7 @@ __global__ __launch_bounds__(256) void k_lin_passes(LinArgs a)
 // all walk until they have left theirs: bound by the latency of those loads,
 // once in about 12 steps.  With one segment and 8 residues a window, loaded as
 // each walk needed them, some walk of the wave waited in nearly every step:
-// 400,000 walks of the log-normal X-drop workload 2.4 -> 1.26 ms, 20,011 local
+// 400,000 walks of the log-normal X-drop workload 2.4 -> 1.0 ms, 100,000 local
 // walks of up to 500 residues 0.64 -> 0.36 ms.
 template <bool LOCAL>
 __global__ __launch_bounds__(kTbThreads) void k_traceback_linear(LinArgs a)

@@ -18,7 +18,8 @@ struct Buf {
 
 struct Timer {
     int kind;  // 0 sw, 1 xdrop, 2 nw, 3 trace, 4 total, 5 + mode: a linear
-               // kernel, 100 + 16 * mode + bin: a DP kernel class
+               // kernel, 8 + mode and 11 + mode: all affine classes in int16
+               // and int32, 100 + 16 * mode + bin: a DP kernel class
     hipEvent_t a, b;
 };
 
