@@ -11,8 +11,7 @@ import pytest
 
 from helpers import oracle_params, pairs_of, rand_seq, seqset
 from oracle import oracle as orc
-from pastis_amd._lib import (EXTENT_DTYPE, PAIR_DTYPE, RESULT_DTYPE,
-                             SCORE_DTYPE)
+from pastis_amd._lib import PAIR_DTYPE, RESULT_DTYPE, SCORE_DTYPE
 from test_emu import EMU, OUT, driver  # noqa: F401  (driver: a fixture)
 
 
@@ -197,52 +196,41 @@ def test_passes_wait_for_one_another_only_on_a_workspace_of_ones_own(
     assert ("k_lin_passes" in names) == (entry == "dev")
 
 
-def _extents(codes, offs, pairs, gap, xdrop):
-    out = []
-    for p in pairs:
-        v = codes[int(offs[p["r"]]):int(offs[p["r"] + 1])]
-        h = codes[int(offs[p["c"]]):int(offs[p["c"] + 1])]
-        x = orc.xdrop_extend(h, v, int(p["seed"][1]), int(p["seed"][0]), 6,
-                             gap, xdrop)
-        out.append((x["beg_v"], x["end_v"], x["beg_h"], x["end_h"]))
-    return np.array(out)
+def _same_as_the_oracle(raw, codes, offs, pairs, gap, xdrop):
+    got = np.frombuffer(raw, RESULT_DTYPE)
+    ref = orc.sxa_batch(codes, offs, pairs["r"], pairs["c"], pairs["seed"],
+                        orc.params(-2, -11, gap, xdrop, 6, 2, 0.7, 30))
+    for f in ("score", "matches", "cols", "gap_opens", "seed"):
+        assert np.array_equal(got[f].astype(np.int64),
+                              ref[f].astype(np.int64)), f
+    return got
 
 
 # Bands of some 250 columns: a few such items took most of a batch's time in
 # the kernel that has its rings in global memory, a lane for an item.
 def test_wide_bands_stay_in_lds(driver, tmp_path):
     rng = np.random.default_rng(13)
-    a = rand_seq(rng, 420)
-    codes, offs = seqset([a, rand_seq(rng, 430), a.copy()])
-    pairs = pairs_of([(0, 1), (0, 2)], [[200, 204, 0, 0], [100, 100, 0, 0]])
+    codes, offs = seqset([rand_seq(rng, 262), rand_seq(rng, 265)])
+    # the second seed leaves little to extend
+    pairs = pairs_of([(0, 1)], [[0, 0, 256, 258]])
     raw, launches = run(driver, tmp_path, codes, offs, pairs, mode=1,
-                        xdrop=125, EMU_XDGAP="-1")
+                        xdrop=250, EMU_XDGAP="-1", EMU_DEV="1")
     names = [n for n, _ in launches]
-    # (two calls: the alignment, and the extents of each seed)
-    assert names.count("k_xdrop_band") and "k_xdrop_pl" not in names
-    n = len(pairs)
-    ext = np.frombuffer(raw[n * RESULT_DTYPE.itemsize:][:n * 8], EXTENT_DTYPE)
-    have = np.stack([ext[f].astype(np.int64) for f in
-                     ("r_beg", "r_end", "c_beg", "c_end")], axis=1)
-    assert np.array_equal(have, _extents(codes, offs, pairs, -1, 125))
+    assert "k_xdrop_band" in names and "k_xdrop_pl" not in names
+    _same_as_the_oracle(raw, codes, offs, pairs, -1, 250)
 
 
 # An X that leaves 16-bit values room for a best score of 2,000: 16 lanes per
 # item to the end all the same, as for homologs of thousands of residues.
 def test_high_scores_stay_in_lds(driver, tmp_path):
     rng = np.random.default_rng(14)
-    a = rand_seq(rng, 300, "WWWWCP")
+    a = rand_seq(rng, 270, "WWWWCP")
     b = a.copy()
     b[::50] = rand_seq(rng, len(b[::50]))
     codes, offs = seqset([a, b])
-    pairs = pairs_of([(0, 1)], [[20, 20, 0, 0]])
+    pairs = pairs_of([(0, 1)], [[4, 4, 0, 260]])
     raw, launches = run(driver, tmp_path, codes, offs, pairs, mode=1,
-                        xdrop=29900, EMU_XDGAP="-1000")
+                        xdrop=29900, EMU_XDGAP="-1000", EMU_DEV="1")
     assert "k_xdrop_pl" not in [n for n, _ in launches]
-    n = len(pairs)
-    assert np.frombuffer(raw[:n * RESULT_DTYPE.itemsize],
-                         RESULT_DTYPE)["score"].min() > 2600
-    ext = np.frombuffer(raw[n * RESULT_DTYPE.itemsize:][:n * 8], EXTENT_DTYPE)
-    have = np.stack([ext[f].astype(np.int64) for f in
-                     ("r_beg", "r_end", "c_beg", "c_end")], axis=1)
-    assert np.array_equal(have, _extents(codes, offs, pairs, -1000, 29900))
+    got = _same_as_the_oracle(raw, codes, offs, pairs, -1000, 29900)
+    assert got["score"][0] > 2200
