@@ -100,7 +100,6 @@ constexpr size_t kMargin = (size_t)1 << 17;
 
 hipError_t hipMalloc(void **p, size_t n)
 {
-    n = (n + 7) & ~(size_t)7;
     char *m = (char *)std::malloc(n + 2 * kMargin + 16);
     if (!m) {
         *p = nullptr;
